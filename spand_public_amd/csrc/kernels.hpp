@@ -106,19 +106,22 @@ hipError_t launch_perm_out(const double* ws, const int* perm, int N, int nrhs, d
                            hipStream_t st);
 hipError_t launch_cm2il(const double* src, int ld, int N, int nrhs, double* dst, hipStream_t st);
 hipError_t launch_il2cm(const double* src, int N, int nrhs, double* dst, int ld, hipStream_t st);
-// mv phases of the preconditioner apply: SOLVE_CHUNK outputs per chunk, pieces of at most
-// MV_PIECE_WORK inner elements and MV_PIECE_TERMS terms; partial holds npieces x
-// SOLVE_CHUNK x nrhs doubles.
-constexpr int SOLVE_CHUNK = 64;
-constexpr int MV_PIECE_WORK = 64;
-constexpr int MV_PIECE_TERMS = 64;
-template <typename T>
-hipError_t launch_mv(const MvGroup* d_groups, const MvChunk* d_chunks, const MvPiece* d_pieces, int npieces,
-                     const MvTerm* d_terms, const int* d_rchunks, int nreduce, double* ws, double* partial, int nrhs,
-                     hipStream_t st);
-// Explicit V, S and the identity X of the Orthogonal ops of one level (WyTask); tiles are
-// the (task, a0, c0) 32 x 32 tiles of the Gram matrices (a0 <= c0). X = S^{-1} is left to
-// launch_trsm.
+// mv phases of the preconditioner apply: chunks of MV_ROWS outputs, inner positions taken
+// MV_STEP at a time. launch_mv runs one phase over the device; launch_mv_tail runs n
+// consecutive small phases in one workgroup (phases: n host descriptors, n <= MV_TAIL_MAX).
+constexpr int MV_ROWS = 16;
+constexpr int MV_STEP = 16;
+constexpr int MV_NW_MAX = 16;
+constexpr int MV_TAIL_MAX = 16;
+constexpr long long MV_TAIL_STEPS = 96;  // a phase of at most this many steps is small
+struct MvTail {
+    MvDevPhase ph[MV_TAIL_MAX];
+    int n;
+};
+template <typename T> hipError_t launch_mv(const MvDevPhase& ph, double* ws, int nrhs, hipStream_t st);
+template <typename T> hipError_t launch_mv_tail(const MvTail& tail, double* ws, int nrhs, hipStream_t st);
+// Explicit V and -S of the Orthogonal ops of one level (WyTask); tiles are the (task, a0,
+// c0) 32 x 32 tiles of the Gram matrices (a0 <= c0).
 template <typename T>
 hipError_t launch_wy(const WyTask* d_tasks, int ntasks, const int4* d_tiles, int ntiles, hipStream_t st);
 template <typename T>

@@ -731,7 +731,7 @@ __global__ void __launch_bounds__(NT) k_schur(const SchurTile* tiles, const Schu
     T acc_c[4];
     for (int q = 0; q < 4; q++) {
         int i = ti, j = tj0 + q;
-        acc_c[q] = (i < t.tm && j < t.tn) ? C[(t.r0 + i) + (size_t)(t.c0 + j) * t.ldc] : T(0);
+        acc_c[q] = (i < t.tm && j < t.tn && !(t.lower & SCHUR_CLEAR)) ? C[(t.r0 + i) + (size_t)(t.c0 + j) * t.ldc] : T(0);
     }
     for (int kk = t.k0; kk < t.k1; kk++) {
         const SchurContrib c = contribs[kk];
@@ -773,7 +773,7 @@ __global__ void __launch_bounds__(NT) k_schur(const SchurTile* tiles, const Schu
         int i = ti, j = tj0 + q;
         if (i < t.tm && j < t.tn) {
             int gi = t.r0 + i, gj = t.c0 + j;
-            if (!t.lower || gi >= gj) C[gi + (size_t)gj * t.ldc] = acc_c[q];
+            if (!(t.lower & SCHUR_LOWER) || gi >= gj) C[gi + (size_t)gj * t.ldc] = acc_c[q];
         }
     }
 }
@@ -826,10 +826,10 @@ __global__ void __launch_bounds__(NT) k_schur_f32_mfma(const SchurTile* tiles, c
         const int i = idx % ST, j = idx / ST;
         if (i < t.tm && j < t.tn) {
             const int gi = t.r0 + i, gj = t.c0 + j;
-            if (!t.lower || gi >= gj) {
+            if (!(t.lower & SCHUR_LOWER) || gi >= gj) {
                 const float sum = (Ps[0][j][i] + Ps[1][j][i]) + (Ps[2][j][i] + Ps[3][j][i]);
                 const auto cp = C + gi + (size_t)gj * t.ldc;
-                *cp = *cp - sum;
+                *cp = (t.lower & SCHUR_CLEAR) ? -sum : *cp - sum;
             }
         }
     }

@@ -1,17 +1,17 @@
 // Preconditioner-apply sweeps and FP64 Krylov vector kernels for gfx950.
 //
 // Tree::solve (src/tree.cpp:1610-1635) replays the recorded operations forward then
-// backward on per-cluster segments of one vector; here every recorded op of one ND level
-// and one kind runs as a single launch (one workgroup per cluster / target segment) on a
-// block of nrhs right-hand sides stored interleaved, x[(xoff + i) * nrhs + r].
-//   trsv   -> ScalingLLT fwd/bwd          src/operations.cpp:95-103 (cblas_dtrsv)
-//   gemv   -> GemmSymmOut/In fwd/bwd       src/operations.cpp:55-93  (cblas_dgemv)
-//   qapply -> Orthogonal fwd/bwd          src/operations.cpp:149-158 (LAPACKE_dormqr)
-//   merge  -> Merge fwd/bwd               src/operations.cpp:166-192
+// backward on per-cluster segments of one vector; here the ops of one ND level run as three
+// launches per direction (tasks.hpp) on a block of nrhs right-hand sides stored interleaved,
+// x[(xoff + i) * nrhs + r]. They replace
+//   E      ScalingLLT fwd/bwd             src/operations.cpp:95-103 (cblas_dtrsv)
+//   G      GemmSymmOut/In fwd/bwd         src/operations.cpp:55-93  (cblas_dgemv)
+//   W      ScalingLLT, Orthogonal, Merge  src/operations.cpp:95-103,149-158,166-192
 // The Krylov kernels back cg (src/is.cpp:39-121): CSR SpMV and deterministic two-pass dots.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "kernels.hpp"
 #include "tasks.hpp"
@@ -32,10 +32,6 @@ constexpr int NT = 256;
 // Segments are FP64 whatever the factor's element type T: an FP32 factor is read as FP32 and
 // applied in FP64 arithmetic, so the preconditioner stays one fixed linear operator.
 using VT = double;
-// Dynamic LDS of the solve kernels: a chunk of up to 8 right-hand sides of the segment (and
-// for the Householder apply two k-vectors per right-hand side); the chunk width is derived
-// from the segment size, and the host rejects segments that would not fit one column.
-
 static inline int grid_for(size_t n) {
     size_t g = (n + NT - 1) / NT;
     return (int)(g > 65536 ? 65536 : (g == 0 ? 1 : g));
@@ -80,215 +76,228 @@ __global__ void __launch_bounds__(NT) k_il2cm(const double* src, int N, int nrhs
 }
 
 // ---------------------------------------------------------------------------------------
-// mv phases (task layouts in tasks.hpp). A workgroup computes one piece: 64 outputs of one
-// chunk over at most MV_PIECE_WORK inner positions, gathered from at most MV_PIECE_TERMS
-// terms. The work is staged in one round so that its global loads are in flight together:
-//   1. one lane per term reads the term record, clips its inner range, and a wavefront scan
-//      packs the terms' ranges into consecutive positions;
-//   2. every thread loads its share of the piece's matrix entries (MV_EPT of them, all
-//      issued before any is stored) into tile[position][output], and the sources of up to
-//      RG_MAX right-hand sides into xl[position][r];
-//   3. 4 partitions of the positions (one wavefront each, position p to partition p % 4)
-//      accumulate each output, and the partitions are added in a fixed order.
-// A chunk with several pieces writes partial sums, which k_mv_reduce adds in piece order
-// after the launch. (Adding them in the chunk's last piece to finish, found by a counter,
-// measured 3-7x slower on gfx950: the device-scope release fence each piece needs writes its
-// XCD's L2 back.)
-constexpr int RG_MAX = 8;
+// mv phases (task layouts in tasks.hpp), on the FP64 matrix cores whatever the factor's type.
+// A chunk is 16 outputs; its inner positions are taken 16 at a time (a step), and step s of
+// the chunk belongs to wavefront s % nw of the nw that share the chunk.
+//   * Each wavefront reads the chunk's term records itself, one lane per term, scans their
+//     step counts, and finds a step's term by a ballot over the lanes: the records cost one
+//     memory round trip whatever their number, and no LDS.
+//   * A step's matrix entries are loaded straight into the operand layout (lane l: output
+//     l % 16, inner positions 4 (l / 16) + q, q = 0..3), with no staging: along a column of A
+//     when not transposed (16 contiguous entries a column), along 4 contiguous entries a lane
+//     when transposed. The next step's loads are issued before a step's products.
+//   * Up to 4 right-hand sides use v_mfma_f64_4x4x4 (four blocks of 4 outputs; a quarter of
+//     the 16x16x4's cycles), up to 16 one v_mfma_f64_16x16x4 tile, up to 32 two.
+// The matrix instructions add their four products in inner order by fused multiply-adds, so
+// an output's sum does not depend on the number of right-hand sides.
+// Bound by the launch and the chain chunk -> terms -> entries for most phases (a level holds
+// few outputs), by the factor's bytes for the largest. 16 outputs a chunk and 16 positions a
+// step keep the padding of short clusters (10 to 60 rows at the lower levels) small.
+// Measured against six phases per level and direction staged through LDS with partial sums
+// added by second launches: 64^3 Laplacian, FP64 factor (619 MB), 4 columns 2.92 -> 0.81 ms;
+// 512^2, 32 columns 4.98 -> 1.00 ms; 40^2, one column 273 -> 89 us.
 constexpr int WAVE = 64;
-constexpr int SC = SOLVE_CHUNK;
-constexpr int NP = NT / SC;                      // 4 partitions of the inner positions
-constexpr int PW = MV_PIECE_WORK;                // positions per piece
-constexpr int MV_EPT = PW * SC / NT;             // matrix entries per thread: 16
-static_assert(MV_PIECE_TERMS <= WAVE, "one lane per term record");
-static_assert(PW * RG_MAX <= 2 * NT, "two source loads per thread");
+using d4 = double __attribute__((ext_vector_type(4)));
 
-struct MvTermL {  // a term's record in LDS, with its clipped inner range and first position
-    const void* A;
-    const int* perm;
-    int rows, lo, len, off, xsrc, trans;
+template <typename T>
+struct MvStep {  // one step's operands
+    T a[4];
+    double x[2][4];
 };
 
-// y (op)= sum: the chunk's outputs, in the group's mode, through dperm if the group has one
-__device__ inline void mv_apply(VT* y, int mode, VT sum) {
-    *y = mode == MV_SUB ? *y - sum : (mode == MV_SETNEG ? -sum : sum);
+// Records of a wavefront's terms, one lane each, and where each term's steps start.
+struct MvLane {
+    const void* A;
+    const int* perm;
+    int ld, lo, hi, xsrc, trans, off;
+};
+
+__device__ inline int rl(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
+template <typename X>
+__device__ inline X* rlp(X* p, int lane) {
+    const unsigned long long u = (unsigned long long)p;
+    const unsigned lo = (unsigned)rl((int)(unsigned)u, lane), hi = (unsigned)rl((int)(unsigned)(u >> 32), lane);
+    return (X*)(((unsigned long long)hi << 32) | lo);
 }
 
-// adds the partial sums of one chunk's pieces in piece order and applies them
-__device__ inline void mv_chunk_reduce(const MvChunk& ch, const MvGroup& g, const VT* partial, VT* ws, int nrhs) {
-    const int no = min(SC, g.n - ch.o0);
-    for (int idx = threadIdx.x; idx < no * nrhs; idx += NT) {
-        const int lane = idx / nrhs, r = idx % nrhs;
-        VT sum = VT(0);
-        for (int p = ch.p0; p < ch.p1; p++) sum += partial[((size_t)p * SC + lane) * nrhs + r];
-        const int o = ch.o0 + lane;
-        mv_apply(ws + (size_t)(g.xdst + (g.dperm ? gp(g.dperm)[o] : o)) * nrhs + r, g.mode, sum);
+// Operands of step s: term t of the lanes, inner positions [j, j + 16) clipped to hi. Rows past
+// the chunk's outputs read its last row (their sums are not stored); positions past hi are
+// zero in both operands.
+template <typename T, int CT>
+__device__ inline void mv_load(const MvLane& L, unsigned long long m, int s, int o0, int no, const double* ws, int nrhs,
+                               int r0, MvStep<T>& st) {
+    const int lane = threadIdx.x & (WAVE - 1);
+    const int t = __popcll(m) - 1;
+    const int j = rl(L.lo, t) + (s - rl(L.off, t)) * MV_STEP;
+    const int nv = min(MV_STEP, rl(L.hi, t) - j);
+    const int ld = rl(L.ld, t), xs = rl(L.xsrc, t);
+    const gptr<const T> A = gp(reinterpret_cast<const T*>(rlp(L.A, t)));
+    const int row = o0 + min(lane & 15, no - 1), kk = 4 * (lane >> 4);
+    if (rl(L.trans, t)) {
+        const gptr<const T> p = A + (size_t)row * ld + j;
+        if (nv == MV_STEP) {
+#pragma unroll
+            for (int q = 0; q < 4; q++) st.a[q] = p[kk + q];
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const T v = p[min(kk + q, nv - 1)];
+                st.a[q] = kk + q < nv ? v : T(0);
+            }
+        }
+    } else {
+        const gptr<const T> p = A + row + (size_t)j * ld;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const T v = p[(size_t)min(kk + q, nv - 1) * ld];
+            st.a[q] = kk + q < nv ? v : T(0);
+        }
+    }
+    const gptr<const int> perm = gp(rlp(L.perm, t));
+    const gptr<const double> x = gp(ws);
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int k = j + min(kk + q, nv - 1);
+        const size_t e = (size_t)(xs + (perm ? perm[k] : k)) * nrhs;
+#pragma unroll
+        for (int c = 0; c < (CT == 0 ? 1 : CT); c++) {
+            const int r = min(r0 + (CT == 0 ? lane & 3 : 16 * c + (lane & 15)), nrhs - 1);
+            const double v = x[e + r];
+            st.x[c][q] = kk + q < nv ? v : 0.0;
+        }
     }
 }
 
-// RED_IN_TILE (only for nrhs <= RG_MAX, one right-hand-side group): the partitions' sums are
-// written over the tile once every partition has read it. That cuts the LDS of a workgroup
-// from 35.7 to 23.4 KB (FP32) and 52.3 to 40.0 KB (FP64): 7 instead of 4 (4 instead of 3)
-// workgroups share a CU, so a phase of up to 1792 (1024) pieces loads in one round.
-template <typename T, bool RED_IN_TILE>
-__global__ void __launch_bounds__(NT) k_mv_piece(const MvPiece* pieces, const MvTerm* terms, VT* ws, VT* partial,
-                                                 int nrhs) {
-    constexpr size_t TILE_B = sizeof(T[PW][SC + 1]), RED_B = sizeof(VT[NP - 1][SC][RG_MAX]);
-    static_assert(TILE_B % alignof(VT) == 0, "red follows the tile");
-    __shared__ __align__(16) unsigned char s_tr[RED_IN_TILE ? (TILE_B > RED_B ? TILE_B : RED_B) : TILE_B + RED_B];
-    // the piece's matrix: inner position x output
-    T (*const tile)[SC + 1] = reinterpret_cast<T (*)[SC + 1]>(s_tr);
-    // partitions 1..3 (partition 0 keeps its registers)
-    VT (*const red)[SC][RG_MAX] = reinterpret_cast<VT (*)[SC][RG_MAX]>(s_tr + (RED_IN_TILE ? 0 : TILE_B));
-    __shared__ VT xl[PW][RG_MAX];           // the sources of the current right-hand-side group
-    __shared__ MvTermL st[MV_PIECE_TERMS];
-    __shared__ unsigned char p2t[PW];       // position -> term
-    __shared__ int s_total;
-    const MvPiece pc = pieces[blockIdx.x];
-    const int o0 = pc.o0, no = pc.no, nt = pc.k1 - pc.k0;
-    const int tid = threadIdx.x, lane = tid % SC, kp = tid / SC;
-    // 1. term records and their positions
-    if (tid < WAVE) {
-        int len = 0;
-        if (tid < nt) {
-            const MvTerm tm = terms[pc.k0 + tid];
-            int lo = 0, hi = tm.trans ? tm.rows : tm.cols;
-            if (nt == 1) {
-                lo = pc.j0;
-                hi = pc.j1;
+// One chunk by the nw wavefronts of a group (sub: this one's place in it); red holds the
+// group's (nw - 1) x 64 lanes x NACC partial sums. Every wavefront of the workgroup calls it
+// (live: the group has a chunk) because the sums meet at workgroup barriers.
+template <typename T, int CT>
+__device__ inline void mv_chunk(const MvDevPhase& ph, int ci, bool live, int sub, double* red, double* ws, int nrhs,
+                                int r0) {
+    constexpr int NACC = CT == 0 ? 1 : 4 * CT;
+    const int lane = threadIdx.x & (WAVE - 1), nw = ph.nw;
+    double acc1 = 0.0;
+    d4 acc[2] = {};
+    MvChunk ch{};
+    if (live) {
+        ch = ph.chunks[ci];
+        for (int kb = ch.k0; kb < ch.k1; kb += WAVE) {
+            const int nt = min(WAVE, ch.k1 - kb);
+            MvLane L{};
+            int n = 0;
+            if (lane < nt) {
+                const MvTerm tm = ph.terms[kb + lane];
+                L.A = tm.A;
+                L.perm = tm.perm;
+                L.ld = tm.ld;
+                L.xsrc = tm.xsrc;
+                L.trans = tm.flags & MV_TRANS;
+                L.lo = (tm.flags & MV_TRI_UP) ? min(tm.len, ch.o0) : 0;
+                L.hi = (tm.flags & MV_TRI_LO) ? min(tm.len, ch.o0 + MV_ROWS) : tm.len;
+                n = (max(0, L.hi - L.lo) + MV_STEP - 1) / MV_STEP;
             }
-            if (tm.tri == 1) hi = min(hi, o0 + SC);
-            if (tm.tri == 2) lo = max(lo, o0);
-            len = max(0, hi - lo);
-            st[tid] = MvTermL{tm.A, tm.perm, tm.rows, lo, len, 0, tm.xsrc, tm.trans};
-        }
-        int incl = len;  // inclusive scan over the wavefront
+            int incl = n;  // inclusive scan over the wavefront
 #pragma unroll
-        for (int d = 1; d < WAVE; d <<= 1) {
-            const int v = __shfl_up(incl, d);
-            if (tid >= d) incl += v;
-        }
-        if (tid < nt) st[tid].off = incl - len;
-        if (tid == WAVE - 1) s_total = incl;
-    }
-    __syncthreads();
-    const int total = s_total;  // <= PW (the planner's bound)
-    for (int p = tid; p < total; p += NT) {  // the last term starting at or before p holds p
-        int lo = 0, hi = nt - 1;
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (st[mid].off <= p) lo = mid;
-            else hi = mid - 1;
-        }
-        p2t[p] = (unsigned char)lo;
-    }
-    __syncthreads();
-    // 2. the matrix entries: entry e of the piece belongs to the term holding position e / SC;
-    // within the term's block q = e - SC * off runs along the outputs of one inner index (A's
-    // column, not transposed) or along the inner indices of one output (A's column, transposed),
-    // so that neighbouring lanes read neighbouring addresses either way
-    const int ne = total * SC;
-    T v[MV_EPT];
-    int dst[MV_EPT];
-#pragma unroll
-    for (int u = 0; u < MV_EPT; u++) {
-        const int e = tid + u * NT;
-        v[u] = T(0);
-        dst[u] = -1;
-        if (e < ne) {
-            const MvTermL& q = st[p2t[e / SC]];
-            const int qe = e - q.off * SC;
-            int p, i;
-            if (q.trans) {
-                p = qe % q.len;
-                i = qe / q.len;
-            } else {
-                p = qe / SC;
-                i = qe % SC;
+            for (int d = 1; d < WAVE; d <<= 1) {
+                const int v = __shfl_up(incl, d);
+                if (lane >= d) incl += v;
             }
-            const gptr<const T> A = gp(reinterpret_cast<const T*>(q.A));
-            if (i < no) v[u] = q.trans ? A[(q.lo + p) + (size_t)(o0 + i) * q.rows] : A[(o0 + i) + (size_t)(q.lo + p) * q.rows];
-            dst[u] = (q.off + p) * (SC + 1) + i;
+            L.off = incl - n;
+            const int total = rl(incl, WAVE - 1);
+            // the term of step s: the last one starting at or before it
+            auto at = [&](int s) { return __ballot(lane < nt && L.off <= s); };
+            MvStep<T> cur, nxt;
+            if (sub < total) mv_load<T, CT>(L, at(sub), sub, ch.o0, ch.no, ws, nrhs, r0, cur);
+            for (int s = sub; s < total; s += nw) {
+                const int s1 = s + nw;
+                if (s1 < total) mv_load<T, CT>(L, at(s1), s1, ch.o0, ch.no, ws, nrhs, r0, nxt);
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const double a = (double)cur.a[q];
+                    if (CT == 0) {
+                        acc1 = __builtin_amdgcn_mfma_f64_4x4x4f64(a, cur.x[0][q], acc1, 0, 0, 0);
+                    } else {
+#pragma unroll
+                        for (int c = 0; c < CT; c++)
+                            acc[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, cur.x[c][q], acc[c], 0, 0, 0);
+                    }
+                }
+                cur = nxt;
+            }
         }
     }
-    auto stage_x = [&](int r0, int rg) {
-        VT xv[2];
-        int xd[2];
+    if (nw > 1) {
+        double* mine = red + (size_t)(sub - 1) * WAVE * NACC + lane;
+        if (sub > 0) {
+            if (CT == 0) mine[0] = acc1;
 #pragma unroll
-        for (int u = 0; u < 2; u++) {
-            const int idx = tid + u * NT;
-            xd[u] = -1;
-            if (idx < total * rg) {
-                const int pos = idx / rg, r = idx % rg;
-                const MvTermL& q = st[p2t[pos]];
-                const int j = q.lo + (pos - q.off);
-                const int src = (!q.trans && q.perm) ? gp(q.perm)[j] : j;
-                xv[u] = ws[(size_t)(q.xsrc + src) * nrhs + r0 + r];
-                xd[u] = pos * RG_MAX + r;
-            }
+            for (int u = 0; u < (CT == 0 ? 0 : NACC); u++) mine[u * WAVE] = acc[u / 4][u % 4];
         }
-#pragma unroll
-        for (int u = 0; u < 2; u++)
-            if (xd[u] >= 0) (&xl[0][0])[xd[u]] = xv[u];
-    };
-    stage_x(0, min(RG_MAX, nrhs));
-#pragma unroll
-    for (int u = 0; u < MV_EPT; u++)
-        if (dst[u] >= 0) (&tile[0][0])[dst[u]] = v[u];
-    __syncthreads();
-    // 3. accumulate, per group of up to RG_MAX right-hand sides
-    for (int r0 = 0; r0 < nrhs; r0 += RG_MAX) {
-        const int rg = min(RG_MAX, nrhs - r0);
-        if (r0 > 0) {
-            __syncthreads();  // every read of xl for the previous group is done
-            stage_x(r0, rg);
-            __syncthreads();
-        }
-        VT acc[RG_MAX];
-#pragma unroll
-        for (int r = 0; r < RG_MAX; r++) acc[r] = VT(0);
-        // positions kp, kp + 4, ... < total (at most 16 per partition), unrolled so that the
-        // LDS reads run ahead; the sum order per output is the position order either way
-#pragma unroll
-        for (int q = 0; q < PW / NP; q++) {
-            const int p = kp + q * NP;
-            if (p < total) {
-                const VT a = tile[p][lane];
-#pragma unroll
-                for (int r = 0; r < RG_MAX; r++)
-                    if (r < rg) acc[r] += a * xl[p][r];
-            }
-        }
-        if (RED_IN_TILE) __syncthreads();  // every partition has read the tile
-        if (kp > 0)
-#pragma unroll
-            for (int r = 0; r < RG_MAX; r++) red[kp - 1][lane][r] = acc[r];
         __syncthreads();
-        if (kp == 0 && lane < no) {
-            if (pc.direct) {
-                VT* y = ws + (size_t)(pc.xdst + o0 + lane) * nrhs + r0;
-                for (int r = 0; r < rg; r++)
-                    mv_apply(y + r, pc.mode, ((acc[r] + red[0][lane][r]) + red[1][lane][r]) + red[2][lane][r]);
-            } else {
-                VT* y = partial + ((size_t)blockIdx.x * SC + lane) * nrhs + r0;
-                for (int r = 0; r < rg; r++) y[r] = ((acc[r] + red[0][lane][r]) + red[1][lane][r]) + red[2][lane][r];
+        if (sub == 0)
+            for (int w = 0; w < nw - 1; w++) {
+                const double* p = red + (size_t)w * WAVE * NACC + lane;
+                if (CT == 0) acc1 += p[0];
+#pragma unroll
+                for (int u = 0; u < (CT == 0 ? 0 : NACC); u++) acc[u / 4][u % 4] += p[u * WAVE];
             }
+    }
+    if (live && sub == 0) {
+        auto put = [&](int i, int r, double v) {  // output i of the chunk, right-hand side r
+            if (i >= ch.no || r >= nrhs) return;
+            const int o = ch.o0 + i;
+            const gptr<double> y = gp(ws) + (size_t)(ch.xdst + (ch.dperm ? gp(ch.dperm)[o] : o)) * nrhs + r;
+            *y = ch.mode == MV_SUB ? *y - v : v;
+        };
+        if (CT == 0) {  // 4x4x4: lane l holds output 4 ((l % 16) / 4) + l / 16, right-hand side l % 4
+            put(4 * ((lane & 15) >> 2) + (lane >> 4), lane & 3, acc1);
+        } else {  // 16x16x4: register v of lane l holds output l / 16 + 4 v, right-hand side l % 16
+#pragma unroll
+            for (int u = 0; u < NACC; u++)
+                put((lane >> 4) + 4 * (u % 4), r0 + 16 * (u / 4) + (lane & 15), acc[u / 4][u % 4]);
         }
-        __syncthreads();  // red is rewritten by the next group
     }
 }
 
-// Chunks with several pieces: add the pieces' partial sums in piece order, then apply.
-__global__ void __launch_bounds__(NT) k_mv_reduce(const MvGroup* groups, const MvChunk* chunks, const int* rchunks,
-                                                  const VT* partial, VT* ws, int nrhs) {
-    const MvChunk ch = chunks[rchunks[blockIdx.x]];
-    mv_chunk_reduce(ch, groups[ch.group], partial, ws, nrhs);
+// Consecutive workgroups run on different XCDs (block b on XCD b % 8): chunk ranges are dealt
+// out so that neighbouring chunks, which share sources and the cache lines of A's columns,
+// meet in one L2. Grid: (8 x workgroups per XCD, blocks of 16 CT right-hand sides).
+constexpr int XCDS = 8;
+template <typename T, int CT>
+__global__ void __launch_bounds__(1024) k_mv(MvDevPhase ph, double* ws, int nrhs) {
+    extern __shared__ double mv_red[];
+    constexpr int NACC = CT == 0 ? 1 : 4 * CT;
+    const int groups = blockDim.x / WAVE / ph.nw;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const int blk = (blockIdx.x % XCDS) * (gridDim.x / XCDS) + blockIdx.x / XCDS;
+    const int g = wv / ph.nw, ci = blk * groups + g;
+    mv_chunk<T, CT>(ph, ci, ci < ph.nchunks, wv % ph.nw, mv_red + (size_t)g * (ph.nw - 1) * WAVE * NACC, ws, nrhs,
+                    blockIdx.y * (CT == 0 ? 4 : 16 * CT));
+}
+
+// Consecutive phases of little work in one workgroup, a barrier between them instead of a
+// launch (about 4.5 us each in a replayed graph, against 2-3 us for such a phase here).
+template <typename T, int CT>
+__global__ void __launch_bounds__(1024) k_mv_tail(MvTail tail, double* ws, int nrhs) {
+    extern __shared__ double mv_red[];
+    constexpr int NACC = CT == 0 ? 1 : 4 * CT;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    for (int p = 0; p < tail.n; p++) {
+        const MvDevPhase ph = tail.ph[p];
+        const int groups = MV_NW_MAX / ph.nw, g = wv / ph.nw;
+        for (int r0 = 0; r0 < nrhs; r0 += (CT == 0 ? 4 : 16 * CT))
+            for (int c0 = 0; c0 < ph.nchunks; c0 += groups) {
+                mv_chunk<T, CT>(ph, c0 + g, c0 + g < ph.nchunks, wv % ph.nw,
+                                mv_red + (size_t)g * (ph.nw - 1) * WAVE * NACC, ws, nrhs, r0);
+                if (ph.nw > 1) __syncthreads();  // the partial sums are read before the next chunk's
+            }
+        __syncthreads();
+    }
 }
 
 // ---------------------------------------------------------------------------------------
 // Compact-WY factors of the Orthogonal ops (task layout in tasks.hpp): Ve = V with its unit
-// diagonal and zeros above; S = diag(1 / tau) + stril(Ve^T Ve); X = identity (the caller
-// then solves S X = I with the batched trsm, so that X = T^T).
+// diagonal and zeros above; S = -diag(1 / tau) - stril(Ve^T Ve).
 template <typename T>
 __global__ void __launch_bounds__(NT) k_wy_explicit(const WyTask* tasks) {
     const WyTask t = tasks[blockIdx.x];
@@ -299,15 +308,13 @@ __global__ void __launch_bounds__(NT) k_wy_explicit(const WyTask* tasks) {
         const int i = (int)(idx % t.m), c = (int)(idx / t.m);
         Ve[idx] = i == c ? T(1) : (i > c ? V[idx] : T(0));
     }
-    // S on and above the diagonal, X
+    // S on and above the diagonal
     const T* tau = reinterpret_cast<const T*>(t.tau);
     T* S = reinterpret_cast<T*>(t.S);
-    T* X = reinterpret_cast<T*>(t.X);
     const size_t kk = (size_t)t.k * t.k;
     for (size_t idx = (size_t)blockIdx.y * NT + threadIdx.x; idx < kk; idx += (size_t)gridDim.y * NT) {
         const int a = (int)(idx % t.k), c = (int)(idx / t.k);
-        if (a <= c) S[idx] = a == c ? T(1) / tau[a] : T(0);
-        X[idx] = a == c ? T(1) : T(0);
+        if (a <= c) S[idx] = a == c ? -(T(1) / tau[a]) : T(0);
     }
 }
 
@@ -344,7 +351,7 @@ __global__ void __launch_bounds__(NT) k_wy_gram(const WyTask* tasks, const int4*
 #pragma unroll
     for (int q = 0; q < 4; q++) {
         const int a = a0 + ta, c = c0 + tc0 + q;
-        if (a < k && c < k && a < c) S[c + (size_t)a * k] = (T)acc[q];
+        if (a < k && c < k && a < c) S[c + (size_t)a * k] = (T)-acc[q];
     }
 }
 
@@ -540,17 +547,37 @@ hipError_t launch_il2cm(const double* src, int N, int nrhs, double* dst, int ld,
     k_il2cm<<<grid_for((size_t)N * nrhs), NT, 0, st>>>(src, N, nrhs, dst, ld);
     return hipGetLastError();
 }
+// Right-hand sides per pass of a phase: 4, 16 or 32 (more run as several passes).
+template <typename F>
+static hipError_t mv_width(int nrhs, F&& f) {
+    if (nrhs <= 4) return f(std::integral_constant<int, 0>());
+    if (nrhs <= 16) return f(std::integral_constant<int, 1>());
+    return f(std::integral_constant<int, 2>());
+}
 template <typename T>
-hipError_t launch_mv(const MvGroup* d_groups, const MvChunk* d_chunks, const MvPiece* d_pieces, int npieces,
-                     const MvTerm* d_terms, const int* d_rchunks, int nreduce, double* ws, double* partial, int nrhs,
-                     hipStream_t st) {
-    if (npieces == 0) return hipSuccess;
-    if (nrhs <= RG_MAX) k_mv_piece<T, true><<<npieces, NT, 0, st>>>(d_pieces, d_terms, ws, partial, nrhs);
-    else k_mv_piece<T, false><<<npieces, NT, 0, st>>>(d_pieces, d_terms, ws, partial, nrhs);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess || nreduce == 0) return e;
-    k_mv_reduce<<<nreduce, NT, 0, st>>>(d_groups, d_chunks, d_rchunks, partial, ws, nrhs);
-    return hipGetLastError();
+hipError_t launch_mv(const MvDevPhase& ph, double* ws, int nrhs, hipStream_t st) {
+    if (ph.nchunks == 0) return hipSuccess;
+    return mv_width(nrhs, [&](auto ct) {
+        constexpr int CT = decltype(ct)::value, NACC = CT == 0 ? 1 : 4 * CT, W = CT == 0 ? 4 : 16 * CT;
+        const int waves = std::max(4, ph.nw), groups = waves / ph.nw;
+        const int nb = (ph.nchunks + groups - 1) / groups;
+        const dim3 grid((nb + XCDS - 1) / XCDS * XCDS, (nrhs + W - 1) / W);
+        const size_t lds = (size_t)groups * (ph.nw - 1) * WAVE * NACC * sizeof(double);
+        k_mv<T, CT><<<grid, waves * WAVE, lds, st>>>(ph, ws, nrhs);
+        return hipGetLastError();
+    });
+}
+template <typename T>
+hipError_t launch_mv_tail(const MvTail& tail, double* ws, int nrhs, hipStream_t st) {
+    if (tail.n == 0) return hipSuccess;
+    return mv_width(nrhs, [&](auto ct) {
+        constexpr int CT = decltype(ct)::value, NACC = CT == 0 ? 1 : 4 * CT;
+        size_t lds = 0;
+        for (int p = 0; p < tail.n; p++)
+            lds = std::max(lds, (size_t)(MV_NW_MAX - MV_NW_MAX / tail.ph[p].nw) * WAVE * NACC * sizeof(double));
+        k_mv_tail<T, CT><<<1, MV_NW_MAX * WAVE, lds, st>>>(tail, ws, nrhs);
+        return hipGetLastError();
+    });
 }
 template <typename T>
 hipError_t launch_wy(const WyTask* d_tasks, int ntasks, const int4* d_tiles, int ntiles, hipStream_t st) {
@@ -633,8 +660,8 @@ hipError_t launch_gather_f64(const int* idx, const double* src, long long n, dou
 #define SPAND_SOLVE_INST(T)                                                                                  \
     template hipError_t launch_perm_in<T>(const double*, size_t, size_t, int, const int*, int, double*, hipStream_t); \
     template hipError_t launch_perm_out<T>(const double*, const int*, int, int, double*, size_t, size_t, hipStream_t); \
-    template hipError_t launch_mv<T>(const MvGroup*, const MvChunk*, const MvPiece*, int, const MvTerm*, const int*, \
-                                     int, double*, double*, int, hipStream_t);                             \
+    template hipError_t launch_mv<T>(const MvDevPhase&, double*, int, hipStream_t);                          \
+    template hipError_t launch_mv_tail<T>(const MvTail&, double*, int, hipStream_t);                         \
     template hipError_t launch_wy<T>(const WyTask*, int, const int4*, int, hipStream_t);                    \
     template hipError_t launch_merge<T>(const MergeTask*, int, const int2*, double*, int, int, hipStream_t);
 SPAND_SOLVE_INST(float)

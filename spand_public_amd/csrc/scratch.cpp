@@ -1,7 +1,7 @@
 // Static device workspace of the allocation-free preconditioner apply
 // (spand_solve_device_noalloc): callers that cannot allocate device memory (code under HIP
 // graph capture, serving loops, harnesses that forbid hipMalloc) apply M^{-1} with the
-// segments and partial sums placed in this file-scope array instead of the tree's own
+// segments placed in this file-scope array instead of the tree's own
 // workspace. Every GPU the library runs on holds one copy of SCRATCH_BYTES until the
 // process ends; calls that overlap on one GPU share it and race.
 #include "scratch.hpp"

@@ -50,12 +50,14 @@ struct GetrfTask {
 
 // One Schur-complement target tile: C[r0:r0+tm, c0:c0+tn] of a block C (ldc rows) receives
 // contributions [k0, k1) in order, each C -= opA(A) opB(B) (gemm / syrk, src/util.cpp:122-156).
-// lower = 1 restricts the update to the lower triangle (syrk on a diagonal block).
+// SCHUR_LOWER restricts the update to the lower triangle (syrk on a diagonal block);
+// SCHUR_CLEAR takes C as zero before the first contribution, whatever it holds.
+enum SchurFlags { SCHUR_LOWER = 1, SCHUR_CLEAR = 2 };
 struct SchurTile {
     void* C;
     int ldc;
     int r0, c0, tm, tn;
-    int lower;
+    int lower;   // SCHUR_LOWER, SCHUR_CLEAR
     int k0, k1;
 };
 struct SchurContrib {
@@ -125,62 +127,52 @@ struct CopyTask {
 // Preconditioner apply (Tree::solve, src/tree.cpp:1610-1635). Vectors are stored
 // interleaved: element i of right-hand side r lives at x[(xoff + i) * nrhs + r].
 //
-// Every recorded op is a matrix-vector product on segments, applied per ND level and op
-// kind in one "mv phase": a set of groups x[dst] (op)= sum_k op(A_k) x[src_k], split into
-// chunks of 64 outputs and, along the inner dimension, into pieces of bounded work, one
-// workgroup each. A chunk with one piece writes its destination directly; otherwise the
-// pieces write partial sums that a second launch adds in piece order (deterministic).
-//   ScalingLLT   (src/operations.cpp:95-103):  x := Linv x,        x := Linv^T x
-//   ScalingPLUQ  (src/operations.cpp:114-121): x := Linv x[perm],  x := (U^{-T})^T x
-//   Gemm*        (src/operations.cpp:31-93):   x_n -= A x_s / A^T x_s
-//   Orthogonal   (src/operations.cpp:149-158): Q = I - V T V^T (compact WY over all kept
-//                reflectors), X = T^T: y := -V^T x, z := -X y (fwd) or -X^T y (bwd), x -= V z
+// The recorded ops of a level run as three mv phases per direction, each a set of groups
+// x[dst] (op)= sum_k op(A_k) x[src_k] whose destinations are never sources of the same
+// phase, so one launch covers a phase whatever the order of its workgroups:
+//   E   ScalingLLT / ScalingPLUQ of the eliminated clusters (src/operations.cpp:95-121):
+//       xe := Linv x[perm] into a segment of its own, back x := Linv^T xe or (U^{-T})^T xe
+//   G   Gemm* (src/operations.cpp:31-93): x_n -= A xe, back xe -= A^T x_n
+//   W   the scaling and the Orthogonal op of a remaining cluster in one matrix
+//       (src/operations.cpp:95-121,149-158), W = Q^T Linv: its first r outputs (the kept
+//       rank) go to the cluster's place in its parent's segment (Merge,
+//       src/operations.cpp:166-192), the rest to the sibling's segment; back x := W^T y
 struct MvTerm {
-    const void* A;     // rows x cols, ld rows, the factor's element type
+    const void* A;     // op(A)'s element (output o, inner j): A[o + j ld], transposed A[j + o ld]
     const int* perm;   // not transposed: inner index j reads source element perm[j]
-    int rows, cols;
+    int ld, len;       // column stride of A, inner positions
     int xsrc;          // source segment
-    int trans;         // 0: output = row of A, inner = column; 1: output = column, inner = row
-    int tri;           // inner-range clip of a triangular A for outputs [o0, o0 + 64):
-                       // 1 inner < o0 + 64, 2 inner >= o0, 0 none
-    int pad;
+    int flags;         // MV_TRANS, and the inner-range clip of a triangular A for the outputs
+                       // [o0, o0 + 16): MV_TRI_LO inner < o0 + 16, MV_TRI_UP inner >= o0
 };
-enum MvMode { MV_SUB = 0, MV_SETNEG = 1, MV_SET = 2 };  // x -= s, x = -s, x = s
-struct MvGroup {
-    int xdst, n;  // destination segment and length
-    int k0, k1;   // term range
-    int mode;
-    int pad;
-    const int* dperm;  // nullptr, or output o goes to xdst + dperm[o] (then always through
-                       // the partial sums: a permuted destination is never written directly)
-};
-struct MvChunk {
-    int group, o0;  // outputs [o0, o0 + 64) of the group
-    int p0, p1;     // its pieces (indices into the phase's piece array)
-};
-struct MvPiece {
-    int chunk;
-    int k0, k1;    // terms; when k1 == k0 + 1 only inner indices [j0, j1) of term k0
-    int j0, j1;
-    int direct;    // the chunk's only piece: writes the destination itself
-    // copies of its chunk / group fields, so that a workgroup reads one record
-    int o0, no;    // the chunk's first output and output count
+enum MvFlags { MV_TRANS = 1, MV_TRI_LO = 2, MV_TRI_UP = 4 };
+enum MvMode { MV_SUB = 0, MV_SET = 1 };  // x -= s, x = s
+struct MvChunk {       // up to MV_ROWS outputs of one group
+    int k0, k1;        // terms of the group
+    int o0, no;        // outputs [o0, o0 + no)
     int xdst, mode;
+    const int* dperm;  // nullptr, or output o goes to xdst + dperm[o]
+};
+// One mv phase: its chunks, and the wavefronts that share a chunk's inner positions.
+struct MvDevPhase {
+    const MvChunk* chunks;
+    const MvTerm* terms;
+    int nchunks, nw;
 };
 // Explicit Householder vectors V (unit diagonal, zeros above) and the compact-WY factor of
 // one Orthogonal op, built at factorization. Q = H_0 H_1 ... H_{k-1} = I - V T V^T with T
-// upper triangular and T^{-1} = diag(1 / tau) + striu(V^T V) (the UT transform); the solve
-// stores X = T^T = S^{-1}, S = T^{-T} = diag(1 / tau) + stril(V^T V), computed by a
-// triangular solve against the identity.
+// upper triangular and T^{-1} = diag(1 / tau) + striu(V^T V) (the UT transform), so
+// W = Q^T Linv = Linv - V Z with Z = S^{-1} V^T Linv, S = diag(1 / tau) + stril(V^T V).
+// Stored is -S: Y = -V^T Linv is what the Schur kernel leaves in a cleared block, and the
+// triangular solve (-S) Z = Y gives Z.
 struct WyTask {
     const void* V;    // m x k reflectors as stored by the QR (R on and above the diagonal)
     const void* tau;
     void* Ve;         // m x k explicit V
-    void* S;          // k x k lower: diag(1 / tau) + stril(V^T V)
-    void* X;          // k x k, set to the identity here (then S^{-1} by the trsm)
+    void* S;          // k x k lower: -diag(1 / tau) - stril(V^T V)
     int m, k;
 };
-struct MergeTask {  // Merge (src/operations.cpp:166-192)
+struct MergeTask {  // Merge (src/operations.cpp:166-192) of children without a W phase
     int pxoff;
     int c0, c1;  // range into (child xoff, child size) pairs
     int pad;

@@ -500,11 +500,19 @@ void Tree::factorize() {
 }
 
 // Host-side records of the solve ops of one level, turned into mv phases at its end.
-struct TrsvTask {  // ScalingLLT / ScalingPLUQ of one cluster
+struct TrsvTask {  // ScalingLLT / ScalingPLUQ of one eliminated cluster
     const void* L;   // forward factor (explicit inverse, lower)
     const void* Lb;  // backward factor (lower, applied transposed)
     const int* perm;
-    int n, xoff;
+    int n, xoff, eoff;  // the cluster's segment, and the segment of its scaled right-hand side
+};
+struct ScaleTask {  // ScalingLLT / ScalingPLUQ and Orthogonal of one remaining cluster
+    const void* W;   // forward: Q^T L^{-1} (L^{-1}, lower, without an Orthogonal op)
+    const void* Wb;  // backward, applied transposed: Q^T U^{-T} (W for an SPD tree)
+    const int* perm;
+    int cluster, n, r;      // size and kept rank
+    int xoff, dst, sib;     // own segment, place in the parent's, the sibling's segment
+    bool q;                 // an Orthogonal op with a nonzero rank: W and Wb are full
 };
 struct GemvGroup { int xdst, n, k0, k1; };
 struct GemvTerm {
@@ -512,70 +520,54 @@ struct GemvTerm {
     int rows, cols, xsrc, trans;
 };
 
-// One mv phase on the host: groups and terms, then split into chunks and pieces.
+// One mv phase on the host: terms, and chunks of MV_ROWS outputs.
 struct MvPlan {
-    std::vector<MvGroup> groups;
     std::vector<MvTerm> terms;
     std::vector<MvChunk> chunks;
-    std::vector<MvPiece> pieces;
-    std::vector<int> rchunks;
     int family = KF_GEMV;
-    bool inplace = false;  // destinations are also sources: every chunk goes through partials
+    int nw = 1;
+    long long steps = 0;  // MV_STEP-wide steps over all chunks
+    size_t esz = sizeof(double);
     SweepWork work;
 
-    void split(size_t esz) {
-        const int W = MV_PIECE_WORK;
-        for (int gi = 0; gi < (int)groups.size(); gi++) {
-            const MvGroup& g = groups[gi];
-            for (int o0 = 0; o0 < g.n; o0 += SOLVE_CHUNK) {
-                const int no = std::min(SOLVE_CHUNK, g.n - o0);
-                const int ci = (int)chunks.size(), p0 = (int)pieces.size();
-                int pk0 = -1, pwork = 0;
-                auto flush = [&](int kend) {
-                    if (pk0 >= 0) {
-                        const MvTerm& t = terms[pk0];
-                        pieces.push_back({ci, pk0, kend, 0, t.trans ? t.rows : t.cols, 0, 0, 0, 0, 0});
-                    }
-                    pk0 = -1;
-                    pwork = 0;
-                };
-                for (int k = g.k0; k < g.k1; k++) {
-                    const MvTerm& t = terms[k];
-                    int lo = 0, hi = t.trans ? t.rows : t.cols;
-                    if (t.tri == 1) hi = std::min(hi, o0 + SOLVE_CHUNK);
-                    if (t.tri == 2) lo = std::max(lo, o0);
-                    const int len = std::max(0, hi - lo);
-                    work.mat_bytes += (double)no * len * esz;
-                    work.flops += 2.0 * no * len;
-                    work.vec_elems += len;
-                    if (len > W) {  // a long term alone: pieces of W inner indices
-                        flush(k);
-                        for (int j = lo; j < hi; j += W)
-                            pieces.push_back({ci, k, k + 1, j, std::min(hi, j + W), 0, 0, 0, 0, 0});
-                    } else {
-                        // short terms share a piece: at most W inner indices and
-                        // MV_PIECE_TERMS terms (one lane of a wavefront reads each record)
-                        if (pk0 >= 0 && (pwork + len > W || k - pk0 >= MV_PIECE_TERMS)) flush(k);
-                        if (pk0 < 0) pk0 = k;
-                        pwork += len;
-                    }
-                }
-                flush(g.k1);
-                const int p1 = (int)pieces.size();
-                if (p1 == p0) continue;
-                chunks.push_back({gi, o0, p0, p1});
-                for (int q = p0; q < p1; q++) {
-                    pieces[q].o0 = o0;
-                    pieces[q].no = no;
-                    pieces[q].xdst = g.xdst;
-                    pieces[q].mode = g.mode;
-                }
-                work.vec_elems += 2.0 * no;
-                if (p1 - p0 == 1 && !inplace && !g.dperm) pieces[p0].direct = 1;
-                else rchunks.push_back(ci);
+    // n outputs at xdst from the terms [k0, terms.size())
+    void group(int xdst, int n, int k0, int mode, const int* dperm = nullptr) {
+        const int k1 = (int)terms.size();
+        for (int o0 = 0; o0 < n; o0 += MV_ROWS) {
+            const int no = std::min(MV_ROWS, n - o0);
+            chunks.push_back({k0, k1, o0, no, xdst, mode, dperm});
+            long long st = 0;
+            for (int k = k0; k < k1; k++) {
+                const MvTerm& t = terms[k];
+                const int lo = (t.flags & MV_TRI_UP) ? std::min(t.len, o0) : 0;
+                const int hi = (t.flags & MV_TRI_LO) ? std::min(t.len, o0 + MV_ROWS) : t.len;
+                const int len = std::max(0, hi - lo);
+                work.mat_bytes += (double)no * len * esz;
+                work.flops += 2.0 * no * len;
+                work.vec_elems += len;
+                st += (len + MV_STEP - 1) / MV_STEP;
             }
+            work.vec_elems += 2.0 * no;
+            steps += st;
+            steps_max = std::max(steps_max, st);
         }
     }
+    // Wavefronts per chunk: enough to have MV_WAVES in flight over the device (16 on each of
+    // 256 CUs), while the longest chunk has a step for each; the wavefronts of one workgroup
+    // for a phase of few steps, which runs in one. 2048 / 4096 / 8192 / 16384 wavefronts: 854
+    // / 805 / 828 / 844 us for the FP64 apply of the 64^3 Laplacian on 4 columns; two steps
+    // each instead of one: 836 us at 4096.
+    void finish() {
+        constexpr long long MV_WAVES = 4096;
+        if (steps <= MV_TAIL_STEPS) {
+            while (nw < MV_NW_MAX && (long long)chunks.size() * nw < MV_NW_MAX && steps_max >= 2 * nw) nw *= 2;
+            return;
+        }
+        while (nw < MV_NW_MAX && (long long)chunks.size() * nw < MV_WAVES && steps_max >= 2 * nw) nw *= 2;
+    }
+
+  private:
+    long long steps_max = 0;
 };
 
 // Stable grouping of n items by key (keys in [0, nkeys)): groups in order of first
@@ -682,21 +674,20 @@ static long long env_or(const char* name, long long dflt) {
     return (e && *e) ? std::strtoll(e, nullptr, 10) : dflt;
 }
 
-// One Orthogonal op of the solve: y = -V^T x, z = -T^T y (forward) or -T y (backward),
-// x -= V z, with X = T^T stored (compact WY over its kept reflectors).
+// One Orthogonal op to fold into its cluster's scaling (scale: index into sv_scale).
 struct QOp {
     const void* Ve;
-    const void* X;
-    int m, k, xoff, yoff;
+    const void* S;
+    int m, k, cluster;
 };
 
 // One level's solve-plan inputs, kept on the host for the transposed phases (built and
 // uploaded at the first transposed solve).
 struct HostPhases {
-    std::vector<TrsvTask> sv_elim, sv_scale;
+    std::vector<TrsvTask> sv_elim;
+    std::vector<ScaleTask> sv_scale;
     std::vector<GemvGroup> fwd_groups, bwd_groups;
     std::vector<GemvTerm> fwd_t, bwd_terms;
-    std::vector<QOp> qops;
 };
 
 // Host side of one level's preconditioner-apply plan, before upload.
@@ -705,77 +696,81 @@ struct SolvePlanHost {
     HostPhases inputs;
     std::vector<MergeTask> mt;
     std::vector<int2> mchildren;
-    long long max_pieces = 0;
 };
 
-// Phase builders. A triangular sweep (ScalingLLT / ScalingPLUQ of each cluster): forward
-// x := L x with the gathered source P^T x, backward x := Lb^T x.
-static MvPlan trsv_phase(const std::vector<TrsvTask>& v, bool backward) {
+// Phase builders. E: the eliminated clusters' scaling, between a cluster's segment and the
+// segment of its scaled right-hand side. down: x := F^T xe, else xe := F x, with F the forward
+// (fwd) or backward factor; a row permutation is the forward factor's (P^T on its input).
+static MvPlan elim_phase(size_t esz, const std::vector<TrsvTask>& v, bool fwd, bool down) {
     MvPlan m;
+    m.esz = esz;
     m.family = KF_TRMV;
-    m.inplace = true;
     for (auto& t : v) {
         const int k0 = (int)m.terms.size();
-        if (!backward) m.terms.push_back({t.L, t.perm, t.n, t.n, t.xoff, 0, 1, 0});
-        else m.terms.push_back({t.Lb, nullptr, t.n, t.n, t.xoff, 1, 2, 0});
-        m.groups.push_back({t.xoff, t.n, k0, k0 + 1, MV_SET, 0, nullptr});
+        const void* F = fwd ? t.L : t.Lb;
+        const int* p = fwd ? t.perm : nullptr;
+        if (!down) {
+            m.terms.push_back({F, p, t.n, t.n, t.xoff, MV_TRI_LO});
+            m.group(t.eoff, t.n, k0, MV_SET);
+        } else {
+            m.terms.push_back({F, nullptr, t.n, t.n, t.eoff, MV_TRANS | MV_TRI_UP});
+            m.group(t.xoff, t.n, k0, MV_SET, p);
+        }
     }
+    m.finish();
     return m;
 }
 
-// x_dst -= sum_k op(A_k) x_src(k) for every group
-static MvPlan gemv_phase(const std::vector<GemvGroup>& gs, const std::vector<GemvTerm>& ts) {
+// W: the remaining clusters' scaling and Orthogonal op, between a cluster's segment and its
+// kept (parent's) and eliminated (sibling's) places. down: x := W^T y, else y := W x.
+static MvPlan scale_phase(size_t esz, const std::vector<ScaleTask>& v, bool fwd, bool down) {
     MvPlan m;
+    m.esz = esz;
+    m.family = KF_QAPPLY;
+    for (auto& t : v) {
+        const char* W = reinterpret_cast<const char*>(fwd ? t.W : t.Wb);
+        const int* p = fwd ? t.perm : nullptr;
+        // without an Orthogonal op W is lower triangular and its outputs go to one place
+        const bool split = t.q;
+        const int r = split ? t.r : t.n, dst = split || t.r > 0 ? t.dst : t.sib;
+        const int tri = split ? 0 : (down ? MV_TRI_UP : MV_TRI_LO);
+        int k0 = (int)m.terms.size();
+        if (!down) {
+            m.terms.push_back({W, p, t.n, t.n, t.xoff, tri});
+            m.group(dst, r, k0, MV_SET);
+            if (split) {
+                k0 = (int)m.terms.size();
+                m.terms.push_back({W + (size_t)r * esz, p, t.n, t.n, t.xoff, 0});
+                m.group(t.sib, t.n - r, k0, MV_SET);
+            }
+        } else {
+            m.terms.push_back({W, nullptr, t.n, r, dst, MV_TRANS | tri});
+            if (split) m.terms.push_back({W + (size_t)r * esz, nullptr, t.n, t.n - r, t.sib, MV_TRANS});
+            m.group(t.xoff, t.n, k0, MV_SET, p);
+        }
+    }
+    m.finish();
+    return m;
+}
+
+// G: x_dst -= sum_k op(A_k) x_src(k) for every group
+static MvPlan gemv_phase(size_t esz, const std::vector<GemvGroup>& gs, const std::vector<GemvTerm>& ts) {
+    MvPlan m;
+    m.esz = esz;
     m.family = KF_GEMV;
     for (auto& g : gs) {
         const int k0 = (int)m.terms.size();
         for (int k = g.k0; k < g.k1; k++)
-            m.terms.push_back({ts[k].A, nullptr, ts[k].rows, ts[k].cols, ts[k].xsrc, ts[k].trans, 0, 0});
-        m.groups.push_back({g.xdst, g.n, k0, (int)m.terms.size(), MV_SUB, 0, nullptr});
+            m.terms.push_back({ts[k].A, nullptr, ts[k].rows, ts[k].trans ? ts[k].rows : ts[k].cols, ts[k].xsrc,
+                               ts[k].trans ? MV_TRANS : 0});
+        m.group(g.xdst, g.n, k0, MV_SUB);
     }
-    return m;
-}
-
-// Orthogonal ops, step 0..2: y = -V^T x, z = -X y (forward) or -X^T y (backward), x -= V z
-static MvPlan q_phase(const std::vector<QOp>& qops, int step, bool backward) {
-    MvPlan m;
-    m.family = KF_QAPPLY;
-    for (auto& q : qops) {
-        const int k0 = (int)m.terms.size();
-        if (step == 0) {
-            m.terms.push_back({q.Ve, nullptr, q.m, q.k, q.xoff, 1, 2, 0});
-            m.groups.push_back({q.yoff, q.k, k0, k0 + 1, MV_SETNEG, 0, nullptr});
-        } else if (step == 1) {  // X = T^T lower: z = -X y (fwd), -X^T y (bwd)
-            m.terms.push_back({q.X, nullptr, q.k, q.k, q.yoff, backward ? 1 : 0, backward ? 2 : 1, 0});
-            m.groups.push_back({q.yoff + q.k, q.k, k0, k0 + 1, MV_SETNEG, 0, nullptr});
-        } else {
-            m.terms.push_back({q.Ve, nullptr, q.m, q.k, q.yoff + q.k, 0, 1, 0});
-            m.groups.push_back({q.xoff, q.m, k0, k0 + 1, MV_SUB, 0, nullptr});
-        }
-    }
-    return m;
-}
-
-// The transpose of trsv_phase: (L P^T)^T = P L^T (P as a permuted destination), (Lb^T)^T = Lb.
-static MvPlan trsv_phase_t(const std::vector<TrsvTask>& v, bool backward) {
-    MvPlan m;
-    m.family = KF_TRMV;
-    m.inplace = true;
-    for (auto& t : v) {
-        const int k0 = (int)m.terms.size();
-        if (!backward) {
-            m.terms.push_back({t.L, nullptr, t.n, t.n, t.xoff, 1, 2, 0});
-            m.groups.push_back({t.xoff, t.n, k0, k0 + 1, MV_SET, 0, t.perm});
-        } else {
-            m.terms.push_back({t.Lb, nullptr, t.n, t.n, t.xoff, 0, 1, 0});
-            m.groups.push_back({t.xoff, t.n, k0, k0 + 1, MV_SET, 0, nullptr});
-        }
-    }
+    m.finish();
     return m;
 }
 
 // The transpose of gemv_phase: x_src(k) -= op(A_k)^T x_dst, grouped by source segment.
-static MvPlan gemv_phase_t(const std::vector<GemvGroup>& gs, const std::vector<GemvTerm>& ts) {
+static MvPlan gemv_phase_t(size_t esz, const std::vector<GemvGroup>& gs, const std::vector<GemvTerm>& ts) {
     struct TT {
         int dst, n;
         GemvTerm t;
@@ -788,73 +783,52 @@ static MvPlan gemv_phase_t(const std::vector<GemvGroup>& gs, const std::vector<G
             items.push_back({t.xsrc, n_in, GemvTerm{t.A, t.rows, t.cols, g.xdst, t.trans ? 0 : 1}});
         }
     std::stable_sort(items.begin(), items.end(), [](const TT& a, const TT& b) { return a.dst < b.dst; });
-    MvPlan m;
-    m.family = KF_GEMV;
+    std::vector<GemvGroup> tg;
+    std::vector<GemvTerm> tt;
     for (size_t q = 0; q < items.size();) {
-        const int k0 = (int)m.terms.size();
-        const int dst = items[q].dst, n = items[q].n;
-        for (; q < items.size() && items[q].dst == dst; q++) {
-            const GemvTerm& t = items[q].t;
-            m.terms.push_back({t.A, nullptr, t.rows, t.cols, t.xsrc, t.trans, 0, 0});
-        }
-        m.groups.push_back({dst, n, k0, (int)m.terms.size(), MV_SUB, 0, nullptr});
+        const int k0 = (int)tt.size(), dst = items[q].dst, n = items[q].n;
+        for (; q < items.size() && items[q].dst == dst; q++) tt.push_back(items[q].t);
+        tg.push_back({dst, n, k0, (int)tt.size()});
     }
-    return m;
+    return gemv_phase(esz, tg, tt);
 }
 
-// The level's mv phases: forward {trsv Elim, gemv, trsv Scale, Q 0..2}, backward
-// {Q 0..2, trsv Scale', gemv, trsv Elim'}, each split into chunks and pieces. The inputs
-// are kept for the transposed phases.
+// The level's mv phases: forward E, G, W, backward W', G', E'. The inputs are kept for the
+// transposed phases.
 static SolvePlanHost build_solve_plan(size_t esz, HostPhases in, std::vector<MergeTask> mt,
                                       std::vector<int2> mchildren) {
     SolvePlanHost h;
-    h.fwd.push_back(trsv_phase(in.sv_elim, false));
-    h.fwd.push_back(gemv_phase(in.fwd_groups, in.fwd_t));
-    h.fwd.push_back(trsv_phase(in.sv_scale, false));
-    for (int q = 0; q < 3; q++) h.fwd.push_back(q_phase(in.qops, q, false));
-    for (int q = 0; q < 3; q++) h.bwd.push_back(q_phase(in.qops, q, true));
-    h.bwd.push_back(trsv_phase(in.sv_scale, true));
-    h.bwd.push_back(gemv_phase(in.bwd_groups, in.bwd_terms));
-    h.bwd.push_back(trsv_phase(in.sv_elim, true));
-    for (auto* v : {&h.fwd, &h.bwd})
-        for (auto& m : *v) {
-            m.split(esz);
-            h.max_pieces = std::max(h.max_pieces, (long long)m.pieces.size());
-        }
+    h.fwd.push_back(elim_phase(esz, in.sv_elim, true, false));
+    h.fwd.push_back(gemv_phase(esz, in.fwd_groups, in.fwd_t));
+    h.fwd.push_back(scale_phase(esz, in.sv_scale, true, false));
+    h.bwd.push_back(scale_phase(esz, in.sv_scale, false, true));
+    h.bwd.push_back(gemv_phase(esz, in.bwd_groups, in.bwd_terms));
+    h.bwd.push_back(elim_phase(esz, in.sv_elim, false, true));
     h.mt = std::move(mt);
     h.mchildren = std::move(mchildren);
     h.inputs = std::move(in);
     return h;
 }
 
-// The adjoint apply's phases of one level. Forward level l applies F = Q S G E (E first),
-// backward B = E' G' S' Q' (Q' first); M^{-T} runs B^T (E'^T, G'^T, S'^T, Q'^T = the forward
-// Q) going up and F^T (Q^T = the backward Q, S^T, G^T, E^T) coming down.
-static void build_transposed(size_t esz, const HostPhases& in, std::vector<MvPlan>& up, std::vector<MvPlan>& down,
-                             long long& max_pieces) {
-    up.push_back(trsv_phase_t(in.sv_elim, true));
-    up.push_back(gemv_phase_t(in.bwd_groups, in.bwd_terms));
-    up.push_back(trsv_phase_t(in.sv_scale, true));
-    for (int q = 0; q < 3; q++) up.push_back(q_phase(in.qops, q, false));
-    for (int q = 0; q < 3; q++) down.push_back(q_phase(in.qops, q, true));
-    down.push_back(trsv_phase_t(in.sv_scale, false));
-    down.push_back(gemv_phase_t(in.fwd_groups, in.fwd_t));
-    down.push_back(trsv_phase_t(in.sv_elim, false));
-    for (auto* v : {&up, &down})
-        for (auto& m : *v) {
-            m.split(esz);
-            max_pieces = std::max(max_pieces, (long long)m.pieces.size());
-        }
+// The adjoint apply's phases of one level. Forward level l applies F = W G E (E first),
+// backward B = E' G' W' (W' first); M^{-T} runs B^T (E'^T, G'^T, W'^T) going up and F^T (W^T,
+// G^T, E^T) coming down.
+static void build_transposed(size_t esz, const HostPhases& in, std::vector<MvPlan>& up, std::vector<MvPlan>& down) {
+    up.push_back(elim_phase(esz, in.sv_elim, false, false));
+    up.push_back(gemv_phase_t(esz, in.bwd_groups, in.bwd_terms));
+    up.push_back(scale_phase(esz, in.sv_scale, false, false));
+    down.push_back(scale_phase(esz, in.sv_scale, true, true));
+    down.push_back(gemv_phase_t(esz, in.fwd_groups, in.fwd_t));
+    down.push_back(elim_phase(esz, in.sv_elim, true, true));
 }
 
 // Uploads phase lists (one Packer) and returns their device descriptors, in order.
 static std::vector<std::vector<MvPhase>> upload_phases(Tree& tree, std::vector<std::vector<MvPlan>*> lists,
                                                        void* (Tree::*upload)(const Packer&), Packer& ps,
                                                        void** base) {
-    std::vector<std::array<size_t, 5>> offs;
+    std::vector<std::array<size_t, 2>> offs;
     for (auto* v : lists)
-        for (auto& m : *v)
-            offs.push_back({ps.add(m.groups), ps.add(m.terms), ps.add(m.chunks), ps.add(m.pieces), ps.add(m.rchunks)});
+        for (auto& m : *v) offs.push_back({ps.add(m.terms), ps.add(m.chunks)});
     void* dsv = (tree.*upload)(ps);
     *base = dsv;
     std::vector<std::vector<MvPhase>> out;
@@ -863,15 +837,10 @@ static std::vector<std::vector<MvPhase>> upload_phases(Tree& tree, std::vector<s
         out.emplace_back();
         for (auto& m : *v) {
             const auto& o = offs[oi++];
-            if (m.pieces.empty()) continue;
+            if (m.chunks.empty()) continue;
             MvPhase ph;
-            ph.groups = Packer::at<MvGroup>(dsv, o[0]);
-            ph.terms = Packer::at<MvTerm>(dsv, o[1]);
-            ph.chunks = Packer::at<MvChunk>(dsv, o[2]);
-            ph.pieces = Packer::at<MvPiece>(dsv, o[3]);
-            ph.rchunks = Packer::at<int>(dsv, o[4]);
-            ph.npieces = (int)m.pieces.size();
-            ph.nreduce = (int)m.rchunks.size();
+            ph.d = {Packer::at<MvChunk>(dsv, o[1]), Packer::at<MvTerm>(dsv, o[0]), (int)m.chunks.size(), m.nw};
+            ph.steps = m.steps;
             ph.family = m.family;
             ph.w = m.work;
             out.back().push_back(ph);
@@ -896,19 +865,18 @@ void Tree::upload_solve_plan(int level, void* host_plan) {
     lsv.merge = Packer::at<MergeTask>(dsv, s_m);
     lsv.n_merge = (int)h.mt.size();
     lsv.children = Packer::at<int2>(dsv, s_mc);
-    max_pieces_ = std::max(max_pieces_, h.max_pieces);
     if (fsymm_ != 0) tplans_[level].reset(new HostPhases(std::move(h.inputs)));
 }
 
 // Builds and uploads the transposed phases of every level (first transposed solve after a
-// factorization). The partial-sum area grows with them if needed.
+// factorization).
 void Tree::upload_transposed() {
     const size_t esz = fprec_ == 0 ? sizeof(double) : sizeof(float);
     bool any = false;
     for (int l = 0; l < nlevels_; l++) {
         if (!tplans_[l]) continue;
         std::vector<MvPlan> up, down;
-        build_transposed(esz, *tplans_[l], up, down, max_pieces_);
+        build_transposed(esz, *tplans_[l], up, down);
         Packer ps;
         void* dsv = nullptr;
         auto ph = upload_phases(*this, {&up, &down}, &Tree::upload_tasks, ps, &dsv);
@@ -957,7 +925,8 @@ struct LevelPlan {
     std::vector<int> fill_edges;
     long long fill_elems = 0;
     std::vector<long long> fill_off;  // by position in fill_edges
-    std::vector<TrsvTask> sv_elim, sv_scale;
+    std::vector<TrsvTask> sv_elim;
+    std::vector<ScaleTask> sv_scale;
     std::vector<CopyTask> inv_init;  // identity blocks that become explicit inverses L^{-1}
     std::vector<std::pair<int, GemvTerm>> fwd_list;  // (destination cluster, term), in op order
     std::vector<GemvGroup> bwd_groups;
@@ -991,7 +960,6 @@ struct LevelPlan {
     std::vector<QOp> qops;
     std::vector<WyTask> wy;
     std::vector<int4> wy_tiles;
-    std::vector<TrsmTask> wy_trsm;
     std::vector<MergeTask> mt;
     std::vector<int2> mchildren;
     int left = 0;  // dofs left after the level
@@ -1163,6 +1131,8 @@ void Tree::plan_elimination(LevelPlan<T>& L) {
         const int n = s.size;
         // edges_ may grow (fill-in) below: keep the pivot block pointer, not a reference
         const HEdge piv = edges_[s.out[0]];
+        const int eoff = (int)ws_len_;  // the scaled right-hand side of the apply
+        ws_len_ += n;
         if (piv.ident) throw Error(ERR_STATE, "internal: identity pivot on an eliminated cluster");
         if (gen) {
             // getf_cluster + panel_getf + gemm_edges, PLU branch (src/tree.cpp:929-956)
@@ -1204,7 +1174,7 @@ void Tree::plan_elimination(LevelPlan<T>& L) {
                 push_trsm(trsmE, piv.A, Li, n, n, 0, sizeof(T));
                 push_trsm(trsmE, Ut, Wi, n, n, 0, sizeof(T));
                 lst.flops_trsm += 2.0 * n * n * n;
-                sv_elim.push_back({Li, Wi, pp, n, (int)s.xoff});
+                sv_elim.push_back({Li, Wi, pp, n, (int)s.xoff, eoff});
             }
             factor_bytes_ += (size_t)n * (n + 1) * sizeof(T) + (size_t)n * sizeof(int);
             std::vector<GemvTerm> mine;
@@ -1213,7 +1183,7 @@ void Tree::plan_elimination(LevelPlan<T>& L) {
                 ops_.push_back({OP_GEMM_OUT, c, nb, n, size(nb), size(nb), n, ilvl_, edges_[e].A, nullptr});
                 factor_bytes_ += (size_t)n * size(nb) * sizeof(T);
                 if (n > 0 && size(nb) > 0) {
-                    fwd_list.push_back({nb, GemvTerm{edges_[e].A, size(nb), n, (int)s.xoff, 0}});
+                    fwd_list.push_back({nb, GemvTerm{edges_[e].A, size(nb), n, eoff, 0}});
                 }
             }
             for (int e : in) {
@@ -1225,7 +1195,7 @@ void Tree::plan_elimination(LevelPlan<T>& L) {
             if (!mine.empty()) {
                 int k0 = (int)bwd_terms.size();
                 for (auto it = mine.rbegin(); it != mine.rend(); ++it) bwd_terms.push_back(*it);
-                bwd_groups.push_back({(int)s.xoff, n, k0, (int)bwd_terms.size()});
+                bwd_groups.push_back({eoff, n, k0, (int)bwd_terms.size()});
             }
             set_eliminated(c);
             continue;
@@ -1282,7 +1252,7 @@ void Tree::plan_elimination(LevelPlan<T>& L) {
             inv_init.push_back({nullptr, Li, n, n, n, 0});
             push_trsm(trsmE, piv.A, Li, n, n, 0, sizeof(T));
             lst.flops_trsm += (double)n * n * n;
-            sv_elim.push_back({Li, Li, nullptr, n, (int)s.xoff});
+            sv_elim.push_back({Li, Li, nullptr, n, (int)s.xoff, eoff});
         }
         factor_bytes_ += (size_t)n * (n + 1) / 2 * sizeof(T);
         std::vector<GemvTerm> mine;
@@ -1291,7 +1261,7 @@ void Tree::plan_elimination(LevelPlan<T>& L) {
             ops_.push_back({OP_GEMM_SYMM_OUT, c, nb, n, size(nb), size(nb), n, ilvl_, edges_[e].A, nullptr});
             factor_bytes_ += (size_t)n * size(nb) * sizeof(T);
             if (n > 0 && size(nb) > 0) {
-                fwd_list.push_back({nb, GemvTerm{edges_[e].A, size(nb), n, (int)s.xoff, 0}});
+                fwd_list.push_back({nb, GemvTerm{edges_[e].A, size(nb), n, eoff, 0}});
                 mine.push_back({edges_[e].A, size(nb), n, (int)cls_[nb].xoff, 1});
             }
         }
@@ -1300,14 +1270,14 @@ void Tree::plan_elimination(LevelPlan<T>& L) {
             ops_.push_back({OP_GEMM_SYMM_IN, c, nb, n, size(nb), n, size(nb), ilvl_, edges_[e].A, nullptr});
             factor_bytes_ += (size_t)n * size(nb) * sizeof(T);
             if (n > 0 && size(nb) > 0) {
-                fwd_list.push_back({nb, GemvTerm{edges_[e].A, n, size(nb), (int)s.xoff, 1}});
+                fwd_list.push_back({nb, GemvTerm{edges_[e].A, n, size(nb), eoff, 1}});
                 mine.push_back({edges_[e].A, n, size(nb), (int)cls_[nb].xoff, 0});
             }
         }
         if (!mine.empty()) {
             int k0 = (int)bwd_terms.size();
             for (auto it = mine.rbegin(); it != mine.rend(); ++it) bwd_terms.push_back(*it);
-            bwd_groups.push_back({(int)s.xoff, n, k0, (int)bwd_terms.size()});
+            bwd_groups.push_back({eoff, n, k0, (int)bwd_terms.size()});
         }
         set_eliminated(c);
     }
@@ -1459,7 +1429,7 @@ void Tree::plan_scaling(LevelPlan<T>& L) {
                 push_trsm(trsmA, piv.A, Li, n, n, 0, sizeof(T));
                 push_trsm(trsmA, Ut, Wi, n, n, 0, sizeof(T));
                 lst.flops_trsm += 2.0 * n * n * n;
-                sv_scale.push_back({Li, Wi, pp, n, (int)s.xoff});
+                sv_scale.push_back({Li, Wi, pp, c, n, n, (int)s.xoff, -1, -1, false});
             }
         }
         for (int c : live) {
@@ -1499,7 +1469,7 @@ void Tree::plan_scaling(LevelPlan<T>& L) {
                 inv_init.push_back({nullptr, Li, s.size, s.size, s.size, 0});
                 push_trsm(trsmA, piv.A, Li, s.size, s.size, 0, sizeof(T));
                 lst.flops_trsm += (double)s.size * s.size * s.size;
-                sv_scale.push_back({Li, Li, nullptr, s.size, (int)s.xoff});
+                sv_scale.push_back({Li, Li, nullptr, c, s.size, s.size, (int)s.xoff, -1, -1, false});
             }
         }
         for (int c : live) {
@@ -1988,13 +1958,8 @@ void Tree::apply_ranks(LevelPlan<T>& L) {
     auto& qops = L.qops;
     auto& wy = L.wy;
     auto& wy_tiles = L.wy_tiles;
-    auto& wy_trsm = L.wy_trsm;
     auto& t_lvl1 = L.t_lvl1;
     auto& t_lvl2 = L.t_lvl2;
-    auto push_trsm = [&L](std::vector<TrsmTask>& v, const void* A, void* B, int n, int m, int side, size_t es,
-                          const void* src = nullptr, const int* perm = nullptr) {
-        spand::push_trsm(v, A, B, n, m, side, es, src, perm, L.cwp);
-    };
     for (size_t p = 0; p < plist.size(); p++) {
         const int c = plist[p];
         const int r = hsize[c];
@@ -2019,14 +1984,11 @@ void Tree::apply_ranks(LevelPlan<T>& L) {
                 // compact WY over all r kept reflectors, for the solve: Q = I - Ve T Ve^T
                 void* Ve = arena_.alloc((size_t)s0 * r * sizeof(T));
                 void* Sm = arena_.alloc((size_t)r * r * sizeof(T));
-                void* X = arena_.alloc((size_t)r * r * sizeof(T));
                 const int tw = (int)wy.size();
-                wy.push_back({t->Q, t->tau, Ve, Sm, X, s0, r});
+                wy.push_back({t->Q, t->tau, Ve, Sm, s0, r});
                 for (int c0 = 0; c0 < r; c0 += 32)
                     for (int a0 = 0; a0 <= c0; a0 += 32) wy_tiles.push_back(make_int4(tw, a0, c0, 0));
-                push_trsm(wy_trsm, Sm, X, r, r, 0, sizeof(T));
-                qops.push_back({Ve, X, s0, r, (int)cls_[c].xoff, (int)ws_len_});
-                ws_len_ += 2 * r;  // the y and z segments of the apply
+                qops.push_back({Ve, Sm, s0, r, c});
             }
             HCluster sib;
             sib.start = cls_[c].start + r;
@@ -2035,7 +1997,9 @@ void Tree::apply_ranks(LevelPlan<T>& L) {
             sib.spars = cls_[c].spars;
             sib.elim = true;
             sib.order = (int)cls_.size();
-            sib.xoff = cls_[c].xoff + r;
+            sib.xoff = ws_len_;  // the W phase leaves the eliminated part there
+            ws_len_ += s0 - r;
+            cls_[c].sibx = sib.xoff;
             const int sid = (int)cls_.size();
             cls_.push_back(sib);
             others_.push_back(sid);
@@ -2052,6 +2016,78 @@ void Tree::apply_ranks(LevelPlan<T>& L) {
     lst.t_spars = t_lvl2 - t_lvl1;
 }
 
+// Folds each Orthogonal op into its cluster's scaling for the apply: W = Q^T L^{-1} (and
+// Q^T U^{-T} for PLU) over the explicit inverse, W = Linv - Ve Z with (-S) Z = -Ve^T Linv: the
+// explicit V and -S, then Y = -Ve^T Linv by the Schur kernel into a cleared block, one batched
+// triangular solve, and the update of Linv by the Schur kernel again. Zeros above the diagonal
+// of Ve and Linv clip the inner ranges of both products.
+template <typename T>
+void Tree::fold_orthogonal(LevelPlan<T>& L) {
+    FactorRun& R = *L.run;
+    const hipStream_t st = R.st;
+    auto& wy = L.wy;
+    auto& wy_tiles = L.wy_tiles;
+    if (wy.empty()) return;
+    const size_t esz = sizeof(T);
+    std::vector<int> at(cls_.size(), -1);  // cluster -> its scaling task
+    for (size_t k = 0; k < L.sv_scale.size(); k++) at[L.sv_scale[k].cluster] = (int)k;
+    std::vector<SchurTile> ty, tw;
+    std::vector<SchurContrib> cy, cw;
+    std::vector<TrsmTask> tz;
+    for (auto& q : L.qops) {
+        ScaleTask& t = L.sv_scale[at[q.cluster]];
+        const int m = q.m, k = q.k;
+        const char* Ve = reinterpret_cast<const char*>(q.Ve);
+        t.q = true;
+        for (int side = 0; side < (t.Wb == t.W ? 1 : 2); side++) {
+            char* Li = reinterpret_cast<char*>(const_cast<void*>(side == 0 ? t.W : t.Wb));
+            char* Z = reinterpret_cast<char*>(arena_.alloc((size_t)k * m * esz));
+            for (int c0 = 0; c0 < m; c0 += 32) {
+                const int tn = std::min(32, m - c0);
+                for (int r0 = 0; r0 < k; r0 += 32) {  // Y(r0.., c0..): rows from max(r0, c0) on
+                    const int i0 = std::max(r0, c0), n0 = (int)cy.size();
+                    cy.push_back({Ve + (size_t)i0 * esz, Li + (size_t)i0 * esz, m - i0, m, m, 1, 0, 0});
+                    ty.push_back({Z, k, r0, c0, std::min(32, k - r0), tn, SCHUR_CLEAR, n0, n0 + 1});
+                }
+                for (int r0 = 0; r0 < m; r0 += 32) {  // W(r0.., c0..): columns of Ve up to the rows
+                    const int n0 = (int)cw.size();
+                    cw.push_back({Ve, Z, std::min(k, r0 + 32), m, k, 0, 0, 0});
+                    tw.push_back({Li, m, r0, c0, std::min(32, m - r0), tn, 0, n0, n0 + 1});
+                }
+            }
+            push_trsm(tz, q.S, Z, k, m, 0, esz, nullptr, nullptr, L.cwp);
+        }
+    }
+    Packer pl;
+    const int sp = split_trsm(tz);
+    const size_t o_w = pl.add(wy), o_t = pl.add(wy_tiles), o_z = pl.add(tz), o_ty = pl.add(ty), o_cy = pl.add(cy),
+                 o_tw = pl.add(tw), o_cw = pl.add(cw);
+    void* dl = upload_tasks(pl);
+    double lb = 0, lf = 0;
+    for (auto& w : wy) {
+        lb += (3.0 * w.m * w.k + 2.0 * w.k * w.k) * sizeof(T);
+        lf += (double)w.m * w.k * w.k;
+    }
+    hip_check(timed(prof_, KF_LARFT, st, lb, lf,
+                    [&] {
+                        return launch_wy<T>(Packer::at<WyTask>(dl, o_w), (int)wy.size(), Packer::at<int4>(dl, o_t),
+                                            (int)wy_tiles.size(), st);
+                    }),
+              "compact WY");
+    auto schur = [&](const std::vector<SchurTile>& t, const std::vector<SchurContrib>& c, size_t o1, size_t o2) {
+        const Work w = work_schur(t, c, esz);
+        hip_check(timed(prof_, KF_LARFT, st, w.bytes, w.flops,
+                        [&] {
+                            return launch_schur<T>(Packer::at<SchurTile>(dl, o1), (int)t.size(),
+                                                   Packer::at<SchurContrib>(dl, o2), st);
+                        }),
+                  "Orthogonal into scaling");
+    };
+    schur(ty, cy, o_ty, o_cy);
+    run_trsm<T>(st, dl, tz, o_z, sp, "compact WY solve");
+    schur(tw, cw, o_tw, o_cw);
+}
+
 // Merge (src/tree.cpp:1435-1445, 1106-1184): parents, their merged edges, and the
 // compact-WY launches of the Orthogonal ops.
 template <typename T>
@@ -2059,9 +2095,6 @@ void Tree::merge_level(LevelPlan<T>& L) {
     FactorRun& R = *L.run;
     const hipStream_t st = R.st;
     LevelStats& lst = *L.lst;
-    auto& wy = L.wy;
-    auto& wy_tiles = L.wy_tiles;
-    auto& wy_trsm = L.wy_trsm;
     auto& mt = L.mt;
     auto& mchildren = L.mchildren;
     auto& left = L.left;
@@ -2076,15 +2109,21 @@ void Tree::merge_level(LevelPlan<T>& L) {
             MergeTask m{(int)ws_len_, (int)mchildren.size(), 0, 0};
             for (int ch : P.children) {
                 pos[ch] = off;
-                mchildren.push_back(make_int2((int)cls_[ch].xoff, cls_[ch].size));
+                cls_[ch].pdst = ws_len_ + off;
+                // scaled children are written to their place by the W phase
+                if (!L.do_sparsify_level && cls_[ch].size > 0) {
+                    mchildren.push_back(make_int2((int)cls_[ch].xoff, cls_[ch].size));
+                    m.pxoff = (int)ws_len_ + off;
+                    m.c0 = (int)mchildren.size() - 1;
+                    m.c1 = (int)mchildren.size();
+                    mt.push_back(m);
+                }
                 off += cls_[ch].size;
             }
-            m.c1 = (int)mchildren.size();
             P.size = P.osize = off;
             P.xoff = ws_len_;
             ws_len_ += off;
             ops_.push_back({OP_MERGE, p, -1, off, 0, 0, 0, ilvl_, nullptr, nullptr});
-            if (off > 0) mt.push_back(m);
         }
         long long melems = 0;
         std::vector<long long> moff;   // by new edge id - first_new
@@ -2155,29 +2194,7 @@ void Tree::merge_level(LevelPlan<T>& L) {
                         [&] { return launch_copy<T>(Packer::at<CopyTask>(dm, o_c), (int)copies.size(), st); }),
                   "merge copy");
     }
-    if (!wy.empty()) {
-        Packer pl;
-        const int sp_wy = split_trsm(wy_trsm);
-        size_t o_w = pl.add(wy), o_t = pl.add(wy_tiles), o_s = pl.add(wy_trsm);
-        void* dl = upload_tasks(pl);
-        double lb = 0, lf = 0;
-        for (auto& w : wy) {
-            lb += (3.0 * w.m * w.k + 3.0 * w.k * w.k) * sizeof(T);
-            lf += (double)w.m * w.k * w.k;
-        }
-        hip_check(timed(prof_, KF_LARFT, st, lb, lf,
-                        [&] {
-                            return launch_wy<T>(Packer::at<WyTask>(dl, o_w), (int)wy.size(),
-                                                Packer::at<int4>(dl, o_t), (int)wy_tiles.size(), st);
-                        }),
-                  "compact WY");
-        Work w = work_trsm(wy_trsm, sizeof(T));
-        hip_check(timed(prof_, KF_TRSM, st, w.bytes, w.flops,
-                        [&] {
-                            return launch_trsm<T>(Packer::at<TrsmTask>(dl, o_s), (int)wy_trsm.size(), sp_wy, st);
-                        }),
-                  "compact WY inverse");
-    }
+    fold_orthogonal(L);
     lst.t_merge = wall() - t_lvl2;
     left = 0;
     for (int c : bottoms_[current_bottom_])
@@ -2203,7 +2220,6 @@ void Tree::plan_level_solve(LevelPlan<T>& L) {
     auto& n_potrf_elim = L.n_potrf_elim;
     auto& plist = L.plist;
     auto& nwaves = L.nwaves;
-    auto& qops = L.qops;
     auto& mt = L.mt;
     auto& mchildren = L.mchildren;
     auto& left = L.left;
@@ -2226,8 +2242,19 @@ void Tree::plan_level_solve(LevelPlan<T>& L) {
                 fwd_groups.push_back({(int)cls_[gkeys[gi]].xoff, n, k0, (int)fwd_t.size()});
             }
         }
-        HostPhases in{std::move(sv_elim),    std::move(sv_scale),  std::move(fwd_groups), std::move(bwd_groups),
-                      std::move(fwd_t),      std::move(bwd_terms), std::move(qops)};
+        // where the scaled clusters' outputs go: kept part, eliminated part
+        for (ScaleTask& t : sv_scale) {
+            HCluster& c = cls_[t.cluster];
+            if (c.pdst < 0 && c.size > 0) {  // no level above: a segment of its own
+                c.pdst = ws_len_;
+                ws_len_ += c.size;
+            }
+            t.r = c.size;
+            t.dst = (int)c.pdst;
+            t.sib = (int)c.sibx;
+        }
+        HostPhases in{std::move(sv_elim),    std::move(sv_scale), std::move(fwd_groups),
+                      std::move(bwd_groups), std::move(fwd_t),    std::move(bwd_terms)};
         pending_solve[ilvl_] =
             std::async(std::launch::async, [esz = sizeof(T), in = std::move(in), mt = std::move(mt),
                                             mchildren = std::move(mchildren)]() mutable {
@@ -2270,7 +2297,6 @@ void Tree::factorize_impl() {
         s.dofs_left_nd = nl;
     }
     factor_bytes_ = 0;
-    max_pieces_ = 0;
     // level-0 blocks
     T* base0 = reinterpret_cast<T*>(arena_.alloc((size_t)std::max<long long>(level0_elems_, 1) * sizeof(T)));
     hip_check(timed(prof_, KF_FILL, st, (double)level0_elems_ * sizeof(T), 0,
@@ -2527,8 +2553,7 @@ void Tree::apply_any(double* d_x, int nrhs, size_t sx, size_t sr, hipStream_t st
 }
 
 size_t Tree::apply_workspace_bytes(int nrhs) const {
-    const size_t seg = (size_t)ws_len_ * nrhs, part = (size_t)max_pieces_ * SOLVE_CHUNK * nrhs;
-    return (seg + part) * sizeof(double);
+    return (size_t)ws_len_ * nrhs * sizeof(double);
 }
 
 void Tree::solve_device_noalloc(double* d_x, int nrhs, int ldx, hipStream_t st) {
@@ -2588,9 +2613,7 @@ void Tree::drop_apply_graphs() {
 template <typename T>
 void Tree::apply_impl(double* dx, int nrhs, size_t sx, size_t sr, hipStream_t st_caller, bool transpose,
                       double* ws_ext) {
-    // ws: the segments (FP64 whatever the factor's element type T), then the partial sums
-    // of the largest mv phase
-    const size_t seg = (size_t)ws_len_ * nrhs;
+    // ws: the segments (FP64 whatever the factor's element type T)
     const size_t need = apply_workspace_bytes(nrhs);
     if (!ws_ext && need > ws_cap_) {
         drop_apply_graphs();  // they address the old workspace
@@ -2600,7 +2623,6 @@ void Tree::apply_impl(double* dx, int nrhs, size_t sx, size_t sr, hipStream_t st
         ws_cap_ = need;
     }
     double* ws = ws_ext ? ws_ext : reinterpret_cast<double*>(d_ws_);
-    double* partial = ws + seg;
     const double vsz = sizeof(double);
     // The whole apply (a fixed list of about 100-300 launches once the factorization is done)
     // is captured once per configuration in a hipGraph and replayed: not while launches are
@@ -2624,11 +2646,23 @@ void Tree::apply_impl(double* dx, int nrhs, size_t sx, size_t sr, hipStream_t st
         }
         hip_check(timed(prof_, fam, st, w.mat_bytes + w.vec_elems * nrhs * vsz, w.flops * nrhs, launch), what);
     };
+    // Consecutive phases of few steps run together in one workgroup (not while launches are
+    // timed, so that every phase keeps its family).
+    MvTail tail;
+    tail.n = 0;
+    auto flush = [&] {
+        if (tail.n == 1) hip_check(launch_mv<T>(tail.ph[0], ws, nrhs, st), "mv");
+        else if (tail.n > 1) hip_check(launch_mv_tail<T>(tail, ws, nrhs, st), "mv tail");
+        tail.n = 0;
+    };
     auto run_phase = [&](const MvPhase& ph) {
-        run(ph.family, ph.w, "mv", [&] {
-            return launch_mv<T>(ph.groups, ph.chunks, ph.pieces, ph.npieces, ph.terms, ph.rchunks, ph.nreduce, ws,
-                                partial, nrhs, st);
-        });
+        if (!prof_.on() && ph.steps <= MV_TAIL_STEPS) {
+            if (tail.n == MV_TAIL_MAX) flush();
+            tail.ph[tail.n++] = ph.d;
+            return;
+        }
+        flush();
+        run(ph.family, ph.w, "mv", [&] { return launch_mv<T>(ph.d, ws, nrhs, st); });
     };
     SweepWork wp;
     wp.vec_elems = (double)N_ * 2.0 + (double)N_ * 4.0 / vsz / nrhs;
@@ -2636,17 +2670,22 @@ void Tree::apply_impl(double* dx, int nrhs, size_t sx, size_t sr, hipStream_t st
     for (int l = 0; l < nlevels_; l++) {
         const LevelSolve& p = solve_plan_[l];
         for (const MvPhase& ph : transpose ? p.tfwd : p.fwd) run_phase(ph);
-        if (p.n_merge)
+        if (p.n_merge) {
+            flush();
             run(KF_MERGE, p.w_merge, "merge",
                 [&] { return launch_merge<T>(p.merge, p.n_merge, p.children, ws, nrhs, 1, st); });
+        }
     }
     for (int l = nlevels_ - 1; l >= 0; l--) {
         const LevelSolve& p = solve_plan_[l];
-        if (p.n_merge)
+        if (p.n_merge) {
+            flush();
             run(KF_MERGE, p.w_merge, "merge",
                 [&] { return launch_merge<T>(p.merge, p.n_merge, p.children, ws, nrhs, 0, st); });
+        }
         for (const MvPhase& ph : transpose ? p.tbwd : p.bwd) run_phase(ph);
     }
+    flush();
     run(KF_PERM, wp, "perm out", [&] { return launch_perm_out<T>(ws, d_perm_, N_, nrhs, dx, sx, sr, st); });
     if (graph) {
         hipGraph_t g = nullptr;

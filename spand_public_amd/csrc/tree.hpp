@@ -73,6 +73,8 @@ struct HCluster {
     std::vector<int> out;  // edge ids; out[0] is the pivot (self edge)
     std::vector<int> in;   // edge ids of edges (n -> self), n != self
     long long xoff = -1;   // segment of the cluster's x in the solve workspace
+    long long pdst = -1;   // its place in the parent's segment
+    long long sibx = -1;   // the segment of the part its sparsification eliminated
 };
 
 struct HEdge {
@@ -109,14 +111,10 @@ struct SweepWork {
     double mat_bytes = 0, vec_elems = 0, flops = 0;
 };
 
-// One mv phase of the preconditioner apply (device task arrays, see MvPiece).
+// One mv phase of the preconditioner apply (device task arrays, see MvChunk).
 struct MvPhase {
-    const MvGroup* groups = nullptr;
-    const MvTerm* terms = nullptr;
-    const MvChunk* chunks = nullptr;
-    const MvPiece* pieces = nullptr;
-    const int* rchunks = nullptr;
-    int npieces = 0, nreduce = 0;
+    MvDevPhase d{};
+    long long steps = 0;  // inner steps over all chunks
     int family = 0;  // kernel family for the timer
     SweepWork w;
 };
@@ -170,12 +168,12 @@ class Tree {
     // symmetric, so this is solve(); a GEN (PLU) tree runs its transposed phase lists.
     void solve_transpose(double* x, int nrhs, int ldx, bool on_device, hipStream_t st);
     void solve_any(double* x, int nrhs, int ldx, bool on_device, hipStream_t st, bool transpose);
-    // M^{-1} applied in place to nrhs device columns (ld >= N) with the segments and partial
-    // sums in the library's static device workspace (scratch.hpp): no device allocation, no
+    // M^{-1} applied in place to nrhs device columns (ld >= N) with the segments in the
+    // library's static device workspace (scratch.hpp): no device allocation, no
     // event; the launches are ordered on st. Throws ERR_ARG when the apply needs more than
     // SCRATCH_BYTES.
     void solve_device_noalloc(double* d_x, int nrhs, int ldx, hipStream_t st);
-    // Bytes of workspace an apply on nrhs columns needs (segments + partial sums).
+    // Bytes of workspace an apply on nrhs columns needs (the segments).
     size_t apply_workspace_bytes(int nrhs) const;
     // M^{-1} (or M^{-T}) applied in place to an interleaved device block (element (i, r) at
     // x[i*nrhs+r]).
@@ -238,6 +236,7 @@ class Tree {
     template <typename T> void launch_level(LevelPlan<T>& L);
     template <typename T> void apply_ranks(LevelPlan<T>& L);
     template <typename T> void merge_level(LevelPlan<T>& L);
+    template <typename T> void fold_orthogonal(LevelPlan<T>& L);
     template <typename T> void plan_level_solve(LevelPlan<T>& L);
     template <typename T>
     void run_potrf(hipStream_t st, void* dt, const std::vector<PotrfTask>& v, size_t off, const char* what);
@@ -343,7 +342,6 @@ class Tree {
     void* d_ws_ = nullptr;
     size_t ws_cap_ = 0;
     long long ws_len_ = 0;   // segments in the workspace (per right-hand side)
-    long long max_pieces_ = 0;  // largest mv phase, in pieces (sizes the partial-sum buffer)
 
     hipStream_t aux_stream();
     hipStream_t aux_st_ = nullptr;
