@@ -19,6 +19,8 @@
 
 #include <cfloat>
 #include <algorithm>
+#include <atomic>
+#include <type_traits>
 #include <cstdint>
 #include <limits>
 
@@ -1277,17 +1279,19 @@ __device__ inline int seg_find(const int* col0, int nseg, int j) {
     return lo;
 }
 
-// CPW consecutive values of T from LDS aligned to their size (8 or 16-byte reads)
+// CPW consecutive values of T from LDS aligned to their size (4, 8 or 16-byte reads)
 template <typename T, int CPW>
 __device__ inline void lds_row_group(const T* p, T (&out)[CPW]) {
-    static_assert(CPW * sizeof(T) % 8 == 0, "whole 8-byte reads");
-    __builtin_memcpy(out, __builtin_assume_aligned(p, CPW * sizeof(T) >= 16 ? 16 : 8), CPW * sizeof(T));
+    constexpr int B = (int)(CPW * sizeof(T));
+    static_assert(B == 4 || B % 8 == 0, "whole reads");
+    __builtin_memcpy(out, __builtin_assume_aligned(p, B >= 16 ? 16 : B), B);
 }
 
 template <typename T, int CPW>
 __device__ inline void lds_store_group(T* p, const T (&in)[CPW]) {
-    static_assert(CPW * sizeof(T) % 8 == 0, "whole 8-byte writes");
-    __builtin_memcpy(__builtin_assume_aligned(p, CPW * sizeof(T) >= 16 ? 16 : 8), in, CPW * sizeof(T));
+    constexpr int B = (int)(CPW * sizeof(T));
+    static_assert(B == 4 || B % 8 == 0, "whole writes");
+    __builtin_memcpy(__builtin_assume_aligned(p, B >= 16 ? 16 : B), in, B);
 }
 
 // (value desc, position asc) maximum over the 64 lanes of a wavefront, carrying a tag; the
@@ -1712,72 +1716,102 @@ __device__ inline size_t slab_idx(int rows, int r, int j) {
 }
 
 // Relay words of the persistent RRQR: 64-bit words (tag << 32 | 32-bit payload) stored and
-// loaded whole by device-scope relaxed atomics (on gfx950 these bypass the per-XCD L2
-// caches, which are not coherent with each other). A reader that sees the tag it waits for
-// sees the payload of the same store, so no fence orders data and flag: each word is its
-// own flag. Tags are step + 1; k_rrqr_init clears the words to tag 0 before the launch.
+// loaded whole by relaxed atomics. A reader that sees the tag it waits for sees the payload
+// of the same store, so no fence orders data and flag: each word is its own flag. Tags are
+// step + 1; k_rrqr_init clears the words to tag 0 before the launch.
+// Loads are device scope: they pass the CU's L1 and read the XCD's L2. Stores are device
+// scope too (through the L2, which is not coherent with the other XCDs' L2s) unless every
+// slab of the cluster runs on one XCD (`local`): then the store may stay in their common L2,
+// and a word takes 225 ns from store to reader instead of 470-640 ns (measured one way,
+// two workgroups in turn).
 using RelayWord = unsigned long long;
 typedef __attribute__((address_space(1))) RelayWord GRelayWord;
 
-__device__ inline void relay_put(GRelayWord* p, unsigned tag, unsigned v) {
-    __hip_atomic_store(p, ((RelayWord)tag << 32) | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+__device__ inline void relay_put(GRelayWord* p, unsigned tag, unsigned v, bool local) {
+    const RelayWord w = ((RelayWord)tag << 32) | v;
+    if (local) __hip_atomic_store(p, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    else __hip_atomic_store(p, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+// The XCD this workgroup runs on (HW_REG_XCC_ID, 4 bits).
+__device__ inline unsigned xcc_id() { return __builtin_amdgcn_s_getreg((3 << 11) | 20); }
 // a value of T as sizeof(T) / 4 relay words
 template <typename T>
-__device__ inline void relay_put_val(GRelayWord* p, unsigned tag, T x) {
+__device__ inline void relay_put_val(GRelayWord* p, unsigned tag, T x, bool local) {
     if constexpr (sizeof(T) == 4) {
-        relay_put(p, tag, __float_as_uint(x));
+        relay_put(p, tag, __float_as_uint(x), local);
     } else {
         const unsigned long long b = (unsigned long long)__double_as_longlong(x);
-        relay_put(p, tag, (unsigned)b);
-        relay_put(p + 1, tag, (unsigned)(b >> 32));
+        relay_put(p, tag, (unsigned)b, local);
+        relay_put(p + 1, tag, (unsigned)(b >> 32), local);
     }
 }
-// Waits until the first n of the words p[0..N) all carry `tag` (n loads in flight per poll,
-// one round trip when the data is there); payloads in v. False after spin_max polls
-// (RRQR_SPIN_MAX unless the caller lowers it) or once *fail is set: the launch is
-// cooperative, so every slab is resident and a correct schedule never comes near the
-// bound; the host turns the flag into an error.
-template <int N>
-__device__ inline bool relay_get_all(const GRelayWord* const (&p)[N], int n, unsigned tag, unsigned (&v)[N],
-                                     int* fail, long long spin_max) {
+// One failed poll of a bounded wait: true if the wait gives up, after spin_max polls
+// (RRQR_SPIN_MAX unless the caller lowers it) or once *fail is set: the launch is cooperative,
+// so every slab is resident and a correct schedule never comes near the bound; the host turns
+// the flag into an error.
+__device__ inline bool relay_give_up(long long spins, int* fail, long long spin_max) {
+    if (spins >= spin_max ||
+        ((spins & 63) == 63 && __hip_atomic_load(fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
+        __hip_atomic_store(fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return true;
+    }
+    __builtin_amdgcn_s_sleep(1);
+    return false;
+}
+// Waits until a word carries `tag`; its payload in v.
+__device__ inline bool relay_get(const GRelayWord* p, unsigned tag, unsigned& v, int* fail, long long spin_max) {
     for (long long spins = 0;; spins++) {
-        RelayWord w[N];
-#pragma unroll
-        for (int k = 0; k < N; k++)
-            w[k] = k < n ? __hip_atomic_load(p[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : ((RelayWord)tag << 32);
+        const RelayWord w = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        v = (unsigned)w;
+        if ((unsigned)(w >> 32) == tag) return true;
+        if (relay_give_up(spins, fail, spin_max)) return false;
+    }
+}
+// Waits for a column's words: rows 64 k + lane (WD words each, p at row lane), blocks k from kb
+// to the one of the last row, all loads in flight together; the words of rows in [i, rows) have
+// to carry the tag.
+template <int RPL, int WD>
+__device__ inline bool relay_get_rows(const GRelayWord* p, int kb, int i, int rows, unsigned tag,
+                                      RelayWord (&w)[RPL * WD], int* fail, long long spin_max) {
+    const int lane = threadIdx.x & 63;
+    for (long long spins = 0;; spins++) {
         bool ok = true;
 #pragma unroll
-        for (int k = 0; k < N; k++) ok = ok && (unsigned)(w[k] >> 32) == tag;
-        if (ok) {
+        for (int k = 0; k < RPL; k++)
 #pragma unroll
-            for (int k = 0; k < N; k++) v[k] = (unsigned)w[k];
-            return true;
+            for (int x = 0; x < WD; x++)
+                w[k * WD + x] = k >= kb && 64 * k < rows
+                                    ? __hip_atomic_load(p + 64 * k * WD + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                                    : 0;
+#pragma unroll
+        for (int k = 0; k < RPL; k++) {
+            const int r = 64 * k + lane;
+            bool have = true;
+#pragma unroll
+            for (int x = 0; x < WD; x++) have = have && (unsigned)(w[k * WD + x] >> 32) == tag;
+            ok = ok && (have || r < i || r >= rows);
         }
-        if (spins >= spin_max ||
-            ((spins & 63) == 63 && __hip_atomic_load(fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
-            __hip_atomic_store(fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            return false;
-        }
-        __builtin_amdgcn_s_sleep(1);
+        if (__all(ok)) return true;
+        if (relay_give_up(spins, fail, spin_max)) return false;
     }
 }
-// relay layout of one cluster: candidates [2][nslab][4] (norm low, norm high, position),
-// then candidate columns [2][nslab][max_rows * sizeof(T) / 4]
+// relay layout of one cluster: candidates [2][nsub][4] (norm low, norm high, position and
+// column, and in the first buffer the slab's XCD, published once), then candidate columns
+// [2][nsub][max_rows * sizeof(T) / 4]
 template <typename T>
 __device__ inline GRelayWord* relay_cand(const RrqrBig& B, int buf, int slab) {
-    return (GRelayWord*)(B.vbuf) + ((size_t)buf * B.nslab + slab) * 4;
+    return (GRelayWord*)(B.vbuf) + ((size_t)buf * B.nsub + slab) * 4;
 }
 template <typename T>
 __device__ inline GRelayWord* relay_col(const RrqrBig& B, int buf, int slab) {
-    return (GRelayWord*)(B.vbuf) + (size_t)2 * B.nslab * 4 +
-           ((size_t)buf * B.nslab + slab) * B.t.max_rows * (sizeof(T) / 4);
+    return (GRelayWord*)(B.vbuf) + (size_t)2 * B.nsub * 4 +
+           ((size_t)buf * B.nsub + slab) * B.t.max_rows * (sizeof(T) / 4);
 }
-__device__ inline void relay_put_cand(GRelayWord* p, unsigned tag, double v, int pos) {
+__device__ inline void relay_put_cand(GRelayWord* p, unsigned tag, double v, int key, bool local) {
     const unsigned long long b = (unsigned long long)__double_as_longlong(v);
-    relay_put(p, tag, (unsigned)b);
-    relay_put(p + 1, tag, (unsigned)(b >> 32));
-    relay_put(p + 2, tag, (unsigned)pos);
+    relay_put(p, tag, (unsigned)b, local);
+    relay_put(p + 1, tag, (unsigned)(b >> 32), local);
+    relay_put(p + 2, tag, (unsigned)key, local);
 }
 
 // pivot column and reflector buffers (2 x max_rows): LDS, or the task's global buffer
@@ -1822,13 +1856,10 @@ __global__ void __launch_bounds__(STEP_NT) k_rrqr_init(const RrqrBig* bigs, cons
         B.dims[4] = 2;  // 2: the steps store every kept reflector in Q; 1: the wave kernel left them in A
         if (B.dims[3] == 0) signal_store(B.done, 1);
     }
-    if (B.relay) {  // the persistent launch's relay words of this slab: tag 0 (no step)
-        for (int b = 0; b < 2; b++) {
-            GRelayWord* c = relay_cand<T>(B, b, sl.slab);
-            if (tid < 4) c[tid] = 0;
-            GRelayWord* col = relay_col<T>(B, b, sl.slab);
-            for (int r = tid; r < B.t.max_rows * (int)(sizeof(T) / 4); r += STEP_NT) col[r] = 0;
-        }
+    if (B.relay) {  // this slab's share of the persistent launch's relay words: tag 0 (no step)
+        GRelayWord* const wd = (GRelayWord*)B.vbuf;
+        const size_t n = (size_t)2 * B.nsub * (4 + (size_t)B.t.max_rows * (sizeof(T) / 4));
+        for (size_t k = (size_t)sl.slab * STEP_NT + tid; k < n; k += (size_t)B.nslab * STEP_NT) wd[k] = 0;
     }
     const gptr<T> A = gp(reinterpret_cast<T*>(B.t.scratch));
     const int mc = B.t.max_cols;
@@ -2152,426 +2183,626 @@ __global__ void __launch_bounds__(SLAB * NW) k_rrqr_step(const RrqrBig* bigs, co
 }
 
 // Persistent form of the stepped RRQR: one cooperative launch runs every pivot step of the
-// clusters of a wave (or of the part of it that the device holds at once), and each
-// cluster's slabs pace each other only. After its update at step i, every slab publishes
-// its best column (candidate for pivot i + 1: partial norm, position, rows i + 1..) in relay
-// words tagged i + 2; at step i + 1 each slab waits for the candidates of its cluster,
-// takes the first maximum and reads the winner's rows, then recomputes the step's dlarfg
-// itself: two reads through memory per step (the candidates, then the winner's rows), one
-// publication, and no fences.
-// Wavefront wv of NW holds, for its lane's column, rows r = 16 q + CPW wv + k (k < CPW =
-// 16 / NW, q < RW) in registers for the whole factorization. Row r belongs to chain
-// (r - i) % 16 of the w_j sums at step i and to chain (r - i - 1) % 16 of the norm sums,
-// each chain summed in increasing rows, so every sum runs in the 16-chain order of
-// k_rrqr_step. The sums run over every cached row with the reflector zero above row i and
-// past the last row (s_v) and a 0/1 mask for the norms (s_m): a zero term leaves a chain's
-// sum unchanged bit for bit, and the loops test rows only per group of CPW (skipping the
-// groups wholly above row i or past the last row). The pivot's owner keeps the reflector
-// (beta, v) in its registers; the registers and the final maps go back to the slab storage
-// at the end, where k_rrqr_finish copies the reflectors into Q.
-// Wavefronts per SIMD the register budget targets: the cached values plus 96 registers
-// (a few loop-invariant values may spill); 128 cached registers take the whole file (the
-// accumulation registers hold what does not fit).
-template <typename T, int RW, int NW>
-constexpr int wave_occupancy() {
-    constexpr int c = (NCH / NW) * RW * (int)(sizeof(T) / 4);
-    return c > 64 ? 1 : 512 / (c + 96) > 8 ? 8 : 512 / (c + 96);
+// clusters of a dependency wave (or of the part of it that the device holds at once), and
+// each cluster's slabs pace each other only. A slab is one wavefront, alone in its
+// workgroup: L lanes hold a column (64 / L columns a slab), lane h of a column the rows
+// r = 16 q + (16 / L) h + k (k < 16 / L, q < RW) in registers for the whole factorization.
+// Bound by the chain of a step, not by bytes or flops (a step's arithmetic is a few hundred
+// cycles), so the chain is what the layout shortens: every sum of a column stays in its
+// lanes (the rows of one residue modulo 16 are one chain of the fixed summation order, and
+// the halving tree over the 16 chains pairs the same residues whatever the step), every
+// scalar is computed by all lanes, nothing waits at a workgroup barrier, and LDS only turns a
+// column (registers of L lanes, or relay words) into a vector that all lanes read. Measured
+// against slabs of 64 columns held by 4 or 8 wavefronts with about ten barriers a step, on the
+// same clusters: 64^3 Laplacian 34.9 -> 21.7 ms a factorization (FP32), 48.0 -> 33.3 (FP64),
+// 96^3 variable kappa (FP32, with the per-step launches of clusters over 512 rows) 204 -> 129.
+// A step takes 3.5 (90 rows) to 6 us (300 rows): candidates 1.1, the pivot column 0.5, dlarfg
+// 0.4, v 0.15, w_j 0.3, the downdate 0.3, the slab's best 0.3, update 0.15, publication 0.5.
+// Step i: wait for every slab's candidate (norm, position, column), take the first maximum,
+// read the winner's rows, compute its dlarfg scalars and reflector, w_j = v^T a_j, downdate
+// the norms with row i of the updated columns (recomputing those that lost their accuracy),
+// publish the best column's norm for step i + 1, update the columns, publish that column's
+// rows. Two reads through memory a step, one publication of each kind, no fences.
+// Groups of 16 rows wholly above row i are skipped; in the group that holds row i the
+// reflector is zero above it, and rows past the last hold zeros, so a skipped row adds an
+// exact zero to its chain and every sum keeps the 16-chain order (FP64: bit for bit the
+// one-workgroup kernel's and the oracle's). Position p of a column is kept by its lanes: the
+// pivot takes position i and the column at i the pivot's.
+// The rank test of step i is taken after the step has published: what it would have skipped
+// (the step's reflector and update) touches only rows and positions past the rank, which
+// are not kept, and the division stays off the chain.
+// beta and the reflector go to Q step by step; the registers (R above the pivots' diagonals)
+// and the final positions go back to the slab storage at the end, for k_rrqr_finish.
+
+// LDS of one wavefront, written by some of its lanes and read by others: the wavefront's LDS
+// accesses run in order, so only the compiler must not move them across.
+__device__ inline void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
-template <typename T, int RW, int NW>
-__global__ void __launch_bounds__(SLAB * NW, (wave_occupancy<T, RW, NW>()))
+template <int CTRL>
+__device__ inline int dpp_mov(int v) {
+    return __builtin_amdgcn_update_dpp(v, v, CTRL, 0xF, 0xF, false);
+}
+// x of the lane whose number differs in bit XOR (1, 2, 4 or 8), within a row of 16 lanes
+template <int XOR, typename T>
+__device__ inline T lane_xor(T x) {
+    auto mv = [](int v) -> int {
+        if constexpr (XOR == 1) return dpp_mov<0xB1>(v);                 // quad_perm [1, 0, 3, 2]
+        else if constexpr (XOR == 2) return dpp_mov<0x4E>(v);            // quad_perm [2, 3, 0, 1]
+        else if constexpr (XOR == 4) return dpp_mov<0x1B>(dpp_mov<0x141>(v));  // half-row and quad mirrors
+        else return dpp_mov<0x128>(v);                                   // row_ror 8
+    };
+    if constexpr (sizeof(T) == 4) return __int_as_float(mv(__float_as_int(x)));
+    else return __hiloint2double(mv(__double2hiint(x)), mv(__double2loint(x)));
+}
+// Maximum (signed) or minimum of an int over the 64 lanes, in every lane; groups of SAME
+// neighbouring lanes hold the same value.
+template <bool MAX, int SAME>
+__device__ inline int wave_ext(int v) {
+    auto pk = [](int a, int b) { return MAX ? max(a, b) : min(a, b); };
+    if constexpr (SAME < 2) v = pk(v, dpp_mov<0xB1>(v));
+    if constexpr (SAME < 4) v = pk(v, dpp_mov<0x4E>(v));
+    if constexpr (SAME < 8) v = pk(v, dpp_mov<0x141>(v));
+    if constexpr (SAME < 16) v = pk(v, dpp_mov<0x140>(v));
+    v = pk(v, __builtin_amdgcn_update_dpp(v, v, 0x142, 0xA, 0xF, false));
+    v = pk(v, __builtin_amdgcn_update_dpp(v, v, 0x143, 0xC, 0xF, false));
+    return __builtin_amdgcn_readlane(v, 63);
+}
+// wave_best for values that are nonnegative or -1 (no candidate): they order like the
+// integers of their bits, so 32-bit reductions replace six steps of a 64-bit compare with a
+// tie test, whose mask arithmetic is the longer chain: high words, then, unless one candidate
+// alone (one group of SAME lanes) has the largest, low words among the equal high ones and
+// positions among the equal values.
+template <int SAME>
+__device__ inline void wave_best_norm(double& v, int& p) {
+    const int hi = __double2hiint(v), lo = __double2loint(v);
+    const int mh = wave_ext<true, SAME>(hi);
+    const unsigned long long top = __ballot(hi == mh);
+    if (__popcll(top) == SAME) {
+        const int at = __ffsll((unsigned long long)top) - 1;
+        v = __hiloint2double(mh, __builtin_amdgcn_readlane(lo, at));
+        p = __builtin_amdgcn_readlane(p, at);
+        return;
+    }
+    const int ml = wave_ext<true, SAME>(hi == mh ? lo ^ INT32_MIN : INT32_MIN);
+    p = wave_ext<false, SAME>(hi == mh && (lo ^ INT32_MIN) == ml ? p : INT32_MAX);
+    v = __hiloint2double(mh, ml ^ INT32_MIN);
+}
+// x of the lane N places round its row of 16 (N = 8, 4, 2, 1)
+template <int N>
+__device__ inline double row_ror(double x) {
+    const int lo = __double2loint(x), hi = __double2hiint(x);
+    return __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, 0x120 + N, 0xF, 0xF, false),
+                            __builtin_amdgcn_update_dpp(lo, lo, 0x120 + N, 0xF, 0xF, false));
+}
+// halving tree over the 16 residues of a column whose lane h holds residues CPL h + k in c[k]
+// (every lane of the column gets the sum)
+template <int L, typename A>
+__device__ inline A residue_tree(A (&c)[16 / L]) {
+#pragma clang fp contract(off)
+    constexpr int CPL = 16 / L;
+    if constexpr (L == 2) {
+#pragma unroll
+        for (int k = 0; k < CPL; k++) c[k] = c[k] + lane_xor<1>(c[k]);  // +8
+    } else if constexpr (L == 4) {
+#pragma unroll
+        for (int k = 0; k < CPL; k++) {
+            c[k] = c[k] + lane_xor<2>(c[k]);  // +8
+            c[k] = c[k] + lane_xor<1>(c[k]);  // +4
+        }
+    } else if constexpr (L == 8) {
+#pragma unroll
+        for (int k = 0; k < CPL; k++) {
+            c[k] = c[k] + lane_xor<4>(c[k]);  // +8
+            c[k] = c[k] + lane_xor<2>(c[k]);  // +4
+            c[k] = c[k] + lane_xor<1>(c[k]);  // +2
+        }
+    } else if constexpr (L == 16) {
+        c[0] = c[0] + lane_xor<8>(c[0]);
+        c[0] = c[0] + lane_xor<4>(c[0]);
+        c[0] = c[0] + lane_xor<2>(c[0]);
+        c[0] = c[0] + lane_xor<1>(c[0]);
+    }
+#pragma unroll
+    for (int w = CPL / 2; w > 0; w >>= 1)
+#pragma unroll
+        for (int k = 0; k < w; k++) c[k] = c[k] + c[k + w];
+    return c[0];
+}
+// sum of x[r]^2 over the rows of blocks of 128 from row i's on of a vector of 16 RW rows in LDS
+// (the caller leaves zeros at and above row i and past the last row), chains by residue: lane l
+// takes residue l % 16 (the four rows of 16 lanes do the same work), every lane gets the sum.
+// The reads of a block run ahead of the chain's additions.
+template <int RW>
+__device__ inline double sumsq16_wave(int i, const double* x) {
+#pragma clang fp contract(off)
+    const double* xl = x + (threadIdx.x & 15);
+    int iw = i;
+    asm volatile("" : "+s"(iw));
+    double c = 0.0;
+#pragma unroll
+    for (int q0 = 0; q0 < RW; q0 += 8) {
+        constexpr int NB = 8;
+        if (NCH * (q0 + NB) <= iw) continue;
+        double v[NB];
+#pragma unroll
+        for (int k = 0; k < NB; k++)
+            if (q0 + k < RW) v[k] = xl[NCH * (q0 + k)];
+#pragma unroll
+        for (int k = 0; k < NB; k++)
+            if (q0 + k < RW) c = fma(v[k], v[k], c);
+    }
+    c = c + row_ror<8>(c);
+    c = c + row_ror<4>(c);
+    c = c + row_ror<2>(c);
+    return c + row_ror<1>(c);
+}
+// a[q][k] of a lane's rows, q and k uniform: log2(RW) scalar branches and CPL - 1 selects
+template <int LO, int HI, int RW, int CPL, typename T>
+__device__ __attribute__((always_inline)) inline T row_at(const T (&a)[RW][CPL], int q, int k) {
+    if constexpr (HI - LO == 1) {
+        T x = T(0);  // not a[LO][0]: a choice between two elements would become an indexed load
+#pragma unroll
+        for (int u = 0; u < CPL; u++) x = u == k ? a[LO][u] : x;
+        asm volatile("" : "+v"(x));  // a value of its own in each branch: a stays in registers
+        return x;
+    } else {
+        constexpr int MID = (LO + HI) / 2;
+        return q < MID ? row_at<LO, MID>(a, q, k) : row_at<MID, HI>(a, q, k);
+    }
+}
+
+// A lane whose column rows take at most 64 registers keeps the reflector's rows too, from w_j
+// to the update; longer ones read them from LDS again.
+template <typename T, int L, int RW>
+constexpr bool wave_keeps_v() {
+    return 16 / L * RW * (int)(sizeof(T) / 4) <= 64;
+}
+template <typename T, int L, int RW>
+constexpr int wave_occupancy() {
+    constexpr int c = 16 / L * RW * (int)(sizeof(T) / 4) * (wave_keeps_v<T, L, RW>() ? 2 : 1);
+    return 512 / (c + 112) > 4 ? 4 : 512 / (c + 112);
+}
+template <typename T, int L, int RW>
+__global__ void __launch_bounds__(64, (wave_occupancy<T, L, RW>()))
     k_rrqr_wave(const RrqrBig* bigs, const RrqrSlab* slabs, int nsteps, double tol, int* fail, long long spin_max) {
 #pragma clang fp contract(off)
-    static_assert(NCH % NW == 0, "chains split evenly over the wavefronts");
-    constexpr int NTH = SLAB * NW, CPW = NCH / NW, RMAX = NCH * RW;
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    __shared__ double s_part[NCH][SLAB];
-    __shared__ double sh[4], s_ch[NCH + 1];
-    __shared__ __align__(16) T s_col[RMAX];  // the pivot column
-    __shared__ __align__(16) T s_v[RMAX];    // its reflector; zero above row i and past the last row
-    __shared__ __align__(16) T s_m[RMAX];    // 1 for rows i + 1 .. rows - 1, else 0
-    __shared__ T s_tm[SLAB], s_rowi[SLAB];
-    __shared__ int s_upd[SLAB], s_pos[SLAB], s_rc[SLAB];
-    __shared__ int s_p, s_ca, s_cb, s_best, s_ok, s_ok_col, s_anyrc;
+    constexpr int CPL = NCH / L, SC = 64 / L, RMAX = NCH * RW, WD = (int)(sizeof(T) / 4);
+    constexpr int RPL = (RMAX + 63) / 64;     // rows per lane of a vector
+    constexpr bool KEEP = wave_keeps_v<T, L, RW>();
+    // rows are skipped (wholly above row i or past the last) by blocks of BQ groups of 16: one
+    // scalar branch for 64 bytes of a lane's values
+    constexpr int BQ = L * 4 / (int)sizeof(T) > 0 ? L * 4 / (int)sizeof(T) : 1;
+    static_assert(KEEP || RW % BQ == 0, "whole blocks");
+    __shared__ __align__(16) T s_col[RMAX + 64];  // the pivot column; zero past the last row
+    __shared__ __align__(16) T s_v[RMAX + 64];    // its reflector; zero above row i and past the last row
+    __shared__ double s_x[RMAX + 64];             // the pivot column below row i, for its norm
     const RrqrSlab sl = slabs[blockIdx.x];
+    if (sl.big < 0) return;  // a place left empty to keep clusters on one XCD
     const RrqrBig B = bigs[sl.big];
-    const int tid = threadIdx.x, lane = tid % SLAB;
-    const int wv = __builtin_amdgcn_readfirstlane(tid / SLAB);  // uniform: row tests are scalar
-    const int r0 = CPW * wv;                                      // first cached row
+    const int lane = threadIdx.x, c = lane / L, h = lane % L;
     const gptr<const int> dims = gp(reinterpret_cast<const int*>(B.dims));
     const int rows = dims[0], cols = dims[1], mn = dims[2];
     int stop = dims[3];
-    const int ns = B.nslab, mc = B.t.max_cols;
-    int* p2c = reinterpret_cast<int*>(smem_raw);  // position -> column, this workgroup's copy
+    const int ns = B.nsub, mc = B.t.max_cols;
     const gptr<T> tau_out = gp(reinterpret_cast<T*>(B.t.tau));
-    const int j = sl.slab * SLAB + lane;
+    const int j = sl.slab * SC + c;
     const bool jin = j < cols && rows > 0;
-    T a[CPW][RW];
+    T a[RW][CPL];
+    const size_t at0 = slab_idx(rows, CPL * h, j);
     {
-        const gptr<const T> aslab = gp(reinterpret_cast<const T*>(B.t.scratch)) + (size_t)sl.slab * rows * SLAB + lane;
+        const gptr<const T> src = gp(reinterpret_cast<const T*>(B.t.scratch)) + (jin ? at0 : 0);
+        // this lane's rows, opaque here and below: a row test shared between the load, the
+        // steps and the store back would be kept as a lane mask per row through the steps
+        int left = jin ? rows - CPL * h : 0;
+        asm volatile("" : "+v"(left));
 #pragma unroll
         for (int q = 0; q < RW; q++)
 #pragma unroll
-            for (int k = 0; k < CPW; k++) {
-                const int r = NCH * q + r0 + k;
-                a[k][q] = (jin && r < rows) ? aslab[(size_t)r * SLAB] : T(0);
-            }
+            for (int k = 0; k < CPL; k++)
+                a[q][k] = NCH * q + k < left ? src[(size_t)(NCH * q + k) * SLAB] : T(0);
     }
-    for (int k = tid; k < cols; k += NTH) p2c[k] = k;
-    for (int r = tid; r < RMAX; r += NTH) {
+    for (int r = lane; r < RMAX + 64; r += 64) {
         s_v[r] = T(0);
-        s_m[r] = r < rows ? T(1) : T(0);
+        s_col[r] = T(0);
+        s_x[r] = 0.0;
     }
-    if (tid < SLAB) s_pos[tid] = j;
     double vn1 = 0.0, vn2 = 0.0;
-    if (wv == 0 && jin) {
-        vn1 = B.t.norms[j];
-        vn2 = B.t.norms[mc + j];
+    if (jin) {
+        vn1 = gp(B.t.norms)[j];
+        vn2 = gp(B.t.norms)[mc + j];
     }
+    double ratio = vn1 / vn2;
+    int pos = jin ? j : INT32_MAX;  // the column's position
     const double tol3z = sqrt(DBL_EPSILON * 0.5);
     const int fixed = rank_fixed(tol, mn);
-    double sref = 0.0;
-    // candidate of step 0 (k_rrqr_init left the slab's best in cand_*[slab]), tag 1; its
-    // column goes through LDS as in the steps
-    const bool run = rows > 0 && mn > 0 && stop > 0;
-    const int bp0 = run ? B.cand_p[sl.slab] : INT32_MAX;
-    if (run && tid == 0) relay_put_cand(relay_cand<T>(B, 0, sl.slab), 1u, B.cand_v[sl.slab], bp0);
-    if (bp0 != INT32_MAX && lane == bp0 % SLAB) {
-#pragma unroll
-        for (int q = 0; q < RW; q++) {
-            T x[CPW];
-#pragma unroll
-            for (int k = 0; k < CPW; k++) x[k] = a[k][q];
-            lds_store_group<T, CPW>(s_col + NCH * q + r0, x);
+    double sref = 0.0, clear = 0.0;
+    int vblock = 0;      // the block of 64 rows that holds the last reflector's 1
+    int turn = sl.slab;  // the next step whose reflector this slab stores
+    const unsigned xcc = xcc_id();
+    bool local = false;  // from step 0 on: every slab of the cluster runs on this XCD
+    // positions and columns below 2^15 (the host's condition): a candidate's position and
+    // column travel as one word that orders like the position
+    double best = -1.0;
+    int key = INT32_MAX;
+    auto pick = [&](int i) {  // the slab's first maximum among the columns at positions >= i
+        best = -1.0;
+        key = INT32_MAX;
+        if (jin && pos >= i) {
+            best = vn1;
+            key = pos << 16 | j;
         }
-    }
-    __syncthreads();
-    if (bp0 != INT32_MAX) {
-        GRelayWord* dst = relay_col<T>(B, 0, sl.slab);
-        for (int r = tid; r < rows; r += NTH) relay_put_val<T>(dst + (size_t)r * (sizeof(T) / 4), 1u, s_col[r]);
+        wave_best_norm<L>(best, key);
+    };
+    auto publish_cand = [&](int buf, unsigned tag) {
+        if (lane == 0 && ns > 1) relay_put_cand(relay_cand<T>(B, buf, sl.slab), tag, best, key, local);
+    };
+    // the slabs' candidates of a step, this lane's: words of slabs k0 + 64 q + lane
+    constexpr int CH = 2;  // up to 2 x 64 slabs' words in flight
+    RelayWord cw[CH * 3];
+    auto load_cands = [&](int buf, int k0) {
+        const int nu = min(CH, (ns - k0 + 63) / 64);
+#pragma unroll
+        for (int q = 0; q < CH; q++) {
+            const GRelayWord* const w = relay_cand<T>(B, buf, min(k0 + 64 * q + lane, ns - 1));
+#pragma unroll
+            for (int x = 0; x < 3; x++)
+                cw[3 * q + x] = q < nu ? __hip_atomic_load(w + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+        }
+    };
+    // the candidate's rows from row i0 on into s_col, and out to the other slabs. The first
+    // look at the next step's candidates (buffer buf) is issued before the stores: a wait for
+    // a later load would also wait for the stores' acknowledgements.
+    auto publish_col = [&](int i0, int buf, unsigned tag) {
+        if (key == INT32_MAX) {
+            if (ns > 1) load_cands(buf, 0);
+            return;
+        }
+        const int bj = (key & 0xffff) - sl.slab * SC;
+        if (c == bj) {
+            int iw = i0, rw = rows;
+            asm volatile("" : "+s"(iw), "+s"(rw));
+#pragma unroll
+            for (int q0 = 0; q0 < RW; q0 += BQ) {
+                if (NCH * (q0 + BQ) <= iw || NCH * q0 >= rw) continue;
+#pragma unroll
+                for (int q = q0; q < q0 + BQ && q < RW; q++)
+                    lds_store_group<T, CPL>(s_col + NCH * q + CPL * h, a[q]);
+            }
+        }
+        wave_lds_fence();
+        if (ns > 1) {
+            load_cands(buf, 0);
+            GRelayWord* dst = relay_col<T>(B, buf, sl.slab);
+#pragma unroll
+            for (int k = 0; k < RPL; k++) {
+                const int r = 64 * k + lane;
+                if (r >= i0 && r < rows) relay_put_val<T>(dst + (size_t)r * WD, tag, s_col[r], local);
+            }
+        }
+    };
+    const bool run = rows > 0 && mn > 0 && stop > 0;
+    if (run) {
+        pick(0);
+        publish_cand(0, 1u);
+        if (lane == 0 && ns > 1) relay_put(relay_cand<T>(B, 0, sl.slab) + 3, 1u, xcc, false);
+        publish_col(0, 0, 1u);
     }
     bool abandoned = false;
     for (int i = 0; i < nsteps; i++) {
         if (rows == 0 || i >= mn || i >= stop) break;  // the same decision in every slab of the cluster
         const int cur = i & 1, nxt = cur ^ 1;
         const unsigned tag = (unsigned)i + 1u;
-        // this wavefront's row window [i, rows) relative to r0, opaque to the compiler so
-        // that no per-row test is hoisted out of the step loop (64 live scalar masks)
-        int iw = i - r0, rw = rows - r0;
-        asm volatile("" : "+s"(rw));
-        if (wv == 0) {  // pivot: first maximum over the slabs' candidates
-            double bv = -1.0;
-            int bp = INT32_MAX;
+        if (ns > 1) {  // pivot: first maximum over the slabs' candidates
+            best = -1.0;
+            key = INT32_MAX;
             bool ok = true;
-            for (int k = lane; k < ns && ok; k += SLAB) {
-                const GRelayWord* c = relay_cand<T>(B, cur, k);
-                const GRelayWord* const pc[3] = {c, c + 1, c + 2};
-                unsigned u[3];
-                ok = relay_get_all<3>(pc, 3, tag, u, fail, spin_max);
+            for (int k0 = 0; k0 < ns && ok; k0 += CH * 64) {
+                const int mine = (ns - k0 - lane + 63) / 64;  // this lane's slabs of the chunk
+                const int n = mine < 0 ? 0 : (mine > CH ? CH : mine);
+                if (k0 > 0) load_cands(cur, k0);
+                for (long long spins = 0;; spins++) {
+                    bool have = true;
+#pragma unroll
+                    for (int x = 0; x < CH * 3; x++) have = have && (x / 3 >= n || (unsigned)(cw[x] >> 32) == tag);
+                    if (__all(have)) break;
+                    if (relay_give_up(spins, fail, spin_max)) {
+                        ok = false;
+                        break;
+                    }
+                    load_cands(cur, k0);
+                }
                 if (ok) {
-                    const double v = __longlong_as_double((long long)(((unsigned long long)u[1] << 32) | u[0]));
-                    const int pp = (int)u[2];
-                    if (v > bv || (v == bv && pp < bp)) {
-                        bv = v;
-                        bp = pp;
+#pragma unroll
+                    for (int q = 0; q < CH; q++) {
+                        if (q >= n) continue;
+                        const double v =
+                            __longlong_as_double((long long)((cw[3 * q + 1] << 32) | (unsigned)cw[3 * q]));
+                        const int kk = (int)(unsigned)cw[3 * q + 2];
+                        if (v > best || (v == best && kk < key)) {
+                            best = v;
+                            key = kk;
+                        }
                     }
                 }
             }
-            wave_best(bv, bp);
-            ok = __all(ok);
-            if (lane == 0) {
-                s_ok = ok;
-                s_ok_col = 1;  // cleared below by a failed read of the winner's rows
-                s_p = bp;
-                s_ca = (bp >= i && bp < cols) ? p2c[bp] : 0;
-                s_cb = p2c[i];
+            if (!__all(ok)) {
+                abandoned = true;
+                break;
+            }
+            wave_best_norm<1>(best, key);
+            if (i == 0) {  // where the cluster's slabs run
+                bool same = true;
+                for (int k = lane; k < ns && ok; k += 64) {
+                    unsigned u = 0;
+                    ok = relay_get(relay_cand<T>(B, cur, k) + 3, tag, u, fail, spin_max);
+                    same = same && ok && u == xcc;
+                }
+                if (!__all(ok)) {
+                    abandoned = true;
+                    break;
+                }
+                local = __all(same);
             }
         }
-        __syncthreads();
-        if (!s_ok) {
-            abandoned = true;
-            break;
-        }
-        const int p = s_p, ca = s_ca, cb = s_cb;
-        if (p < i || p >= cols) {  // cannot happen for i < mn: some column is still free
+        const int p = key >> 16, ca = key & 0xffff;
+        if (key == INT32_MAX || p < i || p >= cols) {  // cannot happen for i < mn: some column is still free
             stop = i;
             break;
         }
-        {  // the winner's rows i.. (published by the owner of column ca at step i - 1)
-            static_assert(RMAX <= 2 * NTH, "at most two rows per thread");
-            constexpr int WD = (int)(sizeof(T) / 4), NWD = 2 * WD;
-            const GRelayWord* src = relay_col<T>(B, cur, ca / SLAB);
-            const int r1 = i + tid, r2 = i + tid + NTH;
-            const int nr = (r1 < rows) + (r2 < rows);
-            if (nr > 0) {
-                const GRelayWord* pw[NWD];
+        T xr[RPL];  // this lane's rows 64 k + lane of the pivot column, from row block kb on
+        T alpha_t = T(0);  // its row i
+        const int kb = i / 64;
+        if (ns > 1) {  // the winner's rows i.. (published by the owner of column ca at step i - 1)
+            const GRelayWord* src = relay_col<T>(B, cur, ca / SC) + (size_t)lane * WD;
+            RelayWord u[RPL * WD];
+            bool ok = relay_get_rows<RPL, WD>(src, kb, i, rows, tag, u, fail, spin_max);
+            if (!__all(ok)) {
+                abandoned = true;
+                break;
+            }
 #pragma unroll
-                for (int k = 0; k < NWD; k++) pw[k] = src + (size_t)(k < WD ? r1 : r2) * WD + k % WD;
-                unsigned u[NWD];
-                if (relay_get_all<NWD>(pw, nr * WD, tag, u, fail, spin_max)) {
-                    T x[2];
+            for (int k = 0; k < RPL; k++) {
+                T x;
+                if constexpr (sizeof(T) == 4) x = __uint_as_float((unsigned)u[k]);
+                else x = __longlong_as_double((long long)((u[2 * k + 1] << 32) | (unsigned)u[2 * k]));
+                xr[k] = 64 * k + lane < rows ? x : T(0);
+                if (64 * k <= i && i < 64 * k + 64) alpha_t = __shfl(xr[k], i & 63);
+            }
+        } else {
 #pragma unroll
-                    for (int h = 0; h < 2; h++) {
-                        if constexpr (sizeof(T) == 4) x[h] = __uint_as_float(u[h]);
-                        else x[h] = __longlong_as_double((long long)(((unsigned long long)u[2 * h + 1] << 32) | u[2 * h]));
-                    }
-                    s_col[r1] = x[0];
-                    if (nr > 1) s_col[r2] = x[1];
+            for (int k = 0; k < RPL; k++) {
+                xr[k] = s_col[64 * k + lane];
+                if (64 * k <= i && i < 64 * k + 64) alpha_t = __shfl(xr[k], i & 63);
+            }
+        }
+        const int kx = i / 128 * 2;  // the norm reads blocks of 128 rows
+#pragma unroll
+        for (int k = 0; k < RPL; k++)
+            if (k >= kx) s_x[64 * k + lane] = 64 * k + lane > i ? (double)xr[k] : 0.0;
+        wave_lds_fence();
+        // dlarfg of s_col[i..rows): every lane computes the scalars
+        double tau_d = 0.0, beta = (double)alpha_t, scal = 1.0;
+        int knt = 0;
+        {
+            const double safmin = DBL_MIN / (DBL_EPSILON * 0.5), rs = 1.0 / safmin;
+            double alpha = beta;
+            const double xs0 = sumsq16_wave<RW>(i, s_x);
+            const double xnorm = sqrt(xs0);
+            if (xnorm != 0.0) {
+                beta = -copysign(lapy2_d(alpha, xnorm), alpha);
+                if (fabs(beta) < safmin) {  // norm of the rescaled vector (reference dlarfg)
+                    do {
+                        knt++;
+                        beta *= rs;
+                        alpha *= rs;
+                    } while (fabs(beta) < safmin && knt < 20);
+                    wave_lds_fence();
+#pragma unroll
+                    for (int k = 0; k < RPL; k++)
+                        if (k >= kx)
+                            s_x[64 * k + lane] = 64 * k + lane > i ? (double)larfg_scale<T>(xr[k], knt, 1.0) : 0.0;
+                    wave_lds_fence();
+                    const double xs = sumsq16_wave<RW>(i, s_x);
+                    beta = -copysign(lapy2_d(alpha, sqrt(xs)), alpha);
+                    tau_d = (beta - alpha) / beta;
+                    scal = 1.0 / (alpha - beta);
+                    for (int k = 0; k < knt; k++) beta *= safmin;
                 } else {
-                    s_ok_col = 0;
+                    tau_d = (beta - alpha) / beta;
+                    scal = 1.0 / (alpha - beta);
                 }
             }
         }
-        __syncthreads();
-        if (!s_ok_col) {
-            abandoned = true;
-            break;
-        }
-        larfg_block<T>((double)s_col[i], s_col + i + 1, rows - i - 1, sh, s_ch);
-        // R_ii as stored (tau = 0 leaves alpha on the diagonal); the QR stops at the rank
-        const double rii = fabs((double)(T)sh[1]);
-        if (i == 0) {
-            sref = rii;
-        } else if (fixed < 0 && !(rii / sref >= tol)) {
-            stop = i;
-            break;
-        }
-        const double taud = sh[0];
-        const T tau = (T)taud;
-        if (taud != 0.0) {
-            const int knt = (int)sh[3];
-            for (int r = i + 1 + tid; r < rows; r += NTH) s_v[r] = larfg_scale<T>(s_col[r], knt, sh[2]);
-        }
-        const bool own_pivot = ca / SLAB == sl.slab;
-        if (tid == 0) {
-            if (i > 0) s_v[i - 1] = T(0);
-            s_v[i] = T(1);
-            s_m[i] = T(0);
-            p2c[i] = ca;
-            p2c[p] = cb;
-            if (own_pivot) {
-                s_pos[ca % SLAB] = i;
-                tau_out[i] = tau;
+        const T tau = (T)tau_d;
+        const bool refl = tau_d != 0.0;
+        if (refl) {  // v: 1 on row i, zero above it and past the last row (where the column is zero)
+            if (knt > 0) {
+#pragma unroll
+                for (int k = 0; k < RPL; k++) xr[k] = larfg_scale<T>(xr[k], knt, 1.0);
             }
-            if (cb / SLAB == sl.slab && cb != ca) s_pos[cb % SLAB] = p;
+            const T sc = (T)scal;
+            const int kz = vblock;  // the last reflector's rows above this block are zero already
+            vblock = i / 64;
+#pragma unroll
+            for (int k = 0; k < RPL; k++) {
+                const int r = 64 * k + lane;
+                xr[k] = xr[k] * sc;
+                if (k >= kz) s_v[r] = r > i ? xr[k] : (r == i ? T(1) : T(0));
+            }
         }
-        __syncthreads();
-        const int pos = s_pos[lane];
+        if (j == ca) pos = i;
+        else if (pos == i) pos = p;
+        wave_lds_fence();
         const bool active = jin && pos > i;
-        // a_j += tm_j v (v is 1 on row i and 0 above it) on this thread's rows of its column
-        auto update_column = [&](T tmj) {
-#pragma unroll
-            for (int q = 0; q < RW; q++) {
-                if (NCH * q + CPW <= iw || NCH * q >= rw) continue;
-                T v[CPW];
-                lds_row_group<T, CPW>(s_v + NCH * q + r0, v);
-#pragma unroll
-                for (int k = 0; k < CPW; k++) a[k][q] = fma(v[k], tmj, a[k][q]);
-            }
-        };
-        // this column's update of the step, applied once: to the columns whose norm must be
-        // recomputed and to the slab's candidate before the candidate is published, to the
-        // others after it (off the path the other slabs wait on)
+        // this step's row window, opaque to the compiler so that the tests of the row groups
+        // stay scalar branches in the loops
+        int iw = i, rw = rows;
+        asm volatile("" : "+s"(iw), "+s"(rw));
         T tm = T(0);
         bool pending = false;
-        if (taud != 0.0) {  // w_j = v^T a_j, chain (r - i) % 16
-            T c[CPW];
+        T vk[KEEP ? RW : 1][CPL];
+        if constexpr (KEEP) {  // one run of LDS reads, no branch between them
 #pragma unroll
-            for (int k = 0; k < CPW; k++) c[k] = T(0);
-            if (active) {
+            for (int q = 0; q < RW; q++) lds_row_group<T, CPL>(s_v + NCH * q + CPL * h, vk[q]);
+        }
+        // f(group, reflector rows of the group) over the blocks of the row window; from LDS, the
+        // next block's rows are read before a block's products
+        auto blocks = [&](auto&& f) __attribute__((always_inline)) {
+            if constexpr (KEEP) {
 #pragma unroll
-                for (int q = 0; q < RW; q++) {
-                    if (NCH * q + CPW <= iw || NCH * q >= rw) continue;  // rows all above i or past the last
-                    T v[CPW];
-                    lds_row_group<T, CPW>(s_v + NCH * q + r0, v);
+                for (int q0 = 0; q0 < RW; q0 += BQ) {
+                    if (NCH * (q0 + BQ) <= iw || NCH * q0 >= rw) continue;
 #pragma unroll
-                    for (int k = 0; k < CPW; k++) c[k] = fma(a[k][q], v[k], c[k]);
+                    for (int q = q0; q < q0 + BQ && q < RW; q++) f(q, vk[q]);
+                }
+            } else {
+                T v[2][BQ][CPL];
+#pragma unroll
+                for (int u = 0; u < BQ; u++) lds_row_group<T, CPL>(s_v + NCH * u + CPL * h, v[0][u]);
+#pragma unroll
+                for (int q0 = 0; q0 < RW; q0 += BQ) {
+                    const int b = (q0 / BQ) & 1;
+                    if (q0 + BQ < RW)
+#pragma unroll
+                        for (int u = 0; u < BQ; u++)
+                            lds_row_group<T, CPL>(s_v + NCH * (q0 + BQ + u) + CPL * h, v[b ^ 1][u]);
+                    if (NCH * (q0 + BQ) <= iw || NCH * q0 >= rw) continue;
+#pragma unroll
+                    for (int q = q0; q < q0 + BQ && q < RW; q++) f(q, v[b][q - q0]);
                 }
             }
+        };
+        if (refl) {  // w_j = v^T a_j
+            T w[CPL];
 #pragma unroll
-            for (int k = 0; k < CPW; k++) s_part[(r0 + k - i % NCH + NCH) % NCH][lane] = (double)c[k];
-            __syncthreads();
-            if (wv == 0) {
-                const T w = tree16_lds_t<T>(&s_part[0][lane], SLAB);
-                s_tm[lane] = -tau * w;
-                s_upd[lane] = w != T(0);  // dger skips columns with w_j = 0
-            }
-            __syncthreads();
-            pending = active && s_upd[lane];
-            tm = pending ? s_tm[lane] : T(0);
+            for (int k = 0; k < CPL; k++) w[k] = T(0);
+            blocks([&](int q, const T (&v)[CPL]) {
+#pragma unroll
+                for (int k = 0; k < CPL; k++) w[k] = fma(a[q][k], v[k], w[k]);
+            });
+            const T wj = residue_tree<L, T>(w);
+            pending = active && wj != T(0);  // dger skips columns with w_j = 0
+            tm = pending ? -tau * wj : T(0);
         }
-        // row i of every column after the update (its new value is a_ij + tm: v_i = 1), for
-        // the norm downdate
-        if (iw >= 0 && iw / NCH < RW && iw % NCH < CPW) {
-            const int kq = iw % NCH, qq = iw / NCH;
-            T x = T(0);
-#pragma unroll
-            for (int q = 0; q < RW; q++)
-#pragma unroll
-                for (int k = 0; k < CPW; k++)
-                    if (k == kq && q == qq) x = a[k][q];
-            s_rowi[lane] = pending ? x + tm : x;
-        }
-        __syncthreads();
-        // downdate (wavefront 0): the columns whose downdated norm has lost its accuracy are
-        // flagged for the recomputation over rows > i of the updated column
-        if (wv == 0) {
-            int rc = 0;
-            if (active && vn1 != 0.0) {
-                const double qv = fabs((double)s_rowi[lane]) / vn1;
-                double temp = 1.0 - qv * qv;
-                temp = fmax(temp, 0.0);
-                const double rr = vn1 / vn2;
-                const double temp2 = temp * rr * rr;
-                if (temp2 <= tol3z) {
-                    if (i < rows - 1) {
-                        rc = 1;
-                    } else {
-                        vn1 = 0.0;
-                        vn2 = 0.0;
-                    }
+        // row i of the column after the update (v_i = 1), for the norm downdate
+        const int ik = i % NCH;
+        T xi = row_at<0, RW>(a, iw / NCH, ik % CPL);
+        if constexpr (L > 1) xi = __shfl(xi, (lane & ~(L - 1)) + ik / CPL);
+        if (pending) xi = xi + tm;
+        // the columns whose downdated norm has lost its accuracy are flagged for the
+        // recomputation over rows > i of the updated column
+        bool rc = false;
+        if (active && vn1 != 0.0) {
+            const double qv = fabs((double)xi) / vn1;
+            double temp = 1.0 - qv * qv;
+            temp = fmax(temp, 0.0);
+            const double temp2 = temp * ratio * ratio;
+            if (temp2 <= tol3z) {
+                if (i < rows - 1) {
+                    rc = true;
                 } else {
-                    vn1 = vn1 * sqrt(temp);
+                    vn1 = 0.0;
+                    vn2 = 0.0;
+                }
+            } else {
+                vn1 = vn1 * sqrt(temp);
+            }
+        }
+        // a_j += tm_j v on the pending columns (v is 1 on row i and 0 above it)
+        auto update = [&] {
+            blocks([&](int q, const T (&v)[CPL]) {
+#pragma unroll
+                for (int k = 0; k < CPL; k++) a[q][k] = fma(v[k], tm, a[q][k]);
+            });
+        };
+        bool updated = false;
+        if (__any(rc)) {
+            if (pending) update();
+            updated = true;
+            double c2[CPL];
+            int above = i - CPL * h;
+            asm volatile("" : "+v"(above));
+#pragma unroll
+            for (int k = 0; k < CPL; k++) c2[k] = 0.0;
+#pragma unroll
+            for (int q = 0; q < RW; q++) {
+                if (NCH * q + NCH <= iw || NCH * q >= rw) continue;
+#pragma unroll
+                for (int k = 0; k < CPL; k++) {
+                    double d = (double)a[q][k];
+                    if (NCH * q <= iw) d = NCH * q + k > above ? d : 0.0;  // the group holding row i
+                    c2[k] = fma(d, d, c2[k]);
                 }
             }
-            s_rc[lane] = rc;
-            const int any = __any(rc);
-            if (lane == 0) s_anyrc = any;
-        }
-        __syncthreads();
-        if (s_anyrc) {  // uniform: the flagged columns updated now, their sums of squares in chains (r - i - 1) % 16
-            const bool rc = s_rc[lane] != 0;
-            if (rc && pending) {
-                update_column(tm);
-                pending = false;
-            }
-            double c2[CPW];
-#pragma unroll
-            for (int k = 0; k < CPW; k++) c2[k] = 0.0;
+            const double nrm = sqrt(residue_tree<L, double>(c2));
             if (rc) {
-#pragma unroll
-                for (int q = 0; q < RW; q++) {
-                    if (NCH * q + CPW <= iw || NCH * q >= rw) continue;
-                    if (NCH * q <= iw) {  // the group holding row i: rows <= i masked out
-                        T m[CPW];
-                        lds_row_group<T, CPW>(s_m + NCH * q + r0, m);
-#pragma unroll
-                        for (int k = 0; k < CPW; k++) {
-                            const double d = (double)(a[k][q] * m[k]);
-                            c2[k] = fma(d, d, c2[k]);
-                        }
-                    } else {  // rows > i (rows past the last hold 0)
-#pragma unroll
-                        for (int k = 0; k < CPW; k++) {
-                            const double d = (double)a[k][q];
-                            c2[k] = fma(d, d, c2[k]);
-                        }
-                    }
-                }
-            }
-#pragma unroll
-            for (int k = 0; k < CPW; k++) s_part[(r0 + k - i % NCH - 1 + 2 * NCH) % NCH][lane] = c2[k];
-            __syncthreads();
-            if (wv == 0 && rc) {
-                vn1 = sqrt(tree16_lds(&s_part[0][lane], SLAB));
-                vn2 = vn1;
+                vn1 = nrm;
+                vn2 = nrm;
             }
         }
-        if (wv == 0) {  // the slab's best column: the candidate for step i + 1
-            double best = -1.0;
-            int bpos = INT32_MAX;
-            if (active) {
-                best = vn1;
-                bpos = pos;
+        pick(i + 1);
+        publish_cand(nxt, tag + 1u);
+        if (pending && !updated) update();
+        publish_col(i + 1, nxt, tag + 1u);
+        // the pivot column is done (never active again): beta and the reflector below it go to
+        // Q, one slab in turn for each step; its rows above (R) stay in its owner's registers
+        if (i == turn) {
+            turn += ns;
+            T* const qi = reinterpret_cast<T*>(B.t.Q) + (size_t)i * rows;
+#pragma unroll
+            for (int k = 0; k < RPL; k++) {
+                const int r = 64 * k + lane;
+                if (r >= i && r < rows) gp(qi)[r] = r == i ? (T)beta : xr[k];
             }
-            wave_best(best, bpos);
-            if (lane == 0) {
-                relay_put_cand(relay_cand<T>(B, nxt, sl.slab), tag + 1u, best, bpos);
-                s_best = bpos != INT32_MAX ? p2c[bpos] : -1;
-            }
+            if (lane == 0) tau_out[i] = tau;
         }
-        __syncthreads();
-        // the candidate column, updated, goes through LDS (s_col is free until the next
-        // step's read), then every thread stores one or two of its rows > i
-        const int best = s_best;
-        if (best >= 0 && lane == best % SLAB) {
-            if (pending) {
-                update_column(tm);
-                pending = false;
-            }
-#pragma unroll
-            for (int q = 0; q < RW; q++) {
-                if (NCH * q + CPW <= iw + 1 || NCH * q >= rw) continue;
-                T x[CPW];
-#pragma unroll
-                for (int k = 0; k < CPW; k++) x[k] = a[k][q];
-                lds_store_group<T, CPW>(s_col + NCH * q + r0, x);
-            }
-        }
-        __syncthreads();
-        if (best >= 0) {
-            GRelayWord* dst = relay_col<T>(B, nxt, sl.slab);
-            for (int r = i + 1 + tid; r < rows; r += NTH) relay_put_val<T>(dst + (size_t)r * (sizeof(T) / 4), tag + 1u, s_col[r]);
-        }
-        if (pending) update_column(tm);  // the other columns' update, after the publication
-        // the pivot column is done (never active again): its owner puts the reflector in its
-        // registers, off the path the other slabs wait on (s_v, s_m and sh hold until the
-        // next step's dlarfg)
-        if (own_pivot && lane == ca % SLAB && taud != 0.0) {  // beta on row i, v below
-#pragma unroll
-            for (int q = 0; q < RW; q++) {
-                if (NCH * q + CPW <= iw || NCH * q >= rw) continue;
-                T v[CPW], m[CPW];
-                lds_row_group<T, CPW>(s_v + NCH * q + r0, v);
-                lds_row_group<T, CPW>(s_m + NCH * q + r0, m);
-#pragma unroll
-                for (int k = 0; k < CPW; k++)
-                    if (m[k] != T(0)) a[k][q] = v[k];  // rows i + 1 .. rows - 1
-            }
-            if (iw >= 0 && iw / NCH < RW && iw % NCH < CPW) {
-                const int kq = iw % NCH, qq = iw / NCH;
-#pragma unroll
-                for (int q = 0; q < RW; q++)
-#pragma unroll
-                    for (int k = 0; k < CPW; k++)
-                        if (k == kq && q == qq) a[k][q] = (T)sh[1];
-            }
+        ratio = vn1 / vn2;  // for the next downdate
+        // R_ii as stored (tau = 0 leaves alpha on the diagonal); the QR stops at the rank. A
+        // value clear of the threshold needs no division.
+        const double rii = fabs((double)(T)beta);
+        if (i == 0) {
+            sref = rii;
+            clear = tol * sref * (1.0 + 1e-9);
+        } else if (fixed < 0 && !(rii > clear) && !(rii / sref >= tol)) {
+            stop = i;
+            break;
         }
     }
     if (abandoned) {
         // the host reports the failed wait. The cluster's maps and slab storage are not the
         // QR's (this slab's registers are dropped; its cluster's other slabs abandon too, or
         // finish without it): rows = 0 makes k_rrqr_finish leave the cluster alone
-        if (tid == 0) gp(B.dims)[0] = 0;
+        if (lane == 0) gp(B.dims)[0] = 0;
         return;
     }
-    // registers back to the slab storage; final maps after `stop` steps, as k_rrqr_finish reads them
+    // registers back to the slab storage; final positions, as k_rrqr_finish reads them
     if (jin) {
-        int rw = rows - r0;
-        asm volatile("" : "+s"(rw));
-        const gptr<T> wb = gp(reinterpret_cast<T*>(B.t.scratch)) + (size_t)sl.slab * rows * SLAB + lane;
+        int left = rows - CPL * h;
+        asm volatile("" : "+v"(left));
+        const gptr<T> wb = gp(reinterpret_cast<T*>(B.t.scratch)) + at0;
 #pragma unroll
         for (int q = 0; q < RW; q++)
 #pragma unroll
-            for (int k = 0; k < CPW; k++)
-                if (NCH * q + k < rw) wb[(size_t)(NCH * q + r0 + k) * SLAB] = a[k][q];
-    }
-    if (sl.slab == 0 && rows > 0) {
+            for (int k = 0; k < CPL; k++)
+                if (NCH * q + k < left) wb[(size_t)(NCH * q + k) * SLAB] = a[q][k];
         const int fin = stop & 1;
         const gptr<int> map = gp(B.map);
-        for (int k = tid; k < cols; k += NTH) {
-            map[fin * mc + k] = p2c[k];
-            map[2 * mc + fin * mc + p2c[k]] = k;
+        if (h == 0) {
+            map[fin * mc + pos] = j;
+            map[2 * mc + fin * mc + j] = pos;
         }
-        if (tid == 0) {
-            gp(B.dims)[3] = stop;
-            gp(B.dims)[4] = 1;  // the reflectors are in the pivot columns (k_rrqr_finish copies them)
-        }
+    }
+    if (sl.slab == 0 && rows > 0 && lane == 0) {
+        gp(B.dims)[3] = stop;
+        gp(B.dims)[4] = 1;  // the pivot columns hold R above their diagonals, Q the rest
     }
 }
 
-// One workgroup per slab: every slab copies the reflectors held in its own columns into Q
-// (persistent path: a column at pivot position pos < rank holds reflector pos) and scatters
-// R[:rank, j] of its columns into the shrunk edge blocks.
+// One workgroup per slab: every slab copies R above the diagonals of its pivot columns into Q
+// (persistent path) and scatters R[:rank, j] of its columns into the shrunk edge blocks.
 template <typename T>
 __global__ void __launch_bounds__(NT) k_rrqr_finish(const RrqrBig* bigs, const RrqrSlab* slabs, const RrqrSeg* segs,
                                                     int* dsize, double tol) {
@@ -2599,16 +2830,17 @@ __global__ void __launch_bounds__(NT) k_rrqr_finish(const RrqrBig* bigs, const R
     const int rank = fixed >= 0 ? fixed : stop;
     if (rank >= rows) return;
     const gptr<T> Q = gp(reinterpret_cast<T*>(B.t.Q));
-    // the wave kernel leaves the reflectors in the pivot columns of A; the per-step path has
-    // stored them in Q already, and the pivot columns' R entries come from there
+    // the wave kernel leaves R above the diagonal in the pivot columns of A (beta and the
+    // reflector below are in Q); the per-step path has stored whole columns in Q, and the
+    // pivot columns' R entries come from there
     const bool in_a = B.dims[4] == 1;
     const int j0 = sl.slab * SLAB;
-    if (in_a)  // column j of this slab at pivot position pos < rank holds reflector pos
-        for (int idx = tid; idx < rows * SLAB; idx += NT) {
-            const int r = idx % rows, j = j0 + idx / rows;
-            if (j >= cols) break;  // j grows with idx
+    if (in_a)  // column j of this slab at pivot position pos < rank
+        for (int idx = tid; idx < rank * SLAB; idx += NT) {
+            const int j = j0 + idx % SLAB, r = idx / SLAB;
+            if (j >= cols) continue;
             const int pos = c2p[j];
-            if (pos < rank) Q[r + (size_t)pos * rows] = A[slab_idx(rows, r, j)];
+            if (pos < rank && r < pos) Q[r + (size_t)pos * rows] = A[slab_idx(rows, r, j)];
         }
     for (int idx = tid; idx < rank * SLAB; idx += NT) {
         const int j = j0 + idx % SLAB, r = idx / SLAB;
@@ -2617,7 +2849,8 @@ __global__ void __launch_bounds__(NT) k_rrqr_finish(const RrqrBig* bigs, const R
         const int k = seg_find(s_col0, B.t.nseg, j);
         const int jj = j - s_col0[k], w = s_col0[k + 1] - s_col0[k];
         T* E = reinterpret_cast<T*>(sg[k].E);
-        const T v = (r > pos) ? T(0) : ((!in_a && pos < rank) ? Q[r + (size_t)pos * rows] : A[slab_idx(rows, r, j)]);
+        const bool in_q = pos < rank && (!in_a || r == pos);
+        const T v = (r > pos) ? T(0) : (in_q ? Q[r + (size_t)pos * rows] : A[slab_idx(rows, r, j)]);
         if (sg[k].out) E[jj + (size_t)r * w] = v;
         else E[r + (size_t)jj * rank] = v;
     }
@@ -2883,62 +3116,121 @@ hipError_t launch_rrqr_step(const RrqrBig* d_bigs, const RrqrSlab* d_slabs, int 
     return hipGetLastError();
 }
 
-// Persistent wave launch: rows per thread and wavefronts per slab by the wave's largest
-// cluster (16 / NW * RW values of T per thread, at most 128 registers' worth).
-template <typename T, int RW, int NW>
-static hipError_t wave_capacity_rw(size_t lds_bytes, int* cap) {
+// Persistent wave launch: lanes per column and rows per lane by the wave's largest cluster.
+// The fine form has at most 64 registers of column per lane (and keeps the reflector's rows
+// as well); the dense one up to 96 and fewer slabs, for waves whose slabs would otherwise not
+// fit the device in one launch.
+template <typename T, int L, int RW>
+static hipError_t wave_capacity_rw(int* cap) {
+    // asked for once per kernel form and device (a level asks for every dependency wave)
+    constexpr int DEVS = 64;
+    static std::atomic<int> known[DEVS];
     int dev = 0, ncu = 0, per_cu = 0;
     hipError_t e = hipGetDevice(&dev);
+    if (e == hipSuccess && dev < DEVS && (*cap = known[dev].load(std::memory_order_relaxed)) > 0) return e;
     if (e == hipSuccess) e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-    const void* f = reinterpret_cast<const void*>(k_rrqr_wave<T, RW, NW>);
-    if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f, SLAB * NW, lds_bytes);
+    const void* f = reinterpret_cast<const void*>(k_rrqr_wave<T, L, RW>);
+    if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f, 64, 0);
     *cap = e == hipSuccess ? per_cu * ncu : 0;
+    if (e == hipSuccess && dev < DEVS) known[dev].store(*cap, std::memory_order_relaxed);
     return e;
 }
 
-template <typename T, int RW, int NW>
+template <typename T, int L, int RW>
 static hipError_t launch_wave_rw(const RrqrBig* d_bigs, const RrqrSlab* d_slabs, int nslabs, int nsteps, double tol,
-                                 size_t lds_bytes, int* fail, long long spin_max, hipStream_t st) {
+                                 int* fail, long long spin_max, hipStream_t st) {
     int cap = 0;
-    hipError_t e = wave_capacity_rw<T, RW, NW>(lds_bytes, &cap);
+    hipError_t e = wave_capacity_rw<T, L, RW>(&cap);
     if (e != hipSuccess) return e;
     if (cap < nslabs) return hipErrorCooperativeLaunchTooLarge;
-    const void* f = reinterpret_cast<const void*>(k_rrqr_wave<T, RW, NW>);
+    // A cooperative launch goes through a queue of its own (about 12 us before and after it).
+    // Up to a quarter of what the device holds is launched plainly: launches of one process are
+    // ordered on the null stream, and even those of several processes fit together.
+    if (nslabs <= cap / 4) {
+        k_rrqr_wave<T, L, RW><<<nslabs, 64, 0, st>>>(d_bigs, d_slabs, nsteps, tol, fail, spin_max);
+        return hipGetLastError();
+    }
+    const void* f = reinterpret_cast<const void*>(k_rrqr_wave<T, L, RW>);
     void* args[] = {(void*)&d_bigs, (void*)&d_slabs, (void*)&nsteps, (void*)&tol, (void*)&fail, (void*)&spin_max};
-    return hipLaunchCooperativeKernel(f, dim3(nslabs), dim3(SLAB * NW), args, (unsigned)lds_bytes, st);
+    return hipLaunchCooperativeKernel(f, dim3(nslabs), dim3(64), args, 0, st);
 }
 
-// One dispatch table for the capacity query and the launch: the variant for max_rows.
-template <typename T, bool LAUNCH>
-static hipError_t wave_variant(int max_rows, size_t lds_bytes, int* cap, const RrqrBig* d_bigs,
-                               const RrqrSlab* d_slabs, int nslabs, int nsteps, double tol, int* fail,
-                               long long spin_max, hipStream_t st) {
-#define SPAND_WAVE(RW, NW)                                                                                             \
-    return LAUNCH ? launch_wave_rw<T, RW, NW>(d_bigs, d_slabs, nslabs, nsteps, tol, lds_bytes, fail, spin_max, st) \
-                  : wave_capacity_rw<T, RW, NW>(lds_bytes, cap)
-    if (max_rows <= NCH * 4) SPAND_WAVE(4, 4);
-    if (max_rows <= NCH * 8) SPAND_WAVE(8, 4);
-    if (max_rows <= NCH * 16) SPAND_WAVE(16, 4);
-    if (max_rows <= NCH * 32) SPAND_WAVE(32, 8);
+// One dispatch table for the slab width, the capacity query and the launch: f(lanes per
+// column, rows / 16 per lane) of the variant for max_rows; false beyond WAVE_ROWS_MAX.
+template <typename T, typename F>
+static bool wave_variant(int max_rows, bool dense, F&& f) {
+#define SPAND_WAVE(L, RW)                                                                 \
+    if (max_rows <= NCH * RW) {                                                           \
+        f(std::integral_constant<int, L>(), std::integral_constant<int, RW>());           \
+        return true;                                                                      \
+    }
+    if constexpr (sizeof(T) == 4) {
+        SPAND_WAVE(1, 2)
+        if (dense) {
+            SPAND_WAVE(1, 4)
+            SPAND_WAVE(1, 6)
+            SPAND_WAVE(2, 12)
+            SPAND_WAVE(4, 24)
+            SPAND_WAVE(8, 48)
+        }
+        SPAND_WAVE(2, 4)
+        SPAND_WAVE(2, 6)
+        SPAND_WAVE(4, 8)
+        SPAND_WAVE(4, 12)
+        SPAND_WAVE(8, 16)
+        SPAND_WAVE(8, 24)
+        SPAND_WAVE(8, 32)
+        SPAND_WAVE(16, 48)
+        SPAND_WAVE(16, 64)
+    } else {
+        SPAND_WAVE(1, 2)
+        if (dense) {
+            SPAND_WAVE(1, 3)
+            SPAND_WAVE(2, 6)
+            SPAND_WAVE(4, 12)
+            SPAND_WAVE(8, 24)
+        }
+        SPAND_WAVE(2, 4)
+        SPAND_WAVE(4, 6)
+        SPAND_WAVE(4, 8)
+        SPAND_WAVE(8, 12)
+        SPAND_WAVE(8, 16)
+        SPAND_WAVE(16, 24)
+        SPAND_WAVE(16, 32)
+    }
 #undef SPAND_WAVE
-    return LAUNCH ? hipErrorCooperativeLaunchTooLarge : hipSuccess;
+    return false;
 }
 
 template <typename T>
-hipError_t rrqr_wave_capacity(int max_rows, size_t lds_bytes, int* cap) {
+int rrqr_wave_cols(int max_rows, bool dense) {
+    int cols = 0;
+    wave_variant<T>(max_rows, dense, [&](auto l, auto) { cols = 64 / decltype(l)::value; });
+    return cols;
+}
+
+template <typename T>
+hipError_t rrqr_wave_capacity(int max_rows, bool dense, int* cap) {
     *cap = 0;
-    return wave_variant<T, false>(max_rows, lds_bytes, cap, nullptr, nullptr, 0, 0, 0.0, nullptr, 0, nullptr);
+    hipError_t e = hipSuccess;
+    wave_variant<T>(max_rows, dense,
+                    [&](auto l, auto rw) { e = wave_capacity_rw<T, decltype(l)::value, decltype(rw)::value>(cap); });
+    return e;
 }
 
 // Persistent launch over nslabs slabs (whole clusters): returns hipErrorCooperativeLaunchTooLarge
 // (and launches nothing) when they cannot all be resident at once.
 template <typename T>
 hipError_t launch_rrqr_wave(const RrqrBig* d_bigs, const RrqrSlab* d_slabs, int nslabs, int nsteps, int max_rows,
-                            double tol, size_t lds_bytes, int* fail, long long spin_max, hipStream_t st) {
+                            bool dense, double tol, int* fail, long long spin_max, hipStream_t st) {
     if (nslabs == 0 || nsteps == 0) return hipSuccess;
     if (spin_max < 1) return hipErrorInvalidValue;
-    return wave_variant<T, true>(max_rows, lds_bytes, nullptr, d_bigs, d_slabs, nslabs, nsteps, tol, fail, spin_max,
-                                 st);
+    hipError_t e = hipErrorCooperativeLaunchTooLarge;
+    wave_variant<T>(max_rows, dense, [&](auto l, auto rw) {
+        e = launch_wave_rw<T, decltype(l)::value, decltype(rw)::value>(d_bigs, d_slabs, nslabs, nsteps, tol, fail,
+                                                                       spin_max, st);
+    });
+    return e;
 }
 
 template <typename T>
@@ -2971,9 +3263,10 @@ hipError_t launch_copy(const CopyTask* d_tasks, int ntasks, hipStream_t st) {
     template hipError_t launch_copy<T>(const CopyTask*, int, hipStream_t);                        \
     template hipError_t launch_rrqr_init<T>(const RrqrBig*, const RrqrSlab*, int, const RrqrSeg*, const int*,      \
                                             double, hipStream_t);                                                  \
-    template hipError_t launch_rrqr_wave<T>(const RrqrBig*, const RrqrSlab*, int, int, int, double, size_t, int*, \
+    template hipError_t launch_rrqr_wave<T>(const RrqrBig*, const RrqrSlab*, int, int, int, bool, double, int*,   \
                                             long long, hipStream_t);                                               \
-    template hipError_t rrqr_wave_capacity<T>(int, size_t, int*);                                                  \
+    template hipError_t rrqr_wave_capacity<T>(int, bool, int*);                                                    \
+    template int rrqr_wave_cols<T>(int, bool);                                                                     \
     template hipError_t launch_rrqr_step<T>(const RrqrBig*, const RrqrSlab*, int, int, int, double, size_t, int,  \
                                             long long*, long long, hipStream_t);                                                       \
     template hipError_t launch_rrqr_finish<T>(const RrqrBig*, const RrqrSlab*, int, const RrqrSeg*, int*, double,  \

@@ -102,12 +102,13 @@ struct RrqrBig {
                      // 1 once every kept reflector is stored
     void* vbuf;      // nullptr, or [nslab][2][max_rows] pivot column / reflector buffers
                      // (per-step launches), or the relay words of the persistent launch
-                     // (relay = 1): candidates [2][nslab][4], then candidate columns
-                     // [2][nslab][max_rows * sizeof(T) / 4], 64 bits each
+                     // (relay = 1): candidates [2][nsub][4], then candidate columns
+                     // [2][nsub][max_rows * sizeof(T) / 4], 64 bits each
     long long* done; // host-visible flag, or nullptr: set to 1 by the last step that does
                      // work (rank reached or all min(rows, cols) steps taken)
     int nslab;
     int relay;       // 1: vbuf holds relay words (k_rrqr_init clears them)
+    int nsub;        // slabs of the persistent launch (narrower than 64 columns for long ones)
 };
 struct RrqrSlab {
     int big;   // index into the RrqrBig array

@@ -952,8 +952,10 @@ struct LevelPlan {
     std::vector<std::vector<int>> wregvar;       // the variant of each wreg task
     std::vector<std::pair<int, int>> where;      // (0 small | 1 big | 2 register, index) by plist position
     std::vector<RrqrSeg> segs;
-    std::vector<size_t> wlds_step, wlds_wave;
-    bool persistent = false;
+    std::vector<size_t> wlds_step;
+    std::vector<std::vector<RrqrSlab>> wplace;   // persistent launches: slabs by workgroup
+    std::vector<std::vector<std::array<int, 3>>> wchunk;  // their (first workgroup, workgroups, steps)
+    std::vector<char> wdense;                    // and form
     int step_waves = 0;
     std::vector<size_t> wflag0;
     // kept ranks and merge
@@ -1493,6 +1495,66 @@ void Tree::plan_scaling(LevelPlan<T>& L) {
     }
 }
 
+// Workgroups of the persistent launches of one wave: whole clusters in chunks that the device
+// holds at once (at most cap slabs), one launch each. Block b of a launch runs on XCD b % 8, so
+// a cluster's slabs go to places of one residue, largest clusters first onto the emptiest XCD:
+// its slabs then exchange their candidates through that XCD's L2 (the kernel checks where they
+// run). A cluster that no XCD holds alone spreads over the device, in a chunk of its kind. No
+// chunk at all if some cluster exceeds cap.
+struct SlabPlan {
+    std::vector<RrqrSlab> place;
+    std::vector<std::array<int, 3>> chunk;  // first workgroup, workgroups, steps
+    int spread = 0;                         // chunks whose clusters spread over the XCDs
+};
+static SlabPlan place_slabs(const std::vector<RrqrBig>& big, int cap) {
+    constexpr int XCDS = 8;
+    const int each = cap / XCDS;
+    SlabPlan P;
+    std::vector<int> order(big.size());
+    std::iota(order.begin(), order.end(), 0);
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return big[a].nsub > big[b].nsub; });
+    if (order.empty() || big[order[0]].nsub > cap) return P;
+    auto steps_of = [&](int x) { return std::min(big[x].t.max_rows, big[x].t.max_cols); };
+    size_t x0 = 0;
+    while (x0 < order.size() && big[order[x0]].nsub > each) {  // too long for one XCD
+        const int first = (int)P.place.size();
+        int steps = 0;
+        while (x0 < order.size() && big[order[x0]].nsub > each &&
+               (int)P.place.size() - first + big[order[x0]].nsub <= cap) {
+            for (int k = 0; k < big[order[x0]].nsub; k++) P.place.push_back({order[x0], k});
+            steps = std::max(steps, steps_of(order[x0++]));
+        }
+        P.chunk.push_back({first, (int)P.place.size() - first, steps});
+        P.spread++;
+    }
+    std::vector<int> rest(order.begin() + x0, order.end()), later;
+    while (!rest.empty()) {
+        std::vector<RrqrSlab> on[XCDS];
+        int steps = 0;
+        size_t most = 0;
+        later.clear();
+        for (int x : rest) {
+            auto* q = &on[0];
+            for (auto& o : on)
+                if (o.size() < q->size()) q = &o;
+            if ((int)q->size() + big[x].nsub > each) {
+                later.push_back(x);
+                continue;
+            }
+            for (int k = 0; k < big[x].nsub; k++) q->push_back({x, k});
+            most = std::max(most, q->size());
+            steps = std::max(steps, steps_of(x));
+        }
+        const int first = (int)P.place.size();
+        P.place.resize(first + most * XCDS, {-1, 0});
+        for (int o = 0; o < XCDS; o++)
+            for (size_t k = 0; k < on[o].size(); k++) P.place[first + k * XCDS + o] = on[o][k];
+        P.chunk.push_back({first, (int)(most * XCDS), steps});
+        rest.swap(later);
+    }
+    return P;
+}
+
 // Sparsification plan (src/tree.cpp:1521-1533, 1292-1347): dependency waves, the RRQR
 // path of each cluster (register, one-workgroup LDS or stepped slabs) and its buffers.
 template <typename T>
@@ -1520,8 +1582,6 @@ void Tree::plan_sparsification(LevelPlan<T>& L) {
     auto& where = L.where;
     auto& segs = L.segs;
     auto& wlds_step = L.wlds_step;
-    auto& wlds_wave = L.wlds_wave;
-    auto& persistent = L.persistent;
     auto& step_waves = L.step_waves;
     auto& wflag0 = L.wflag0;
     if (do_sparsify_level) {
@@ -1557,6 +1617,7 @@ void Tree::plan_sparsification(LevelPlan<T>& L) {
         where.assign(plist.size(), {0, 0});
         std::vector<std::vector<std::pair<int, int>>> regp(nwaves);  // (variant, plist position)
         std::vector<RrqrTask> ptask(plist.size());
+        std::vector<int> pcols;  // Asn columns by plist position
         {  // the sparsification knobs from the level's Asn shapes
             std::vector<int> rows, cols;
             for (int c : plist) {
@@ -1567,6 +1628,7 @@ void Tree::plan_sparsification(LevelPlan<T>& L) {
                 rows.push_back(s.size);
                 cols.push_back(nc);
             }
+            pcols = cols;
             shape.n_spars = (int)plist.size();
             if (!rows.empty()) {
                 std::sort(rows.begin(), rows.end());
@@ -1585,6 +1647,33 @@ void Tree::plan_sparsification(LevelPlan<T>& L) {
         const bool reg_path = tune.rrqr_reg != 0;
         const long long big_min_elems = tune.small_elems;
         widx.assign(plist.size(), 0);
+        // Dependency waves that one persistent launch can hold run all their clusters there (64^3
+        // Laplacian, FP32: 29.6 ms a factorization for every RRQR launch, against 37.9 ms with the
+        // shorter clusters in one workgroup each), unless they are all tiny (10 x 40 on a 512^2
+        // grid: 2.3 ms in one workgroup each, 3.1 ms there). The others, and every wave when a
+        // path is asked for through the environment, split by cluster size.
+        constexpr long long TINY_ELEMS = 2000;
+        std::vector<char> all_wave(nwaves, 0);
+        if (tune.source == 0 && env_or("SPAND_RRQR_PERSISTENT", 1) != 0) {
+            std::vector<int> mr(nwaves, 0), mc(nwaves, 0);
+            std::vector<long long> slabs(nwaves, 0), elems(nwaves, 0);
+            for (size_t p = 0; p < plist.size(); p++) {
+                const int w = wave[p], rows = cls_[plist[p]].size;
+                mr[w] = std::max(mr[w], rows);
+                mc[w] = std::max(mc[w], pcols[p]);
+                elems[w] = std::max(elems[w], (long long)rows * pcols[p]);
+            }
+            for (size_t p = 0; p < plist.size(); p++) {
+                const int w = wave[p], sc = rrqr_wave_cols<T>(mr[w], true);
+                if (sc > 0) slabs[w] += std::max(1, (pcols[p] + sc - 1) / sc);
+            }
+            for (int w = 0; w < nwaves; w++) {
+                int cap = 0;
+                if (rrqr_wave_cols<T>(mr[w], true) == 0 || mc[w] >= WAVE_COLS_MAX) continue;
+                hip_check(rrqr_wave_capacity<T>(mr[w], true, &cap), "rrqr wave capacity");
+                all_wave[w] = slabs[w] <= cap && elems[w] > TINY_ELEMS;
+            }
+        }
         for (size_t p = 0; p < plist.size(); p++) {
             const int c = plist[p];
             const HCluster& s = cls_[c];
@@ -1610,12 +1699,13 @@ void Tree::plan_sparsification(LevelPlan<T>& L) {
             t.tau = arena_.alloc((size_t)std::max(1, mn) * sizeof(T));
             lst.flops_rrqr += mn > 0 ? 2.0 * s.size * cols * mn - (2.0 / 3.0) * (double)mn * mn * mn : 0.0;
             const int w = wave[p];
-            const int reg_var = reg_path ? rrqr_reg_variant(sizeof(T), s.size, cols) : -1;
+            const bool one_wg = !all_wave[wave[p]];
+            const int reg_var = reg_path && one_wg ? rrqr_reg_variant(sizeof(T), s.size, cols) : -1;
             if (reg_var >= 0) {
                 // register-resident, one workgroup per cluster
                 ptask[p] = t;
                 regp[w].push_back({reg_var, (int)p});
-            } else if (s.size >= big_min_rows && (long long)s.size * cols > big_min_elems) {
+            } else if (!one_wg || (s.size >= big_min_rows && (long long)s.size * cols > big_min_elems)) {
                 // stepped multi-workgroup path
                 RrqrBig b{};
                 b.nslab = std::max(1, (cols + 63) / 64);
@@ -1657,28 +1747,50 @@ void Tree::plan_sparsification(LevelPlan<T>& L) {
     }
     // pivot-column / reflector buffers of the stepped path: LDS unless a wave's largest
     // cluster needs more than STEP_LDS_MAX, then global buffers for the whole wave
-    // A wave whose clusters all have at most WAVE_ROWS_MAX rows runs as one persistent
-    // launch (candidate-column buffers in vbuf); the per-step launches remain the path
-    // for larger clusters and for waves the device cannot hold at once.
+    // A wave whose clusters fit the persistent launch runs as one launch (relay words in vbuf);
+    // the per-step launches remain the path for longer clusters (over 1024 rows FP32, 512
+    // FP64) and for clusters the device cannot hold at once.
     wlds_step.assign(nwaves, 0);
-    wlds_wave.assign(nwaves, 0);
+    L.wplace.assign(nwaves, {});
+    L.wchunk.assign(nwaves, {});
+    L.wdense.assign(nwaves, 0);
     // The persistent launch is the default (SPAND_RRQR_PERSISTENT=0 returns to one launch
-    // per step): on the 64^3 Laplacian its steps take 6-12 us against about 10.5 us per
-    // step launch, and FP64 and FP32 both gain.
-    persistent = env_or("SPAND_RRQR_PERSISTENT", 1) != 0;
+    // per step, about 10.5 us a step on the 64^3 Laplacian against 2-4 us).
+    const bool persistent = env_or("SPAND_RRQR_PERSISTENT", 1) != 0;
     step_waves = tune.step_waves;  // 4, 8, 16; 0: by slab count
     tunes_[ilvl_] = tune;
     shapes_[ilvl_] = shape;
+    // the fine form unless the dense one takes fewer launches, spread ones counted twice (their
+    // exchanges pass the L2s: 3-4 us a step more with the device full)
+    auto plan_wave = [&](std::vector<RrqrBig>& big, int max_rows, std::vector<RrqrSlab>& place,
+                         std::vector<std::array<int, 3>>& chunk, char& form) {
+        size_t cost = 0;
+        for (bool dense : {false, true}) {
+            const int sc = rrqr_wave_cols<T>(max_rows, dense);
+            int cap = 0;
+            hip_check(rrqr_wave_capacity<T>(max_rows, dense, &cap), "rrqr wave capacity");
+            std::vector<RrqrBig> b = big;
+            for (auto& x : b) x.nsub = std::max(1, (x.t.max_cols + sc - 1) / sc);
+            SlabPlan P = place_slabs(b, cap);
+            const size_t c = P.chunk.size() + P.spread;
+            if (c == 0 || (cost > 0 && c >= cost)) continue;
+            cost = c;
+            big.swap(b);
+            place.swap(P.place);
+            chunk.swap(P.chunk);
+            form = dense;
+            if (cost == 1) break;
+        }
+    };
     for (int w = 0; w < nwaves; w++) {
         const size_t vb = (size_t)std::max(wmaxrows[w], 1) * sizeof(T);
         int wmaxcols = 0;
         for (auto& b : wbig[w]) wmaxcols = std::max(wmaxcols, b.t.max_cols);
-        const size_t lw = ((size_t)wmaxcols * sizeof(int) + 15) / 16 * 16;  // the persistent launch's p2c
-        if (persistent && !wbig[w].empty() && wmaxrows[w] <= WAVE_ROWS_MAX && lw <= (size_t)WAVE_LDS_MAX) {
-            wlds_wave[w] = lw;
-            wlds_step[w] = 2 * vb;  // the per-step fallback (a wave the device cannot hold at once)
+        if (persistent && !wbig[w].empty() && rrqr_wave_cols<T>(wmaxrows[w], false) > 0 && wmaxcols < WAVE_COLS_MAX)
+            plan_wave(wbig[w], wmaxrows[w], L.wplace[w], L.wchunk[w], L.wdense[w]);
+        if (!L.wchunk[w].empty()) {
             for (auto& b : wbig[w]) {
-                b.vbuf = arena_.alloc(rrqr_relay_bytes(sizeof(T), b.nslab, std::max(b.t.max_rows, 1)));
+                b.vbuf = arena_.alloc(rrqr_relay_bytes(sizeof(T), b.nsub, std::max(b.t.max_rows, 1)));
                 b.relay = 1;
             }
         } else if (2 * vb <= (size_t)STEP_LDS_MAX) {
@@ -1743,8 +1855,6 @@ void Tree::launch_level(LevelPlan<T>& L) {
     auto& wregvar = L.wregvar;
     auto& segs = L.segs;
     auto& wlds_step = L.wlds_step;
-    auto& wlds_wave = L.wlds_wave;
-    auto& persistent = L.persistent;
     auto& step_waves = L.step_waves;
     auto& wflag0 = L.wflag0;
     auto& t_lvl0 = L.t_lvl0;
@@ -1760,12 +1870,13 @@ void Tree::launch_level(LevelPlan<T>& L) {
     size_t o_ii = pk.add(inv_init);
     lds_first<T>(getrfS);
     size_t o_gs = pk.add(getrfS);
-    std::vector<size_t> o_w(nwaves), o_b(nwaves), o_s(nwaves), o_r(nwaves);
+    std::vector<size_t> o_w(nwaves), o_b(nwaves), o_s(nwaves), o_r(nwaves), o_p(nwaves);
     for (int w = 0; w < nwaves; w++) {
         o_r[w] = pk.add(wreg[w]);
         o_w[w] = pk.add(wtasks[w]);
         o_b[w] = pk.add(wbig[w]);
         o_s[w] = pk.add(wslab[w]);
+        o_p[w] = pk.add(L.wplace[w]);
     }
     L.t_plan1 = wall();
     void* dt = upload_tasks(pk);
@@ -1856,35 +1967,16 @@ void Tree::launch_level(LevelPlan<T>& L) {
                   "rrqr init");
         // the steps of a wave are timed as one batch (two events per wave)
         bool done = false;
-        if (wlds_wave[w] > 0) {
-            // whole clusters in chunks the device holds at once, one cooperative launch each
-            int cap = 0;
-            hip_check(rrqr_wave_capacity<T>(wmaxrows[w], wlds_wave[w], &cap), "rrqr wave capacity");
-            int maxslab = 0;
-            for (auto& b : wbig[w]) maxslab = std::max(maxslab, b.nslab);
-            if (cap >= maxslab && cap > 0) {
-                const int sl = prof_.start(KF_RRQR_WAVE, st);
-                int launches = 0;
-                size_t x0 = 0, s0 = 0;
-                while (x0 < wbig[w].size()) {
-                    size_t x1 = x0, s1 = s0;
-                    int steps = 0;
-                    while (x1 < wbig[w].size() && (int)(s1 - s0) + wbig[w][x1].nslab <= cap) {
-                        steps = std::max(steps, std::min(wbig[w][x1].t.max_rows, wbig[w][x1].t.max_cols));
-                        s1 += wbig[w][x1].nslab;
-                        x1++;
-                    }
-                    const hipError_t e = launch_rrqr_wave<T>(db, ds + s0, (int)(s1 - s0), steps, wmaxrows[w], tol_,
-                                                             wlds_wave[w], d_info_ + 1, R.spin_max, st);
-                    hip_check(e, "rrqr wave");
-                    launches++;
-                    x0 = x1;
-                    s0 = s1;
-                }
-                prof_.stop(sl, st, 0, 0, launches);
-                done = true;
-                slot_step[w] = sl;
-            }
+        if (!L.wchunk[w].empty()) {
+            const int sl = prof_.start(KF_RRQR_WAVE, st);
+            for (auto& c : L.wchunk[w])
+                hip_check(launch_rrqr_wave<T>(db, Packer::at<RrqrSlab>(dt, o_p[w]) + c[0], c[1], c[2], wmaxrows[w],
+                                              L.wdense[w] != 0, tol_,
+                                              d_info_ + 1, R.spin_max, st),
+                          "rrqr wave");
+            prof_.stop(sl, st, 0, 0, (int)L.wchunk[w].size());
+            done = true;
+            slot_step[w] = sl;
         }
         if (!done) {
             // Steps are launched at most RRQR_STEPS_AHEAD ahead of the device, and none
