@@ -33,11 +33,13 @@ hipError_t launch_potrf_trail(const PotrfTask* d_tasks, int ntasks, int kb, int 
 // task, run the ordered-FMA vector kernel.
 constexpr int TRSM_MFMA_MIN_N = 64;
 template <typename T> hipError_t launch_trsm(const TrsmTask* d_tasks, int ntasks, int mfma_from, hipStream_t st);
-// LU pivots (GEN / PLU): in_lds = 1 runs the batch in LDS (every task must satisfy
-// n (n + 1) sizeof(T) <= GETRF_LDS_BYTES, nmax the largest n), in_lds = 0 in global memory.
-constexpr int GETRF_LDS_BYTES = 65536;
+// LU pivots (GEN / PLU): launch_getrf_panels up to GETRF_PANEL_MAX rows (tasks with diag and
+// moves set, nmax the largest n), launch_getrf for larger ones.
 template <typename T>
-hipError_t launch_getrf(const GetrfTask* d_tasks, int ntasks, int in_lds, int nmax, int* d_info, hipStream_t st);
+hipError_t launch_getrf(const GetrfTask* d_tasks, int ntasks, int* d_info, hipStream_t st);
+constexpr int GETRF_PANEL_MAX = 4096;
+template <typename T>
+hipError_t launch_getrf_panels(const GetrfTask* d_tasks, int ntasks, int nmax, int* d_info, hipStream_t st);
 template <typename T>
 hipError_t launch_schur(const SchurTile* d_tiles, int ntiles, const SchurContrib* d_contribs, hipStream_t st);
 // Small clusters, one workgroup each. lds_bytes (<= RRQR_LDS_MAX) holds a task's Asn when

@@ -603,13 +603,12 @@ __global__ void __launch_bounds__(NT, 3) k_trsm_f32_mfma(const TrsmTask* tasks) 
 // all columns, the column is scaled by 1/a_jj (divided by a_jj when |a_jj| is below the
 // smallest normal number), then a_ic = a_ic + a_ij * (-a_jc) for every trailing element with
 // a_jc != 0 (dger), in j order -- the element recurrence of the oracle. The row
-// permutation is accumulated as swap2perm does (src/util.cpp:76-88). Blocks of at most
-// GETRF_LDS_BYTES are factored in LDS (ld n + 1), larger ones in place in global memory.
-template <typename T, int NTG>
-__global__ void __launch_bounds__(NTG) k_getrf(const GetrfTask* tasks, int in_lds, int* info) {
+// permutation is accumulated as swap2perm does (src/util.cpp:76-88). In place in global
+// memory, for pivots that the panel kernels below do not hold (n > GETRF_PANEL_MAX).
+template <typename T>
+__global__ void __launch_bounds__(1024) k_getrf(const GetrfTask* tasks, int* info) {
 #pragma clang fp contract(off)
-    extern __shared__ __align__(16) unsigned char getrf_lds[];
-    constexpr int NW = NTG / 64;
+    constexpr int NTG = 1024, NW = NTG / 64;
     __shared__ T red_v[NW];
     __shared__ int red_i[NW];
     __shared__ int s_jp, s_nz, bad;
@@ -620,11 +619,8 @@ __global__ void __launch_bounds__(NTG) k_getrf(const GetrfTask* tasks, int in_ld
     const gptr<T> G = gp(reinterpret_cast<T*>(t.A));
     const gptr<T> Ut = gp(reinterpret_cast<T*>(t.Ut));
     const gptr<int> perm = gp(t.perm);
-    T* A = in_lds ? reinterpret_cast<T*>(getrf_lds) : (T*)G;
-    const int ld = in_lds ? n + 1 : n;
-    if (in_lds)
-        for (int c = wv; c < n; c += NW)
-            for (int i = lane; i < n; i += 64) A[i + (size_t)c * ld] = G[i + (size_t)c * n];
+    const gptr<T> A = G;
+    const int ld = n;
     for (int i = tid; i < n; i += NTG) perm[i] = i;
     if (tid == 0) bad = 0;
     __syncthreads();
@@ -2891,6 +2887,255 @@ hipError_t launch_scatter(const long long* off, const double* val, long long n, 
     return hipGetLastError();
 }
 
+// ---------------------------------------------------------------------------------------
+// LU pivots in panels of NB columns, right-looking, the operations of k_getrf on every element
+// in the same order (same bits). One panel is a launch of k_getrf_panel (one workgroup per
+// pivot) and one of k_getrf_trail (one workgroup per 8 columns); k_getrf_split ends the pivot.
+// The LU pivots of a 64^3 convection-diffusion factorization, FP32, up to 472 rows: 6.4 ms;
+// 10.7 ms with those below 128 rows factored in LDS by one workgroup each, 35.9 ms with the
+// others in one workgroup each in global memory as well.
+//
+// Bound: the chain of pivot searches. A panel's rows stay in registers, RPT a thread, and
+// never move: each row carries its position, an interchange swaps two positions, and rows go
+// to their place at the end of the panel. Each wavefront puts its best row, values included,
+// into LDS, so a step has one barrier. NB RPT = 32 values a thread: 1024, 2048 and 4096 rows
+// with 32, 16 and 8 columns.
+template <typename T, int NB, int RPT>
+__global__ void __launch_bounds__(1024) k_getrf_panel(const GetrfTask* tasks, int kb, int* info) {
+#pragma clang fp contract(off)
+    __shared__ T s_row[2][16][NB];
+    __shared__ double s_v[2][16];
+    __shared__ int s_p[2][16];
+    __shared__ int s_moved;
+    const GetrfTask t = tasks[blockIdx.x];
+    const int n = t.n, tid = threadIdx.x, lane = tid % 64, wv = tid / 64, nt = blockDim.x, nw = nt / 64;
+    if (kb >= n) return;
+    const int nr = n - kb, nc = min(NB, nr);
+    const gptr<T> A = gp(reinterpret_cast<T*>(t.A)) + kb + (size_t)kb * n;
+    const gptr<int> perm = gp(t.perm) + kb;
+    const gptr<T> diag = gp(reinterpret_cast<T*>(t.diag)) + kb;
+    const gptr<int> moves = gp(t.moves);
+    T a[RPT][NB];
+    int pos[RPT], pv[RPT];
+#pragma unroll
+    for (int q = 0; q < RPT; q++) {
+        const int r = tid + q * nt;
+        pos[q] = r < nr ? r : INT_MAX;
+        pv[q] = r < nr && kb > 0 ? perm[r] : r;
+#pragma unroll
+        for (int c = 0; c < NB; c++) a[q][c] = r < nr && c < nc ? A[r + (size_t)c * n] : T(0);
+    }
+    if (tid == 0) s_moved = 0;
+    bool bad = false;
+#pragma unroll
+    for (int j = 0; j < NB; j++) {
+        if (j < nc) {
+            // idamax over positions j..: the first of the largest magnitudes, and position j
+            // itself when it holds a NaN or every candidate does
+            double bv = -1.0;
+            int bp = INT_MAX;
+#pragma unroll
+            for (int q = 0; q < RPT; q++)
+                if (pos[q] >= j && pos[q] != INT_MAX) {
+                    const T x = a[q][j];
+                    const double v = x == x ? (double)fabs(x) : (pos[q] == j ? HUGE_VAL : -1.0);
+                    if (v > bv || (v == bv && pos[q] < bp)) { bv = v; bp = pos[q]; }
+                }
+            wave_best_norm<1>(bv, bp);
+            const int b = j & 1;
+#pragma unroll
+            for (int q = 0; q < RPT; q++)
+                if (pos[q] == bp && bp != INT_MAX)
+#pragma unroll
+                    for (int c = j; c < NB; c++) s_row[b][wv][c] = a[q][c];
+            if (lane == 0) { s_v[b][wv] = bv; s_p[b][wv] = bp; }
+            __syncthreads();
+            bv = lane < nw ? s_v[b][lane] : -1.0;
+            bp = lane < nw ? s_p[b][lane] : INT_MAX;
+            const int mine = bp;
+            wave_best_norm<1>(bv, bp);
+            const int jp = bp, ww = __ffsll((unsigned long long)__ballot(mine == jp)) - 1;
+            const T piv = s_row[b][ww][j];
+#pragma unroll
+            for (int q = 0; q < RPT; q++) {
+                const int p = pos[q];
+                pos[q] = p == jp ? j : (p == j ? jp : p);
+            }
+            if (tid == 0) diag[j] = piv;
+            const bool inv = fabs(piv) >= std::numeric_limits<T>::min();
+            const T r = T(1) / piv;
+            if (piv == T(0)) bad = true;
+#pragma unroll
+            for (int q = 0; q < RPT; q++) {
+                const bool below = pos[q] > j;
+                if (below && piv != T(0)) a[q][j] = inv ? a[q][j] * r : a[q][j] / piv;
+            }
+#pragma unroll
+            for (int c = j + 1; c < NB; c++) {
+                const T y = s_row[b][ww][c];
+                if (y != T(0)) {
+                    const T mt = -y;
+#pragma unroll
+                    for (int q = 0; q < RPT; q++) {
+                        const T u = a[q][c] + a[q][j] * mt;
+                        a[q][c] = pos[q] > j ? u : a[q][c];
+                    }
+                }
+            }
+        }
+    }
+    // rows to their places; moves: the rows that the top positions take, then the count and
+    // (to, from) of the others that moved
+    __syncthreads();  // every read of perm is done
+#pragma unroll
+    for (int q = 0; q < RPT; q++) {
+        const int r = tid + q * nt, p = pos[q];
+        if (r >= nr) continue;
+#pragma unroll
+        for (int c = 0; c < NB; c++)
+            if (c < nc) A[p + (size_t)c * n] = a[q][c];
+        perm[p] = pv[q];
+        if (p < nc) moves[p] = r;
+        else if (p != r) {
+            const int k = atomicAdd(&s_moved, 1);
+            moves[GETRF_NB + 1 + 2 * k] = p;
+            moves[GETRF_NB + 2 + 2 * k] = r;
+        }
+    }
+    __syncthreads();
+    if (tid == 0) {
+        moves[GETRF_NB] = s_moved;
+        if (bad) atomicCAS(info, 0, t.cluster + 1);
+    }
+}
+
+// The panel's interchanges on 8 of the other columns and, right of the panel, their rows of U
+// and the update below: a wavefront solves two columns, a lane each row (readlane hands
+// u_j down), then a thread updates rows of all eight, so that an element of L is read once
+// per 8 products and U comes from LDS at one address per wavefront. Eight columns keep
+// n / 8 workgroups busy.
+template <typename T, int NB>
+__global__ void __launch_bounds__(NT) k_getrf_trail(const GetrfTask* tasks, int kb) {
+#pragma clang fp contract(off)
+    constexpr int W = 8;
+    __shared__ T Us[NB][W], Ls[NB][NB + 1], Ms[GETRF_NB][W];
+    __shared__ int s_zero;
+    const GetrfTask t = tasks[blockIdx.y];
+    const int n = t.n, tid = threadIdx.x, c0 = blockIdx.x * W;
+    if (kb >= n || c0 >= n || (c0 >= kb && c0 < kb + NB)) return;
+    const int nr = n - kb, nc = min(NB, nr), w = min(W, n - c0);
+    const gptr<T> P = gp(reinterpret_cast<T*>(t.A)) + kb + (size_t)kb * n;
+    const gptr<T> C = gp(reinterpret_cast<T*>(t.A)) + kb + (size_t)c0 * n;
+    const gptr<const int> moves = gp((const int*)t.moves);
+    const int nm = moves[GETRF_NB];
+    for (int e = tid; e < NB * W; e += NT) {
+        const int i = e % NB, c = e / NB;
+        Us[i][c] = i < nc && c < w ? C[moves[i] + (size_t)c * n] : T(0);
+    }
+    for (int e = tid; e < nm * W; e += NT) {
+        const int i = e % nm, c = e / nm;
+        Ms[i][c] = c < w ? C[moves[GETRF_NB + 2 + 2 * i] + (size_t)c * n] : T(0);
+    }
+    const bool right = c0 > kb;
+    if (right)
+        for (int e = tid; e < NB * NB; e += NT) Ls[e % NB][e / NB] = P[e % NB + (size_t)(e / NB) * n];
+    if (tid == 0) s_zero = 0;
+    __syncthreads();  // every row that moves is read
+    for (int e = tid; e < nm * w; e += NT) {
+        const int i = e % nm, c = e / nm;
+        C[moves[GETRF_NB + 1 + 2 * i] + (size_t)c * n] = Ms[i][c];
+    }
+    if (!right) {
+        for (int e = tid; e < nc * w; e += NT) C[e % nc + (size_t)(e / nc) * n] = Us[e % nc][e / nc];
+        return;
+    }
+    // right of a panel there are columns left, so the panel is a full one (nc == NB)
+    {
+        const int i = tid % 32, c = tid / 32;
+        T u = i < NB ? Us[i % NB][c] : T(0);
+#pragma unroll
+        for (int j = 0; j < NB; j++) {
+            const T y = __shfl(u, j, 32);
+            const T v = u + Ls[i % NB][j] * -y;
+            if (i > j && y != T(0)) u = v;
+        }
+        if (i < NB) {
+            Us[i][c] = u;
+            if (c < w) C[i + (size_t)c * n] = u;
+            if (u == T(0) && c < w) s_zero = 1;
+        }
+    }
+    __syncthreads();
+    const bool zero = s_zero != 0;
+    for (int p = NB + tid; p < nr; p += NT) {
+        T l[8], ln[8], x[W];
+#pragma unroll
+        for (int j = 0; j < 8; j++) ln[j] = P[p + (size_t)j * n];
+#pragma unroll
+        for (int c = 0; c < W; c++) x[c] = c < w ? C[p + (size_t)c * n] : T(0);
+#pragma unroll 1
+        for (int j0 = 0; j0 < NB; j0 += 8) {
+#pragma unroll
+            for (int j = 0; j < 8; j++) l[j] = ln[j];
+            if (j0 + 8 < NB)
+#pragma unroll
+                for (int j = 0; j < 8; j++) ln[j] = P[p + (size_t)(j0 + 8 + j) * n];
+            if (!zero) {
+#pragma unroll
+                for (int j = 0; j < 8; j++)
+#pragma unroll
+                    for (int c = 0; c < W; c++) x[c] = x[c] + l[j] * -Us[j0 + j][c];
+            } else {
+#pragma unroll
+                for (int j = 0; j < 8; j++)
+#pragma unroll
+                    for (int c = 0; c < W; c++) {
+                        const T y = Us[j0 + j][c];
+                        const T v = x[c] + l[j] * -y;
+                        x[c] = y != T(0) ? v : x[c];
+                    }
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < W; c++)
+            if (c < w) C[p + (size_t)c * n] = x[c];
+    }
+}
+
+// split_LU of k_getrf, one workgroup per 32 x 32 tile: the upper tiles leave transposed to
+// Ut through LDS (both sides coalesced); diag holds the pivots, since A's diagonal is
+// overwritten while other tiles still need it.
+template <typename T>
+__global__ void __launch_bounds__(NT) k_getrf_split(const GetrfTask* tasks) {
+#pragma clang fp contract(off)
+    __shared__ T tile[32][33];
+    const GetrfTask t = tasks[blockIdx.y];
+    const int n = t.n, nt = (n + 31) / 32;
+    if ((int)blockIdx.x >= nt * nt) return;
+    const int r0 = blockIdx.x % nt * 32, c0 = blockIdx.x / nt * 32;
+    const gptr<T> A = gp(reinterpret_cast<T*>(t.A)), Ut = gp(reinterpret_cast<T*>(t.Ut));
+    const gptr<const T> diag = gp(reinterpret_cast<const T*>(t.diag));
+    const int x = threadIdx.x % 32;
+    for (int y = threadIdx.x / 32; y < 32; y += NT / 32) {
+        const int r = r0 + x, c = c0 + y;
+        if (r >= n || c >= n) continue;
+        const T d = diag[min(r, c)];
+        const auto ap = A + r + (size_t)c * n;
+        if (r > c) {
+            *ap = *ap * sqrt(fabs(d));
+            tile[y][x] = T(0);
+        } else {
+            const T f = T((d > T(0)) - (d < T(0))) * sqrt(fabs(d));
+            const T inv = T(1) / d;
+            tile[y][x] = r == c ? f * T(1) : f * (inv * *ap);
+            *ap = r == c ? sqrt(fabs(d)) * T(1) : T(0);
+        }
+    }
+    __syncthreads();
+    for (int y = threadIdx.x / 32; y < 32; y += NT / 32)
+        if (c0 + x < n && r0 + y < n) Ut[(c0 + x) + (size_t)(r0 + y) * n] = tile[x][y];
+}
+
 template <typename T>
 hipError_t launch_potrf(const PotrfTask* d_tasks, int ntasks, int* d_info, hipStream_t st) {
     if (ntasks == 0) return hipSuccess;
@@ -2932,15 +3177,42 @@ hipError_t launch_trsm(const TrsmTask* d_tasks, int ntasks, int mfma_from, hipSt
 }
 
 template <typename T>
-hipError_t launch_getrf(const GetrfTask* d_tasks, int ntasks, int in_lds, int nmax, int* d_info, hipStream_t st) {
+hipError_t launch_getrf(const GetrfTask* d_tasks, int ntasks, int* d_info, hipStream_t st) {
     if (ntasks == 0) return hipSuccess;
-    if (in_lds) {
-        const size_t bytes = (size_t)nmax * (nmax + 1) * sizeof(T);
-        if (bytes > (size_t)GETRF_LDS_BYTES) return hipErrorInvalidValue;
-        k_getrf<T, NT><<<ntasks, NT, bytes, st>>>(d_tasks, 1, d_info);
-    } else {
-        k_getrf<T, 1024><<<ntasks, 1024, 0, st>>>(d_tasks, 0, d_info);
+    k_getrf<T><<<ntasks, 1024, 0, st>>>(d_tasks, d_info);
+    return hipGetLastError();
+}
+
+template <typename T, int NB, int RPT>
+static hipError_t getrf_panel_step(const GetrfTask* d_tasks, int ntasks, int kb, int nmax, int* d_info,
+                                   hipStream_t st) {
+    const int rows = (nmax - kb + RPT - 1) / RPT;
+    k_getrf_panel<T, NB, RPT><<<ntasks, (rows + 63) / 64 * 64, 0, st>>>(d_tasks, kb, d_info);
+    if (nmax > NB) k_getrf_trail<T, NB><<<dim3((nmax + 7) / 8, ntasks), NT, 0, st>>>(d_tasks, kb);
+    return hipGetLastError();
+}
+
+template <typename T>
+hipError_t launch_getrf_panels(const GetrfTask* d_tasks, int ntasks, int nmax, int* d_info, hipStream_t st) {
+    if (ntasks == 0 || nmax == 0) return hipSuccess;
+    if (nmax > GETRF_PANEL_MAX) return hipErrorInvalidValue;
+    for (int kb = 0; kb < nmax;) {
+        const int rows = nmax - kb;
+        hipError_t e;
+        if (rows <= 1024) {
+            e = getrf_panel_step<T, 32, 1>(d_tasks, ntasks, kb, nmax, d_info, st);
+            kb += 32;
+        } else if (rows <= 2048) {
+            e = getrf_panel_step<T, 16, 2>(d_tasks, ntasks, kb, nmax, d_info, st);
+            kb += 16;
+        } else {
+            e = getrf_panel_step<T, 8, 4>(d_tasks, ntasks, kb, nmax, d_info, st);
+            kb += 8;
+        }
+        if (e != hipSuccess) return e;
     }
+    const int nt = (nmax + 31) / 32;
+    k_getrf_split<T><<<dim3(nt * nt, ntasks), NT, 0, st>>>(d_tasks);
     return hipGetLastError();
 }
 
@@ -3256,7 +3528,8 @@ hipError_t launch_copy(const CopyTask* d_tasks, int ntasks, hipStream_t st) {
     template hipError_t launch_potrf_panel<T>(const PotrfTask*, int, int, int, int*, hipStream_t);     \
     template hipError_t launch_potrf_trail<T>(const PotrfTask*, int, int, int, hipStream_t);      \
     template hipError_t launch_trsm<T>(const TrsmTask*, int, int, hipStream_t);                   \
-    template hipError_t launch_getrf<T>(const GetrfTask*, int, int, int, int*, hipStream_t);      \
+    template hipError_t launch_getrf<T>(const GetrfTask*, int, int*, hipStream_t);                \
+    template hipError_t launch_getrf_panels<T>(const GetrfTask*, int, int, int*, hipStream_t);    \
     template hipError_t launch_schur<T>(const SchurTile*, int, const SchurContrib*, hipStream_t); \
     template hipError_t launch_rrqr<T>(const RrqrTask*, int, const RrqrSeg*, int*, double, int, hipStream_t); \
     template hipError_t launch_rrqr_reg<T>(const RrqrTask*, int, const RrqrSeg*, int*, double, int, hipStream_t); \

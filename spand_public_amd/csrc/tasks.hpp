@@ -46,7 +46,13 @@ struct GetrfTask {
     int* perm;
     int n;
     int cluster;  // reported through the info array on a zero pivot
+    void* diag;   // panel launches: the n pivots, for split_LU
+    int* moves;   // and the current panel's row interchanges (GETRF_MOVES)
 };
+// moves: the row that each of the panel's GETRF_NB top positions takes, the number of the
+// other rows that moved, and (to, from) of each, all counted from the panel's first row.
+constexpr int GETRF_NB = 32;
+constexpr int GETRF_MOVES = 3 * GETRF_NB + 1;
 
 // One Schur-complement target tile: C[r0:r0+tm, c0:c0+tn] of a block C (ldc rows) receives
 // contributions [k0, k1) in order, each C -= opA(A) opB(B) (gemm / syrk, src/util.cpp:122-156).

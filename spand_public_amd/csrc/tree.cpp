@@ -972,12 +972,15 @@ static void small_first(std::vector<PotrfTask>& v) {
     std::stable_partition(v.begin(), v.end(), [](const PotrfTask& t) { return t.n <= POTRF_SMALL_MAX; });
     std::stable_partition(v.begin(), v.end(), [](const PotrfTask& t) { return t.n <= 64; });
 }
-// LU pivots that fit LDS first (one launch), the larger ones after (another)
+// LU pivots that the panel kernels hold first, with their buffers.
 template <typename T>
-static void lds_first(std::vector<GetrfTask>& v) {
-    std::stable_partition(v.begin(), v.end(), [](const GetrfTask& t) {
-        return (size_t)t.n * (t.n + 1) * sizeof(T) <= (size_t)GETRF_LDS_BYTES;
-    });
+void Tree::order_getrf(std::vector<GetrfTask>& v) {
+    std::stable_partition(v.begin(), v.end(), [](const GetrfTask& t) { return t.n <= GETRF_PANEL_MAX; });
+    for (GetrfTask& t : v)
+        if (t.n <= GETRF_PANEL_MAX) {
+            t.diag = arena_.alloc((size_t)std::max(1, t.n) * sizeof(T));
+            t.moves = reinterpret_cast<int*>(arena_.alloc(GETRF_MOVES * sizeof(int)));
+        }
 }
 
 // Cholesky pivots of one batch: up to POTRF_SMALL_MAX in one launch (one workgroup each;
@@ -1040,34 +1043,34 @@ void Tree::run_trsm(hipStream_t st, void* dt, const std::vector<TrsmTask>& v, si
               what);
 }
 
-// LU pivots of one batch: those that fit LDS in one launch, the larger ones in another.
+// LU pivots of one batch (order_getrf): those that the panel kernels hold, then the others.
 template <typename T>
 void Tree::run_getrf(hipStream_t st, void* dt, const std::vector<GetrfTask>& v, size_t off, const char* what) {
     const size_t esz = sizeof(T);
     if (v.empty()) return;
-    int nl = 0, nmax_l = 0;
-    double lb = 0, lf = 0, gb = 0, gf = 0;
+    int np = 0, nmax = 0;
+    double pb = 0, pf = 0, gb = 0, gf = 0;
     for (auto& t : v) {
         const double n = t.n;
         const double by = (3.0 * n * n) * esz + 4.0 * n, fl = getrf_flops(n);
-        if ((size_t)t.n * (t.n + 1) * esz <= (size_t)GETRF_LDS_BYTES) {
-            nl++;
-            nmax_l = std::max(nmax_l, t.n);
-            lb += by;
-            lf += fl;
+        if (t.n <= GETRF_PANEL_MAX) {
+            np++;
+            nmax = std::max(nmax, t.n);
+            pb += by;
+            pf += fl;
         } else {
             gb += by;
             gf += fl;
         }
     }
     const GetrfTask* d = Packer::at<GetrfTask>(dt, off);
-    if (nl > 0)
-        hip_check(timed(prof_, KF_GETRF, st, lb, lf,
-                        [&] { return launch_getrf<T>(d, nl, 1, nmax_l, d_info_, st); }),
+    if (np > 0)
+        hip_check(timed(prof_, KF_GETRF, st, pb, pf,
+                        [&] { return launch_getrf_panels<T>(d, np, nmax, d_info_, st); }),
                   what);
-    if (nl < (int)v.size())
+    if (np < (int)v.size())
         hip_check(timed(prof_, KF_GETRF, st, gb, gf,
-                        [&] { return launch_getrf<T>(d + nl, (int)v.size() - nl, 0, 0, d_info_, st); }),
+                        [&] { return launch_getrf<T>(d + np, (int)v.size() - np, d_info_, st); }),
                   what);
 }
 
@@ -1140,7 +1143,7 @@ void Tree::plan_elimination(LevelPlan<T>& L) {
             // getf_cluster + panel_getf + gemm_edges, PLU branch (src/tree.cpp:929-956)
             void* Ut = arena_.alloc((size_t)std::max(1, n * n) * sizeof(T));
             int* pp = reinterpret_cast<int*>(arena_.alloc((size_t)std::max(1, n) * sizeof(int)));
-            getrfE.push_back({piv.A, Ut, pp, n, c});
+            getrfE.push_back({piv.A, Ut, pp, n, c, nullptr, nullptr});
             lst.flops_potrf += getrf_flops(n);
             log_shape(SK_GETF, n, 0, 0);
             std::vector<int> out(s.out.begin() + 1, s.out.end()), in(s.in.begin(), s.in.end());
@@ -1333,7 +1336,6 @@ void Tree::launch_elimination(LevelPlan<T>& L) {
     // Nothing planned below feeds the elimination group (fill-in zeroing, identity inits
     // of the explicit inverses, pivots, panels, Schur updates): it is launched now, so the
     // device eliminates while the host plans the level's scaling and sparsification.
-    // LU pivots that fit LDS first (one launch), the larger ones after (another)
     // pivots up to POTRF_SMALL_MAX in one launch (one workgroup each); larger ones (sorted
     // last) one 32-column panel per launch pair
     L.n_potrf_elim = potrfE.size();
@@ -1341,7 +1343,7 @@ void Tree::launch_elimination(LevelPlan<T>& L) {
         small_first(potrfE);
         for (PotrfTask& t : potrfE)
             if (t.n > POTRF_SMALL_MAX) t.dbuf = arena_.alloc(32 * 32 * sizeof(T));
-        lds_first<T>(getrfE);
+        order_getrf<T>(getrfE);
         Packer pe;
         const int sp_te = split_trsm(trsmE);
         const size_t o_pe = pe.add(potrfE), o_te = pe.add(trsmE), o_ti = pe.add(tiles), o_co = pe.add(contribs);
@@ -1419,7 +1421,7 @@ void Tree::plan_scaling(LevelPlan<T>& L) {
             void* Ut = arena_.alloc((size_t)std::max(1, n * n) * sizeof(T));
             int* pp = reinterpret_cast<int*>(arena_.alloc((size_t)std::max(1, n) * sizeof(int)));
             lu[c] = {Ut, pp};
-            getrfS.push_back({piv.A, Ut, pp, n, c});
+            getrfS.push_back({piv.A, Ut, pp, n, c, nullptr, nullptr});
             lst.flops_potrf += getrf_flops(n);
             ops_.push_back({OP_SCALING_PLUQ, c, -1, n, 0, n, n, ilvl_, piv.A, nullptr, Ut, pp});
             factor_bytes_ += (size_t)n * (n + 1) * sizeof(T) + (size_t)n * sizeof(int);
@@ -1868,7 +1870,7 @@ void Tree::launch_level(LevelPlan<T>& L) {
     const int sp_ta = split_trsm(trsmA), sp_tb = split_trsm(trsmB);
     size_t o_ps = pk.add(potrfS), o_ta = pk.add(trsmA), o_tb = pk.add(trsmB), o_sg = pk.add(segs);
     size_t o_ii = pk.add(inv_init);
-    lds_first<T>(getrfS);
+    order_getrf<T>(getrfS);
     size_t o_gs = pk.add(getrfS);
     std::vector<size_t> o_w(nwaves), o_b(nwaves), o_s(nwaves), o_r(nwaves), o_p(nwaves);
     for (int w = 0; w < nwaves; w++) {

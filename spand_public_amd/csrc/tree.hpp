@@ -243,6 +243,8 @@ class Tree {
     template <typename T>
     void run_trsm(hipStream_t st, void* dt, const std::vector<TrsmTask>& v, size_t off, int split, const char* what);
     template <typename T>
+    void order_getrf(std::vector<GetrfTask>& v);
+    template <typename T>
     void run_getrf(hipStream_t st, void* dt, const std::vector<GetrfTask>& v, size_t off, const char* what);
     // ws_ext: a caller-provided workspace of apply_workspace_bytes(nrhs) (then nothing is
     // allocated and no launch is timed), or nullptr for the tree's own.
