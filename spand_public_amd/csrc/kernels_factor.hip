@@ -392,20 +392,64 @@ __global__ void __launch_bounds__(NT) k_potrf_trail(const PotrfTask* tasks, int 
 }
 
 // ---------------------------------------------------------------------------------------
+// 16 x 16 x 4 products on the matrix cores, in the element's own precision. Lane l holds row
+// (column) l % 16 of the A (B) operand at inner index l / 16. D += A B adds the four products in
+// increasing inner index by fused multiply-adds, each rounded, denormals kept: the bits of
+// the scalar chain fma(a_k, b_k, d).
+template <typename T> struct Mat16;
+template <> struct Mat16<double> {
+    using V = double __attribute__((ext_vector_type(4)));
+    static __device__ inline V mac(double a, double b, V d) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, d, 0, 0, 0); }
+    static __device__ inline int row(int lane, int v) { return (lane >> 4) + 4 * v; }  // of register v; column lane % 16
+};
+template <> struct Mat16<float> {
+    using V = float __attribute__((ext_vector_type(4)));
+    static __device__ inline V mac(float a, float b, V d) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, d, 0, 0, 0); }
+    static __device__ inline int row(int lane, int v) { return 4 * (lane >> 4) + v; }
+};
+
+// Value of v in lane Q of the calling lane's quad.
+template <int Q>
+__device__ inline int quad_bcast(int v) { return __builtin_amdgcn_mov_dpp(v, 0x55 * Q, 0xf, 0xf, true); }
+template <int Q>
+__device__ inline float quad_bcast(float v) { return __int_as_float(quad_bcast<Q>(__float_as_int(v))); }
+template <int Q>
+__device__ inline double quad_bcast(double v) {
+    return __hiloint2double(quad_bcast<Q>(__double2hiint(v)), quad_bcast<Q>(__double2loint(v)));
+}
+template <typename T>
+__device__ inline T quad_bcast(T v, int q) {  // q: a constant after unrolling
+    return q == 0 ? quad_bcast<0>(v) : q == 1 ? quad_bcast<1>(v) : q == 2 ? quad_bcast<2>(v) : quad_bcast<3>(v);
+}
+
 // trsm on a chunk of <= 64 independent columns (left) or rows (right), in 32-row blocks of
-// L: the diagonal triangle is solved by one thread per independent index, the rows below
-// by the whole workgroup as an ordered-FMA update. Every element sees the reference BLAS
-// operations in the same order (FP64 bit-identical to the oracle).
+// L. Bound by the chain of the diagonal blocks (32 dependent divisions each for a left solve)
+// and by the blocks' round trips through global memory.
+//   * The diagonal triangle is solved by four lanes per independent index, lane s of the quad
+//     holding rows s, s + 4, .. in registers; the row of a step reaches the others by DPP. One
+//     lane per index left three of four wavefronts idle, and walked 496 multiply-adds, an LDS
+//     read each, where a lane now walks 144.
+//   * The rows below are updated on the matrix cores, 16 rows x 32 indices a wavefront: L's
+//     operand is loaded straight from global memory (16 contiguous rows of 4 columns), X from
+//     LDS, and a tile's lanes run along the contiguous index of the target (left solves
+//     compute it transposed). The vector form read LDS twice per multiply-add.
+// Every element sees the reference BLAS operations in the same order (FP64 bit-identical to
+// the oracle). The trsm launches of one 64^3 Laplacian factorization, FP64: 15.3 ms in the
+// vector form, 6.8 in this one; with the other kernels, factor + PCG 93.3 -> 85.9 ms (FP32
+// 76.4 -> 71.0).
 template <typename T>
 __global__ void __launch_bounds__(NT) k_trsm(const TrsmTask* tasks) {
 #pragma clang fp contract(off)
+    using M = Mat16<T>;
     __shared__ T Bk[PB][64 + 1];
-    __shared__ T Lk[PB][PB + 1];
-    __shared__ T Lr[PB][64 + 1];
+    __shared__ T Lk[PB][PB + 1];  // Lk[k][i]: column k of the diagonal block
+    __shared__ T rd[PB];          // 1 / L(k, k), for right solves
     const TrsmTask t = tasks[blockIdx.x];
     const int n = t.n, m = t.m, ld = t.ldb;
     const int tid = threadIdx.x;
     if (n == 0 || m == 0) return;
+    const int lane = tid & 63, r16 = lane & 15, k4 = lane >> 4;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const gptr<const T> L = gp(reinterpret_cast<const T*>(t.L));
     const gptr<T> G = gp(reinterpret_cast<T*>(t.B));
     const bool left = t.side == 0;
@@ -427,33 +471,30 @@ __global__ void __launch_bounds__(NT) k_trsm(const TrsmTask* tasks) {
         }
         for (int idx = tid; idx < nb * nb; idx += NT) {
             int i = idx % nb, k = idx / nb;
-            Lk[i][k] = L[(kb + i) + (size_t)(kb + k) * n];
+            const T v = L[(kb + i) + (size_t)(kb + k) * n];
+            Lk[k][i] = v;
+            if (i == k && !left) rd[k] = T(1) / v;
         }
         __syncthreads();
-        if (tid < m) {  // column c of the diagonal block, held in registers
-            const int c = tid;
-            T x[PB];
+        if (tid < 4 * m) {  // index c; rows nb.. hold nothing that a row below nb reads
+            const int c = tid >> 2, sub = tid & 3;
+            T x[PB / 4];
 #pragma unroll
-            for (int k = 0; k < PB; k++) x[k] = k < nb ? Bk[k][c] : T(0);
+            for (int q = 0; q < PB / 4; q++) x[q] = 4 * q + sub < nb ? Bk[4 * q + sub][c] : T(0);
 #pragma unroll
             for (int k = 0; k < PB; k++) {
                 if (k < nb) {
-                    T b;
-                    if (left) {
-                        b = x[k] / Lk[k][k];
-                    } else {
-                        const T r = T(1) / Lk[k][k];
-                        b = x[k] * r;
-                    }
-                    x[k] = b;
+                    const T xk = quad_bcast(x[k / 4], k % 4);
+                    const T b = left ? xk / Lk[k][k] : xk * rd[k];
+                    const T u = fma(-b, Lk[k][(k & ~3) + sub], x[k / 4]);
+                    x[k / 4] = sub == k % 4 ? b : (sub > k % 4 ? u : x[k / 4]);
 #pragma unroll
-                    for (int i = k + 1; i < PB; i++)
-                        if (i < nb) x[i] = fma(-b, Lk[i][k], x[i]);
+                    for (int q = k / 4 + 1; q < PB / 4; q++) x[q] = fma(-b, Lk[k][4 * q + sub], x[q]);
                 }
             }
 #pragma unroll
-            for (int k = 0; k < PB; k++)
-                if (k < nb) Bk[k][c] = x[k];
+            for (int q = 0; q < PB / 4; q++)
+                if (4 * q + sub < nb) Bk[4 * q + sub][c] = x[q];
         }
         __syncthreads();
         for (int idx = tid; idx < nb * m; idx += NT) {
@@ -461,138 +502,52 @@ __global__ void __launch_bounds__(NT) k_trsm(const TrsmTask* tasks) {
             if (left) { k = idx % nb; c = idx / nb; } else { c = idx % m; k = idx / m; }
             at(kb + k, c) = Bk[k][c];
         }
-        // rows below the block, 64 at a time: L[i0:i0+64, kb:kb+nb] staged in LDS
-        for (int i0 = kb + nb; i0 < n; i0 += 64) {
-            const int ni = min(64, n - i0);
-            for (int idx = tid; idx < ni * nb; idx += NT) {
-                const int ii = idx % ni, k = idx / ni;
-                Lr[k][ii] = L[(i0 + ii) + (size_t)(kb + k) * n];
-            }
-            __syncthreads();
-            for (int idx = tid; idx < ni * m; idx += NT) {
-                int ii, c;
-                if (left) { ii = idx % ni; c = idx / ni; } else { c = idx % m; ii = idx / m; }
-                T acc = kb == 0 ? first(i0 + ii, c) : at(i0 + ii, c);
-                if (nb == PB) {  // a full block: unrolled, so the LDS reads run ahead of the FMAs
+        // rows below the block (nb = PB then): tiles of 16 rows x 32 indices. Rows and indices
+        // past the end read the last one; what they give is not stored.
+        const int e0 = kb + nb, pairs = (m + 31) / 32, tiles = (n - e0 + 15) / 16 * pairs;
+        for (int tl = wv; tl < tiles; tl += NT / 64) {
+            const int i0 = e0 + tl / pairs * 16, c0 = tl % pairs * 32;
+            const bool two = c0 + 16 < m;
+            const int li = min(i0 + r16, n - 1);
+            T l[PB / 4];
 #pragma unroll
-                    for (int k = 0; k < PB; k++) acc = fma(-Bk[k][c], Lr[k][ii], acc);
-                } else {
-                    for (int k = 0; k < nb; k++) acc = fma(-Bk[k][c], Lr[k][ii], acc);
+            for (int q = 0; q < PB / 4; q++) l[q] = L[li + (size_t)(kb + 4 * q + k4) * n];
+            typename M::V acc[2] = {};
+            auto elem = [&](int h, int v, auto&& f) {  // register v of tile h: row i, index c
+                const int w = M::row(lane, v);
+                const int i = i0 + (left ? r16 : w), c = c0 + 16 * h + (left ? w : r16);
+                f(i, c);
+            };
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+                if (h == 0 || two) {
+#pragma unroll
+                    for (int v = 0; v < 4; v++)
+                        elem(h, v, [&](int i, int c) {
+                            i = min(i, n - 1);
+                            c = min(c, m - 1);
+                            acc[h][v] = kb == 0 ? first(i, c) : at(i, c);
+                        });
                 }
-                at(i0 + ii, c) = acc;
-            }
-            __syncthreads();
-        }
-    }
-}
-
-// ---------------------------------------------------------------------------------------
-// FP32 trsm with the trailing updates on the matrix cores. Same blocking as k_trsm: the
-// 32 x 32 diagonal block is solved by one thread per independent index (the recurrence of
-// k_trsm), and each 64-row group below it is updated as C -= L[i0:i0+64, kb:kb+32] X by
-// v_mfma_f32_32x32x2f32 with FP32 accumulation: four wavefronts, one 32 x 32 output tile
-// each. The tile is laid out so that the lanes of a wavefront run along the contiguous
-// index of the target block: left solves (C(i, c) at i + c ld) compute the tile transposed,
-// D(c, i) = X^T L^T, right solves (C(c, i) at c + i ld) compute D(i, c) = L X. FP32 only:
-// the FP64 path keeps the ordered-FMA recurrence of k_trsm.
-typedef float mfma_f32x16 __attribute__((ext_vector_type(16)));
-__global__ void __launch_bounds__(NT, 3) k_trsm_f32_mfma(const TrsmTask* tasks) {
-    __shared__ float Bk[PB][64 + 1];
-    __shared__ float Lk[PB][PB + 1];
-    __shared__ float Lr[PB][64 + 1];
-    const TrsmTask t = tasks[blockIdx.x];
-    const int n = t.n, m = t.m, ld = t.ldb;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    if (n == 0 || m == 0) return;
-    const float* L = reinterpret_cast<const float*>(t.L);
-    float* G = reinterpret_cast<float*>(t.B);
-    const bool left = t.side == 0;
-    auto at = [&](int i, int c) -> float& { return left ? G[i + (size_t)c * ld] : G[c + (size_t)i * ld]; };
-    const float* S = reinterpret_cast<const float*>(t.src);
-    const int* P = t.perm;
-    auto first = [&](int i, int c) -> float { return S ? S[(P ? P[i] : i) + (size_t)c * ld] : at(i, c); };
-    // this wavefront's output tile: rows rh*32.. of the 64-row group, columns ch*32.. of the chunk
-    const int rh = wv & 1, ch = wv >> 1;
-    for (int kb = 0; kb < n; kb += PB) {
-        const int nb = min(PB, n - kb);
-        for (int idx = tid; idx < PB * 64; idx += NT) {  // zero padding: rows >= nb contribute nothing
-            int k, c;
-            if (left) { k = idx % PB; c = idx / PB; } else { c = idx % 64; k = idx / 64; }
-            Bk[k][c] = (k < nb && c < m) ? (kb == 0 ? first(kb + k, c) : at(kb + k, c)) : 0.0f;
-        }
-        for (int idx = tid; idx < nb * nb; idx += NT) {
-            int i = idx % nb, k = idx / nb;
-            Lk[i][k] = L[(kb + i) + (size_t)(kb + k) * n];
-        }
-        __syncthreads();
-        if (tid < m) {  // column c of the diagonal block, held in registers
-            const int c = tid;
-            float x[PB];
 #pragma unroll
-            for (int k = 0; k < PB; k++) x[k] = k < nb ? Bk[k][c] : 0.0f;
+            for (int q = 0; q < PB / 4; q++)
 #pragma unroll
-            for (int k = 0; k < PB; k++) {
-                if (k < nb) {
-                    float b;
-                    if (left) {
-                        b = x[k] / Lk[k][k];
-                    } else {
-                        const float r = 1.0f / Lk[k][k];
-                        b = x[k] * r;
+                for (int h = 0; h < 2; h++)
+                    if (h == 0 || two) {
+                        const T x = Bk[4 * q + k4][c0 + 16 * h + r16];
+                        acc[h] = left ? M::mac(x, -l[q], acc[h]) : M::mac(-l[q], x, acc[h]);
                     }
-                    x[k] = b;
 #pragma unroll
-                    for (int i = k + 1; i < PB; i++)
-                        if (i < nb) x[i] = fmaf(-b, Lk[i][k], x[i]);
+            for (int h = 0; h < 2; h++)
+                if (h == 0 || two) {
+#pragma unroll
+                    for (int v = 0; v < 4; v++)
+                        elem(h, v, [&](int i, int c) {
+                            if (i < n && c < m) at(i, c) = acc[h][v];
+                        });
                 }
-            }
-#pragma unroll
-            for (int k = 0; k < PB; k++)
-                if (k < nb) Bk[k][c] = x[k];
         }
         __syncthreads();
-        for (int idx = tid; idx < nb * m; idx += NT) {
-            int k, c;
-            if (left) { k = idx % nb; c = idx / nb; } else { c = idx % m; k = idx / m; }
-            at(kb + k, c) = Bk[k][c];
-        }
-        for (int i0 = kb + nb; i0 < n; i0 += 64) {
-            const int ni = min(64, n - i0);
-            for (int idx = tid; idx < PB * 64; idx += NT) {
-                const int ii = idx % 64, k = idx / 64;
-                Lr[k][ii] = (ii < ni && k < nb) ? L[(i0 + ii) + (size_t)(kb + k) * n] : 0.0f;
-            }
-            __syncthreads();
-            if (rh * 32 < ni && ch * 32 < m) {
-                // element v of this lane: tile row (8 (v/4) + 4 (lane/32) + v%4), tile column lane%32
-                const int tc = lane & 31, tr0 = 4 * (lane >> 5);
-                mfma_f32x16 acc;
-#pragma unroll
-                for (int v = 0; v < 16; v++) {
-                    const int tr = 8 * (v >> 2) + tr0 + (v & 3);
-                    // left: tile rows are chunk columns c, tile columns are rows i; right: the reverse
-                    const int ii = rh * 32 + (left ? tc : tr), c = ch * 32 + (left ? tr : tc);
-                    float val = 0.0f;
-                    if (ii < ni && c < m) val = kb == 0 ? first(i0 + ii, c) : at(i0 + ii, c);
-                    acc[v] = val;
-                }
-#pragma unroll
-                for (int k = 0; k < PB; k += 2) {
-                    const int kk = k + (lane >> 5);
-                    const float x = -Bk[kk][ch * 32 + (lane & 31)];
-                    const float l = Lr[kk][rh * 32 + (lane & 31)];
-                    acc = left ? __builtin_amdgcn_mfma_f32_32x32x2f32(x, l, acc, 0, 0, 0)
-                               : __builtin_amdgcn_mfma_f32_32x32x2f32(l, x, acc, 0, 0, 0);
-                }
-#pragma unroll
-                for (int v = 0; v < 16; v++) {
-                    const int tr = 8 * (v >> 2) + tr0 + (v & 3);
-                    const int ii = rh * 32 + (left ? tc : tr), c = ch * 32 + (left ? tr : tc);
-                    if (ii < ni && c < m) at(i0 + ii, c) = acc[v];
-                }
-            }
-            __syncthreads();
-        }
     }
 }
 
@@ -781,6 +736,7 @@ __global__ void __launch_bounds__(NT) k_schur(const SchurTile* tiles, const Schu
 // contributions with v_mfma_f32_32x32x2f32 (FP32 accumulation, the tile computed
 // transposed so that a wavefront's lanes run down the target's columns), and the four
 // partial sums are added in LDS and subtracted from the target once at the end.
+typedef float mfma_f32x16 __attribute__((ext_vector_type(16)));
 __global__ void __launch_bounds__(NT) k_schur_f32_mfma(const SchurTile* tiles, const SchurContrib* contribs) {
     __shared__ float As[SK][ST + 1];
     __shared__ float Bs[SK][ST + 1];
@@ -3143,37 +3099,19 @@ hipError_t launch_potrf(const PotrfTask* d_tasks, int ntasks, int* d_info, hipSt
     return hipGetLastError();
 }
 
-// FP32 updates on the matrix cores. The Schur update takes them unless SPAND_SCHUR_MFMA=0.
-// The trsm's trailing updates only with SPAND_TRSM_MFMA=1: on the 64^3 workload its time is
-// in the sequential diagonal-block solves and the block loads, and the matrix-core form
-// measured slower (12.4 ms against 10.7 ms of trsm per FP32 factorization, kernel trace).
+// The FP32 Schur update adds four partial sums unless SPAND_SCHUR_MFMA=0.
 static bool env_flag(const char* name, bool dflt) {
     const char* e = std::getenv(name);
     if (!e || !e[0]) return dflt;
     return e[0] != '0';
 }
-static bool trsm_mfma_enabled() { return env_flag("SPAND_TRSM_MFMA", false); }
 static bool schur_mfma_enabled() { return env_flag("SPAND_SCHUR_MFMA", true); }
 
 template <typename T>
-hipError_t launch_trsm(const TrsmTask* d_tasks, int ntasks, int mfma_from, hipStream_t st) {
+hipError_t launch_trsm(const TrsmTask* d_tasks, int ntasks, hipStream_t st) {
     if (ntasks == 0) return hipSuccess;
-    int nv = ntasks;  // tasks for the vector kernel
-    if constexpr (sizeof(T) == sizeof(float)) {
-        if (trsm_mfma_enabled()) nv = std::max(0, std::min(mfma_from, ntasks));
-    }
-    if (nv > 0) {
-        k_trsm<T><<<nv, NT, 0, st>>>(d_tasks);
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-    }
-    if constexpr (sizeof(T) == sizeof(float)) {
-        if (nv < ntasks) {
-            k_trsm_f32_mfma<<<ntasks - nv, NT, 0, st>>>(d_tasks + nv);
-            return hipGetLastError();
-        }
-    }
-    return hipSuccess;
+    k_trsm<T><<<ntasks, NT, 0, st>>>(d_tasks);
+    return hipGetLastError();
 }
 
 template <typename T>
@@ -3527,7 +3465,7 @@ hipError_t launch_copy(const CopyTask* d_tasks, int ntasks, hipStream_t st) {
     template hipError_t launch_potrf64<T>(const PotrfTask*, int, int*, hipStream_t);              \
     template hipError_t launch_potrf_panel<T>(const PotrfTask*, int, int, int, int*, hipStream_t);     \
     template hipError_t launch_potrf_trail<T>(const PotrfTask*, int, int, int, hipStream_t);      \
-    template hipError_t launch_trsm<T>(const TrsmTask*, int, int, hipStream_t);                   \
+    template hipError_t launch_trsm<T>(const TrsmTask*, int, hipStream_t);                        \
     template hipError_t launch_getrf<T>(const GetrfTask*, int, int*, hipStream_t);                \
     template hipError_t launch_getrf_panels<T>(const GetrfTask*, int, int, int*, hipStream_t);    \
     template hipError_t launch_schur<T>(const SchurTile*, int, const SchurContrib*, hipStream_t); \

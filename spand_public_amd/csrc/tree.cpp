@@ -593,13 +593,6 @@ static std::vector<int> group_by_first(int n, int nkeys, KeyOf key, std::vector<
     return order;
 }
 
-// Triangles of at most TRSM_MFMA_MIN_N rows first (the vector kernel: they have no trailing
-// update to speak of), longer ones after (FP32: the matrix-core kernel); returns the split.
-static int split_trsm(std::vector<TrsmTask>& v) {
-    auto it = std::stable_partition(v.begin(), v.end(), [](const TrsmTask& t) { return t.n <= TRSM_MFMA_MIN_N; });
-    return (int)(it - v.begin());
-}
-
 static inline double potrf_flops(double n) { return n * n * n / 3.0; }
 static inline double getrf_flops(double n) { return 2.0 * n * n * n / 3.0; }
 
@@ -1032,14 +1025,14 @@ void Tree::run_potrf(hipStream_t st, void* dt, const std::vector<PotrfTask>& v, 
     }
 }
 
-// One trsm batch (split: the first task that may take the matrix-core kernel).
+// One trsm batch.
 template <typename T>
-void Tree::run_trsm(hipStream_t st, void* dt, const std::vector<TrsmTask>& v, size_t off, int split, const char* what) {
+void Tree::run_trsm(hipStream_t st, void* dt, const std::vector<TrsmTask>& v, size_t off, const char* what) {
     const size_t esz = sizeof(T);
     if (v.empty()) return;
     Work w = work_trsm(v, esz);
     hip_check(timed(prof_, KF_TRSM, st, w.bytes, w.flops,
-                    [&] { return launch_trsm<T>(Packer::at<TrsmTask>(dt, off), (int)v.size(), split, st); }),
+                    [&] { return launch_trsm<T>(Packer::at<TrsmTask>(dt, off), (int)v.size(), st); }),
               what);
 }
 
@@ -1345,7 +1338,6 @@ void Tree::launch_elimination(LevelPlan<T>& L) {
             if (t.n > POTRF_SMALL_MAX) t.dbuf = arena_.alloc(32 * 32 * sizeof(T));
         order_getrf<T>(getrfE);
         Packer pe;
-        const int sp_te = split_trsm(trsmE);
         const size_t o_pe = pe.add(potrfE), o_te = pe.add(trsmE), o_ti = pe.add(tiles), o_co = pe.add(contribs);
         const size_t o_ie = pe.add(inv_init), o_ge = pe.add(getrfE);
         void* de = upload_tasks(pe);
@@ -1361,7 +1353,7 @@ void Tree::launch_elimination(LevelPlan<T>& L) {
         }
         run_potrf<T>(st, de, potrfE, o_pe, "potrf elim");
         run_getrf<T>(st, de, getrfE, o_ge, "getrf elim");
-        run_trsm<T>(st, de, trsmE, o_te, sp_te, "trsm elim");
+        run_trsm<T>(st, de, trsmE, o_te, "trsm elim");
         if (!tiles.empty()) {
             Work w = work_schur(tiles, contribs, esz);
             hip_check(timed(prof_, KF_SCHUR, st, w.bytes, w.flops,
@@ -1867,7 +1859,6 @@ void Tree::launch_level(LevelPlan<T>& L) {
     for (PotrfTask& t : potrfS)
         if (t.n > POTRF_SMALL_MAX) t.dbuf = arena_.alloc(32 * 32 * sizeof(T));
     Packer pk;
-    const int sp_ta = split_trsm(trsmA), sp_tb = split_trsm(trsmB);
     size_t o_ps = pk.add(potrfS), o_ta = pk.add(trsmA), o_tb = pk.add(trsmB), o_sg = pk.add(segs);
     size_t o_ii = pk.add(inv_init);
     order_getrf<T>(getrfS);
@@ -1891,8 +1882,8 @@ void Tree::launch_level(LevelPlan<T>& L) {
     }
     run_potrf<T>(st, dt, potrfS, o_ps, "potrf scale");
     run_getrf<T>(st, dt, getrfS, o_gs, "getrf scale");
-    run_trsm<T>(st, dt, trsmA, o_ta, sp_ta, "trsm scale A");
-    run_trsm<T>(st, dt, trsmB, o_tb, sp_tb, "trsm scale B");
+    run_trsm<T>(st, dt, trsmA, o_ta, "trsm scale A");
+    run_trsm<T>(st, dt, trsmB, o_tb, "trsm scale B");
     // stepped-path launch slots, for the post-hoc work attribution below
     std::vector<int> slot_init(nwaves, -1), slot_finish(nwaves, -1);
     std::vector<int> slot_step(nwaves, -1);
@@ -2153,7 +2144,6 @@ void Tree::fold_orthogonal(LevelPlan<T>& L) {
         }
     }
     Packer pl;
-    const int sp = split_trsm(tz);
     const size_t o_w = pl.add(wy), o_t = pl.add(wy_tiles), o_z = pl.add(tz), o_ty = pl.add(ty), o_cy = pl.add(cy),
                  o_tw = pl.add(tw), o_cw = pl.add(cw);
     void* dl = upload_tasks(pl);
@@ -2178,7 +2168,7 @@ void Tree::fold_orthogonal(LevelPlan<T>& L) {
                   "Orthogonal into scaling");
     };
     schur(ty, cy, o_ty, o_cy);
-    run_trsm<T>(st, dl, tz, o_z, sp, "compact WY solve");
+    run_trsm<T>(st, dl, tz, o_z, "compact WY solve");
     schur(tw, cw, o_tw, o_cw);
 }
 

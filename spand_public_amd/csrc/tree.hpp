@@ -241,7 +241,7 @@ class Tree {
     template <typename T>
     void run_potrf(hipStream_t st, void* dt, const std::vector<PotrfTask>& v, size_t off, const char* what);
     template <typename T>
-    void run_trsm(hipStream_t st, void* dt, const std::vector<TrsmTask>& v, size_t off, int split, const char* what);
+    void run_trsm(hipStream_t st, void* dt, const std::vector<TrsmTask>& v, size_t off, const char* what);
     template <typename T>
     void order_getrf(std::vector<GetrfTask>& v);
     template <typename T>
