@@ -387,16 +387,34 @@ __global__ void __launch_bounds__(NT) k_spmv(int N, const int* rowptr, const int
 
 // Sampled outer product on A's pattern: for stored entry p = (i, j) (CSR position, row i),
 // out[csc_of[p]] = alpha * sum over r of u(i, r) v(j, r), the right-hand sides in
-// increasing r; u, v column-major with leading dimension ld. One thread per row.
+// increasing r; u, v column-major with leading dimension ld. OUTER_LANES lanes per row, one
+// stored entry each at a time (a row of a grid's matrix holds 5 or 7): one thread per row
+// walked them in turn, a chain of entries times right-hand sides with too few wavefronts to
+// hide it. OUTER_R right-hand sides' loads are in flight together. 300 x 300 grid, 16 right-hand
+// sides: 43.5 -> 26.8 us.
+constexpr int OUTER_LANES = 8, OUTER_R = 8;
 __global__ void __launch_bounds__(NT) k_sampled_outer(int N, const int* rowptr, const int* colidx, const int* csc_of,
                                                       const double* u, const double* v, int nrhs, int ld,
                                                       double alpha, double* out) {
-    for (int i = blockIdx.x * NT + threadIdx.x; i < N; i += gridDim.x * NT) {
-        for (int p = rowptr[i]; p < rowptr[i + 1]; p++) {
-            const int j = colidx[p];
+    const int sub = threadIdx.x % OUTER_LANES, rows = NT / OUTER_LANES;
+    for (int i = blockIdx.x * rows + threadIdx.x / OUTER_LANES; i < N; i += gridDim.x * rows) {
+        const int end = rowptr[i + 1];
+        for (int p = rowptr[i] + sub; p < end; p += OUTER_LANES) {
+            const int j = colidx[p], at = csc_of[p];
             double acc = 0.0;
-            for (int r = 0; r < nrhs; r++) acc = fma(u[i + (size_t)r * ld], v[j + (size_t)r * ld], acc);
-            out[csc_of[p]] = alpha * acc;
+            int r = 0;
+            for (; r + OUTER_R <= nrhs; r += OUTER_R) {
+                double a[OUTER_R], b[OUTER_R];
+#pragma unroll
+                for (int q = 0; q < OUTER_R; q++) {
+                    a[q] = u[i + (size_t)(r + q) * ld];
+                    b[q] = v[j + (size_t)(r + q) * ld];
+                }
+#pragma unroll
+                for (int q = 0; q < OUTER_R; q++) acc = fma(a[q], b[q], acc);
+            }
+            for (; r < nrhs; r++) acc = fma(u[i + (size_t)r * ld], v[j + (size_t)r * ld], acc);
+            out[at] = alpha * acc;
         }
     }
 }
@@ -604,7 +622,7 @@ hipError_t launch_spmv(int N, const int* rowptr, const int* colidx, const double
 hipError_t launch_sampled_outer(int N, const int* rowptr, const int* colidx, const int* csc_of, const double* u,
                                 const double* v, int nrhs, int ld, double alpha, double* out, hipStream_t st) {
     if (N == 0) return hipSuccess;
-    k_sampled_outer<<<grid_for((size_t)N), NT, 0, st>>>(N, rowptr, colidx, csc_of, u, v, nrhs, ld, alpha, out);
+    k_sampled_outer<<<grid_for((size_t)N * OUTER_LANES), NT, 0, st>>>(N, rowptr, colidx, csc_of, u, v, nrhs, ld, alpha, out);
     return hipGetLastError();
 }
 hipError_t launch_dot(int N, int nrhs, const double* a, const double* b, double* partial, double* out,
