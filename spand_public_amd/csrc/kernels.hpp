@@ -3,7 +3,9 @@
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
+#include <vector>
 
+#include "launch_plan.hpp"
 #include "tasks.hpp"
 
 namespace spand {
@@ -30,12 +32,15 @@ template <typename T>
 hipError_t launch_potrf_trail(const PotrfTask* d_tasks, int ntasks, int kb, int nmax, hipStream_t st);
 template <typename T> hipError_t launch_trsm(const TrsmTask* d_tasks, int ntasks, hipStream_t st);
 // LU pivots (GEN / PLU): launch_getrf_panels up to GETRF_PANEL_MAX rows (tasks with diag and
-// moves set, nmax the largest n), launch_getrf for larger ones.
+// moves set, sorted by n, largest first; plan: plan_getrf of their sizes), launch_getrf for
+// larger ones.
 template <typename T>
 hipError_t launch_getrf(const GetrfTask* d_tasks, int ntasks, int* d_info, hipStream_t st);
 constexpr int GETRF_PANEL_MAX = 4096;
+constexpr int GETRF_NT = 256;  // threads of a trail or split workgroup
 template <typename T>
-hipError_t launch_getrf_panels(const GetrfTask* d_tasks, int ntasks, int nmax, int* d_info, hipStream_t st);
+hipError_t launch_getrf_panels(const GetrfTask* d_tasks, const std::vector<GetrfLaunch>& plan, int* d_info,
+                               hipStream_t st);
 template <typename T>
 hipError_t launch_schur(const SchurTile* d_tiles, int ntiles, const SchurContrib* d_contribs, hipStream_t st);
 // Small clusters, one workgroup each. lds_bytes (<= RRQR_LDS_MAX) holds a task's Asn when

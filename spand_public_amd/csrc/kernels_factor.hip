@@ -2971,13 +2971,13 @@ __global__ void __launch_bounds__(1024) k_getrf_panel(const GetrfTask* tasks, in
 // per 8 products and U comes from LDS at one address per wavefront. Eight columns keep
 // n / 8 workgroups busy.
 template <typename T, int NB>
-__global__ void __launch_bounds__(NT) k_getrf_trail(const GetrfTask* tasks, int kb) {
+__global__ void __launch_bounds__(NT) k_getrf_trail(const GetrfTask* tasks, int kb, int per_task) {
 #pragma clang fp contract(off)
     constexpr int W = 8;
     __shared__ T Us[NB][W], Ls[NB][NB + 1], Ms[GETRF_NB][W];
     __shared__ int s_zero;
-    const GetrfTask t = tasks[blockIdx.y];
-    const int n = t.n, tid = threadIdx.x, c0 = blockIdx.x * W;
+    const GetrfTask t = tasks[blockIdx.x / per_task];
+    const int n = t.n, tid = threadIdx.x, c0 = blockIdx.x % per_task * W;
     if (kb >= n || c0 >= n || (c0 >= kb && c0 < kb + NB)) return;
     const int nr = n - kb, nc = min(NB, nr), w = min(W, n - c0);
     const gptr<T> P = gp(reinterpret_cast<T*>(t.A)) + kb + (size_t)kb * n;
@@ -3058,17 +3058,17 @@ __global__ void __launch_bounds__(NT) k_getrf_trail(const GetrfTask* tasks, int 
     }
 }
 
-// split_LU of k_getrf, one workgroup per 32 x 32 tile: the upper tiles leave transposed to
+// split_LU of k_getrf, one workgroup per 32 x 32 tile (per_task workgroups a pivot): the upper tiles leave transposed to
 // Ut through LDS (both sides coalesced); diag holds the pivots, since A's diagonal is
 // overwritten while other tiles still need it.
 template <typename T>
-__global__ void __launch_bounds__(NT) k_getrf_split(const GetrfTask* tasks) {
+__global__ void __launch_bounds__(NT) k_getrf_split(const GetrfTask* tasks, int per_task) {
 #pragma clang fp contract(off)
     __shared__ T tile[32][33];
-    const GetrfTask t = tasks[blockIdx.y];
-    const int n = t.n, nt = (n + 31) / 32;
-    if ((int)blockIdx.x >= nt * nt) return;
-    const int r0 = blockIdx.x % nt * 32, c0 = blockIdx.x / nt * 32;
+    const GetrfTask t = tasks[blockIdx.x / per_task];
+    const int n = t.n, nt = (n + 31) / 32, tl = blockIdx.x % per_task;
+    if (tl >= nt * nt) return;
+    const int r0 = tl % nt * 32, c0 = tl / nt * 32;
     const gptr<T> A = gp(reinterpret_cast<T*>(t.A)), Ut = gp(reinterpret_cast<T*>(t.Ut));
     const gptr<const T> diag = gp(reinterpret_cast<const T*>(t.diag));
     const int x = threadIdx.x % 32;
@@ -3121,37 +3121,29 @@ hipError_t launch_getrf(const GetrfTask* d_tasks, int ntasks, int* d_info, hipSt
     return hipGetLastError();
 }
 
-template <typename T, int NB, int RPT>
-static hipError_t getrf_panel_step(const GetrfTask* d_tasks, int ntasks, int kb, int nmax, int* d_info,
-                                   hipStream_t st) {
-    const int rows = (nmax - kb + RPT - 1) / RPT;
-    k_getrf_panel<T, NB, RPT><<<ntasks, (rows + 63) / 64 * 64, 0, st>>>(d_tasks, kb, d_info);
-    if (nmax > NB) k_getrf_trail<T, NB><<<dim3((nmax + 7) / 8, ntasks), NT, 0, st>>>(d_tasks, kb);
-    return hipGetLastError();
-}
-
 template <typename T>
-hipError_t launch_getrf_panels(const GetrfTask* d_tasks, int ntasks, int nmax, int* d_info, hipStream_t st) {
-    if (ntasks == 0 || nmax == 0) return hipSuccess;
-    if (nmax > GETRF_PANEL_MAX) return hipErrorInvalidValue;
-    for (int kb = 0; kb < nmax;) {
-        const int rows = nmax - kb;
-        hipError_t e;
-        if (rows <= 1024) {
-            e = getrf_panel_step<T, 32, 1>(d_tasks, ntasks, kb, nmax, d_info, st);
-            kb += 32;
-        } else if (rows <= 2048) {
-            e = getrf_panel_step<T, 16, 2>(d_tasks, ntasks, kb, nmax, d_info, st);
-            kb += 16;
-        } else {
-            e = getrf_panel_step<T, 8, 4>(d_tasks, ntasks, kb, nmax, d_info, st);
-            kb += 8;
-        }
+hipError_t launch_getrf_panels(const GetrfTask* d_tasks, const std::vector<GetrfLaunch>& plan, int* d_info,
+                               hipStream_t st) {
+    for (const GetrfLaunch& l : plan) {
+        const GetrfTask* d = d_tasks + l.first;
+        const long long blocks = (long long)l.count * l.per_task;
+        if (blocks > launch_blocks_max(l.threads) || l.threads > 1024) return hipErrorInvalidValue;
+        auto panel = [&](auto nb) {
+            constexpr int NB = decltype(nb)::value;
+            if (l.kind == GetrfLaunch::PANEL)
+                k_getrf_panel<T, NB, GETRF_NB / NB><<<(unsigned)blocks, l.threads, 0, st>>>(d, l.kb, d_info);
+            else
+                k_getrf_trail<T, NB><<<(unsigned)blocks, NT, 0, st>>>(d, l.kb, l.per_task);
+        };
+        if (l.kind == GetrfLaunch::SPLIT) k_getrf_split<T><<<(unsigned)blocks, NT, 0, st>>>(d, l.per_task);
+        else if (l.nb == 32) panel(std::integral_constant<int, 32>());
+        else if (l.nb == 16) panel(std::integral_constant<int, 16>());
+        else if (l.nb == 8) panel(std::integral_constant<int, 8>());
+        else return hipErrorInvalidValue;
+        const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
-    const int nt = (nmax + 31) / 32;
-    k_getrf_split<T><<<dim3(nt * nt, ntasks), NT, 0, st>>>(d_tasks);
-    return hipGetLastError();
+    return hipSuccess;
 }
 
 template <typename T>
@@ -3467,7 +3459,7 @@ hipError_t launch_copy(const CopyTask* d_tasks, int ntasks, hipStream_t st) {
     template hipError_t launch_potrf_trail<T>(const PotrfTask*, int, int, int, hipStream_t);      \
     template hipError_t launch_trsm<T>(const TrsmTask*, int, hipStream_t);                        \
     template hipError_t launch_getrf<T>(const GetrfTask*, int, int*, hipStream_t);                \
-    template hipError_t launch_getrf_panels<T>(const GetrfTask*, int, int, int*, hipStream_t);    \
+    template hipError_t launch_getrf_panels<T>(const GetrfTask*, const std::vector<GetrfLaunch>&, int*, hipStream_t); \
     template hipError_t launch_schur<T>(const SchurTile*, int, const SchurContrib*, hipStream_t); \
     template hipError_t launch_rrqr<T>(const RrqrTask*, int, const RrqrSeg*, int*, double, int, hipStream_t); \
     template hipError_t launch_rrqr_reg<T>(const RrqrTask*, int, const RrqrSeg*, int*, double, int, hipStream_t); \

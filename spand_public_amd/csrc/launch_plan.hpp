@@ -1,0 +1,25 @@
+// Launch shapes that depend on a whole batch, planned on the host without a device.
+#pragma once
+#include <vector>
+
+namespace spand {
+
+// Workgroups of NTHREADS threads that one launch may have: HIP takes fewer than 2^32 work items
+// along x (and 65,536 workgroups along y and z, which a batch of pivots exceeds: the level-0
+// scaling of a 128^3 grid has 77,949, of a 2048^2 grid 97,539).
+constexpr long long launch_blocks_max(int nthreads) { return ((1ll << 32) - 1) / nthreads; }
+
+// One launch of the LU panel kernels over tasks [first, first + count) of a batch sorted by size,
+// largest first: blocks = count x per_task workgroups of `threads` threads along x.
+struct GetrfLaunch {
+    enum Kind { PANEL, TRAIL, SPLIT };
+    int kind;
+    int kb, nb;      // panel: first column, columns (PANEL, TRAIL)
+    int first, count;
+    int per_task;    // workgroups per task
+    int threads;
+};
+// The launches that factor pivots of n[0] >= n[1] >= .. rows (n[0] <= GETRF_PANEL_MAX), in order.
+std::vector<GetrfLaunch> plan_getrf(const std::vector<int>& n);
+
+}  // namespace spand

@@ -965,10 +965,12 @@ static void small_first(std::vector<PotrfTask>& v) {
     std::stable_partition(v.begin(), v.end(), [](const PotrfTask& t) { return t.n <= POTRF_SMALL_MAX; });
     std::stable_partition(v.begin(), v.end(), [](const PotrfTask& t) { return t.n <= 64; });
 }
-// LU pivots that the panel kernels hold first, with their buffers.
+// LU pivots that the panel kernels hold first, largest first (a panel launch covers the pivots
+// that have rows left), with their buffers.
 template <typename T>
 void Tree::order_getrf(std::vector<GetrfTask>& v) {
-    std::stable_partition(v.begin(), v.end(), [](const GetrfTask& t) { return t.n <= GETRF_PANEL_MAX; });
+    auto end = std::stable_partition(v.begin(), v.end(), [](const GetrfTask& t) { return t.n <= GETRF_PANEL_MAX; });
+    std::stable_sort(v.begin(), end, [](const GetrfTask& a, const GetrfTask& b) { return a.n > b.n; });
     for (GetrfTask& t : v)
         if (t.n <= GETRF_PANEL_MAX) {
             t.diag = arena_.alloc((size_t)std::max(1, t.n) * sizeof(T));
@@ -1041,14 +1043,13 @@ template <typename T>
 void Tree::run_getrf(hipStream_t st, void* dt, const std::vector<GetrfTask>& v, size_t off, const char* what) {
     const size_t esz = sizeof(T);
     if (v.empty()) return;
-    int np = 0, nmax = 0;
+    std::vector<int> sizes;
     double pb = 0, pf = 0, gb = 0, gf = 0;
     for (auto& t : v) {
         const double n = t.n;
         const double by = (3.0 * n * n) * esz + 4.0 * n, fl = getrf_flops(n);
         if (t.n <= GETRF_PANEL_MAX) {
-            np++;
-            nmax = std::max(nmax, t.n);
+            sizes.push_back(t.n);
             pb += by;
             pf += fl;
         } else {
@@ -1057,9 +1058,10 @@ void Tree::run_getrf(hipStream_t st, void* dt, const std::vector<GetrfTask>& v, 
         }
     }
     const GetrfTask* d = Packer::at<GetrfTask>(dt, off);
+    const int np = (int)sizes.size();
     if (np > 0)
         hip_check(timed(prof_, KF_GETRF, st, pb, pf,
-                        [&] { return launch_getrf_panels<T>(d, np, nmax, d_info_, st); }),
+                        [&] { return launch_getrf_panels<T>(d, plan_getrf(sizes), d_info_, st); }),
                   what);
     if (np < (int)v.size())
         hip_check(timed(prof_, KF_GETRF, st, gb, gf,
