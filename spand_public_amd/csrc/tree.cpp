@@ -92,6 +92,12 @@ void DeviceArena::reset() {
     cur_ = 0;
     in_use_ = 0;
 }
+void DeviceArena::release(const Mark& m) {
+    if (chunk_bytes_ == 0) return;
+    for (size_t k = m.cur; k < chunks_.size(); k++) chunks_[k].used = k == m.cur ? m.used : 0;
+    cur_ = m.cur;
+    in_use_ = m.in_use;
+}
 size_t DeviceArena::bytes_reserved() const {
     size_t s = 0;
     for (auto& c : chunks_) s += c.size;
@@ -667,10 +673,10 @@ static long long env_or(const char* name, long long dflt) {
     return (e && *e) ? std::strtoll(e, nullptr, 10) : dflt;
 }
 
-// One Orthogonal op to fold into its cluster's scaling (scale: index into sv_scale).
+// One Orthogonal op to fold into its cluster's scaling: its k kept reflectors of m rows.
 struct QOp {
-    const void* Ve;
-    const void* S;
+    const void* V;
+    const void* tau;
     int m, k, cluster;
 };
 
@@ -953,8 +959,6 @@ struct LevelPlan {
     std::vector<size_t> wflag0;
     // kept ranks and merge
     std::vector<QOp> qops;
-    std::vector<WyTask> wy;
-    std::vector<int4> wy_tiles;
     std::vector<MergeTask> mt;
     std::vector<int2> mchildren;
     int left = 0;  // dofs left after the level
@@ -2043,8 +2047,6 @@ void Tree::apply_ranks(LevelPlan<T>& L) {
     auto& wreg = L.wreg;
     auto& where = L.where;
     auto& qops = L.qops;
-    auto& wy = L.wy;
-    auto& wy_tiles = L.wy_tiles;
     auto& t_lvl1 = L.t_lvl1;
     auto& t_lvl2 = L.t_lvl2;
     for (size_t p = 0; p < plist.size(); p++) {
@@ -2067,16 +2069,7 @@ void Tree::apply_ranks(LevelPlan<T>& L) {
                                                       : &wtasks[wave[p]][where[p].second];
             ops_.push_back({OP_ORTHOGONAL, c, -1, s0, 0, s0, r, ilvl_, t->Q, t->tau});
             factor_bytes_ += ((size_t)s0 * r + (size_t)r * (r + 1) / 2) * sizeof(T);
-            if (r > 0) {
-                // compact WY over all r kept reflectors, for the solve: Q = I - Ve T Ve^T
-                void* Ve = arena_.alloc((size_t)s0 * r * sizeof(T));
-                void* Sm = arena_.alloc((size_t)r * r * sizeof(T));
-                const int tw = (int)wy.size();
-                wy.push_back({t->Q, t->tau, Ve, Sm, s0, r});
-                for (int c0 = 0; c0 < r; c0 += 32)
-                    for (int a0 = 0; a0 <= c0; a0 += 32) wy_tiles.push_back(make_int4(tw, a0, c0, 0));
-                qops.push_back({Ve, Sm, s0, r, c});
-            }
+            if (r > 0) qops.push_back({t->Q, t->tau, s0, r, c});
             HCluster sib;
             sib.start = cls_[c].start + r;
             sib.size = sib.osize = s0 - r;
@@ -2107,24 +2100,47 @@ void Tree::apply_ranks(LevelPlan<T>& L) {
 // Q^T U^{-T} for PLU) over the explicit inverse, W = Linv - Ve Z with (-S) Z = -Ve^T Linv: the
 // explicit V and -S, then Y = -Ve^T Linv by the Schur kernel into a cleared block, one batched
 // triangular solve, and the update of Linv by the Schur kernel again. Zeros above the diagonal
-// of Ve and Linv clip the inner ranges of both products.
+// of Ve and Linv clip the inner ranges of both products. Ve, S and Z are given back to the arena:
+// the later users of the memory are launched behind these on the same stream. Batches of clusters
+// bound what they take.
 template <typename T>
 void Tree::fold_orthogonal(LevelPlan<T>& L) {
-    FactorRun& R = *L.run;
-    const hipStream_t st = R.st;
-    auto& wy = L.wy;
-    auto& wy_tiles = L.wy_tiles;
-    if (wy.empty()) return;
-    const size_t esz = sizeof(T);
+    constexpr size_t BATCH_BYTES = (size_t)512 << 20;
     std::vector<int> at(cls_.size(), -1);  // cluster -> its scaling task
     for (size_t k = 0; k < L.sv_scale.size(); k++) at[L.sv_scale[k].cluster] = (int)k;
+    for (size_t q0 = 0; q0 < L.qops.size();) {
+        size_t q1 = q0, bytes = 0;
+        for (; q1 < L.qops.size() && (q1 == q0 || bytes < BATCH_BYTES); q1++) {
+            const size_t m = L.qops[q1].m, k = L.qops[q1].k;
+            bytes += (3 * m * k + k * k) * sizeof(T);
+        }
+        const auto mark = arena_.mark();
+        fold_batch(L, q0, q1, at);
+        arena_.release(mark);
+        q0 = q1;
+    }
+}
+
+template <typename T>
+void Tree::fold_batch(LevelPlan<T>& L, size_t q0, size_t q1, const std::vector<int>& at) {
+    FactorRun& R = *L.run;
+    const hipStream_t st = R.st;
+    const size_t esz = sizeof(T);
+    std::vector<WyTask> wy;
+    std::vector<int4> wy_tiles;
     std::vector<SchurTile> ty, tw;
     std::vector<SchurContrib> cy, cw;
     std::vector<TrsmTask> tz;
-    for (auto& q : L.qops) {
+    for (size_t x = q0; x < q1; x++) {
+        const QOp& q = L.qops[x];
         ScaleTask& t = L.sv_scale[at[q.cluster]];
         const int m = q.m, k = q.k;
-        const char* Ve = reinterpret_cast<const char*>(q.Ve);
+        // compact WY over the k kept reflectors: Q = I - Ve T Ve^T
+        char* Ve = reinterpret_cast<char*>(arena_.alloc((size_t)m * k * esz));
+        char* S = reinterpret_cast<char*>(arena_.alloc((size_t)k * k * esz));
+        for (int c0 = 0; c0 < k; c0 += 32)
+            for (int a0 = 0; a0 <= c0; a0 += 32) wy_tiles.push_back(make_int4((int)wy.size(), a0, c0, 0));
+        wy.push_back({q.V, q.tau, Ve, S, m, k});
         t.q = true;
         for (int side = 0; side < (t.Wb == t.W ? 1 : 2); side++) {
             char* Li = reinterpret_cast<char*>(const_cast<void*>(side == 0 ? t.W : t.Wb));
@@ -2142,7 +2158,7 @@ void Tree::fold_orthogonal(LevelPlan<T>& L) {
                     tw.push_back({Li, m, r0, c0, std::min(32, m - r0), tn, 0, n0, n0 + 1});
                 }
             }
-            push_trsm(tz, q.S, Z, k, m, 0, esz, nullptr, nullptr, L.cwp);
+            push_trsm(tz, S, Z, k, m, 0, esz, nullptr, nullptr, L.cwp);
         }
     }
     Packer pl;

@@ -51,6 +51,13 @@ class DeviceArena {
     ~DeviceArena();
     void* alloc(size_t bytes);
     void reset();
+    // release(mark()) gives back what was allocated in between (not in the one-allocation-
+    // per-block mode, which keeps it until the reset)
+    struct Mark {
+        size_t cur, used, in_use;
+    };
+    Mark mark() const { return {cur_, cur_ < chunks_.size() ? chunks_[cur_].used : 0, in_use_}; }
+    void release(const Mark& m);
     size_t bytes_in_use() const { return in_use_; }
     size_t bytes_reserved() const;
 
@@ -237,6 +244,7 @@ class Tree {
     template <typename T> void apply_ranks(LevelPlan<T>& L);
     template <typename T> void merge_level(LevelPlan<T>& L);
     template <typename T> void fold_orthogonal(LevelPlan<T>& L);
+    template <typename T> void fold_batch(LevelPlan<T>& L, size_t q0, size_t q1, const std::vector<int>& at);
     template <typename T> void plan_level_solve(LevelPlan<T>& L);
     template <typename T>
     void run_potrf(hipStream_t st, void* dt, const std::vector<PotrfTask>& v, size_t off, const char* what);
