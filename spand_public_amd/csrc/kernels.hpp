@@ -100,6 +100,8 @@ template <typename T>
 hipError_t launch_rrqr_finish(const RrqrBig* d_bigs, const RrqrSlab* d_slabs, int nslabs, const RrqrSeg* d_segs,
                               int* d_size, double tol, size_t lds_bytes, hipStream_t st);
 template <typename T> hipError_t launch_copy(const CopyTask* d_tasks, int ntasks, hipStream_t st);
+// The same from blocks of type TS to blocks of type T.
+template <typename TS, typename T> hipError_t launch_convert(const CopyTask* d_tasks, int ntasks, hipStream_t st);
 
 // Preconditioner sweeps. ws holds the per-cluster segments, interleaved over nrhs.
 // Element (i, r) of the caller's block is at b[i * sx + r * sr].
@@ -126,8 +128,8 @@ struct MvTail {
 };
 template <typename T> hipError_t launch_mv(const MvDevPhase& ph, double* ws, int nrhs, hipStream_t st);
 template <typename T> hipError_t launch_mv_tail(const MvTail& tail, double* ws, int nrhs, hipStream_t st);
-// Explicit V and -S of the Orthogonal ops of one level (WyTask); tiles are the (task, a0,
-// c0) 32 x 32 tiles of the Gram matrices (a0 <= c0).
+// Explicit V and -S, FP64, of Orthogonal ops of type T (WyTask); tiles are the (task, a0, c0)
+// 32 x 32 tiles of the Gram matrices (a0 <= c0).
 template <typename T>
 hipError_t launch_wy(const WyTask* d_tasks, int ntasks, const int4* d_tiles, int ntiles, hipStream_t st);
 template <typename T>

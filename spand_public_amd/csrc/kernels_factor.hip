@@ -2810,15 +2810,15 @@ __global__ void __launch_bounds__(NT) k_rrqr_finish(const RrqrBig* bigs, const R
 }
 
 // ---------------------------------------------------------------------------------------
-template <typename T>
+template <typename TS, typename T>
 __global__ void __launch_bounds__(NT) k_copy(const CopyTask* tasks) {
     const CopyTask t = tasks[blockIdx.x];
-    const gptr<const T> S = gp(reinterpret_cast<const T*>(t.src));
+    const gptr<const TS> S = gp(reinterpret_cast<const TS*>(t.src));
     const gptr<T> D = gp(reinterpret_cast<T*>(t.dst));
     const long long n = (long long)t.rows * t.cols;
     for (long long idx = threadIdx.x; idx < n; idx += NT) {
         int i = (int)(idx % t.rows), j = (int)(idx / t.rows);
-        D[i + (size_t)j * t.ldd] = S ? S[idx] : (i == j ? T(1) : T(0));
+        D[i + (size_t)j * t.ldd] = S ? (T)S[idx] : (i == j + t.c0 ? T(1) : T(0));
     }
 }
 
@@ -3446,9 +3446,17 @@ hipError_t launch_rrqr_finish(const RrqrBig* d_bigs, const RrqrSlab* d_slabs, in
 template <typename T>
 hipError_t launch_copy(const CopyTask* d_tasks, int ntasks, hipStream_t st) {
     if (ntasks == 0) return hipSuccess;
-    k_copy<T><<<ntasks, NT, 0, st>>>(d_tasks);
+    k_copy<T, T><<<ntasks, NT, 0, st>>>(d_tasks);
     return hipGetLastError();
 }
+template <typename TS, typename T>
+hipError_t launch_convert(const CopyTask* d_tasks, int ntasks, hipStream_t st) {
+    if (ntasks == 0) return hipSuccess;
+    k_copy<TS, T><<<ntasks, NT, 0, st>>>(d_tasks);
+    return hipGetLastError();
+}
+template hipError_t launch_convert<float, double>(const CopyTask*, int, hipStream_t);
+template hipError_t launch_convert<double, float>(const CopyTask*, int, hipStream_t);
 
 #define SPAND_INST(T)                                                                              \
     template hipError_t launch_fill<T>(T*, size_t, T, hipStream_t);                               \

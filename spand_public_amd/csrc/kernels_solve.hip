@@ -302,32 +302,31 @@ template <typename T>
 __global__ void __launch_bounds__(NT) k_wy_explicit(const WyTask* tasks) {
     const WyTask t = tasks[blockIdx.x];
     const T* V = reinterpret_cast<const T*>(t.V);
-    T* Ve = reinterpret_cast<T*>(t.Ve);
+    double* Ve = t.Ve;
     const size_t n = (size_t)t.m * t.k;
     for (size_t idx = (size_t)blockIdx.y * NT + threadIdx.x; idx < n; idx += (size_t)gridDim.y * NT) {
         const int i = (int)(idx % t.m), c = (int)(idx / t.m);
-        Ve[idx] = i == c ? T(1) : (i > c ? V[idx] : T(0));
+        Ve[idx] = i == c ? 1.0 : (i > c ? (double)V[idx] : 0.0);
     }
     // S on and above the diagonal
     const T* tau = reinterpret_cast<const T*>(t.tau);
-    T* S = reinterpret_cast<T*>(t.S);
+    double* S = t.S;
     const size_t kk = (size_t)t.k * t.k;
     for (size_t idx = (size_t)blockIdx.y * NT + threadIdx.x; idx < kk; idx += (size_t)gridDim.y * NT) {
         const int a = (int)(idx % t.k), c = (int)(idx / t.k);
-        if (a <= c) S[idx] = a == c ? -(T(1) / tau[a]) : T(0);
+        if (a <= c) S[idx] = a == c ? -(1.0 / (double)tau[a]) : 0.0;
     }
 }
 
 // one workgroup per 32 x 32 tile (a0, c0), a0 <= c0, of one op's Gram matrix; entry
 // (a, c), a < c, goes to S(c, a)
-template <typename T>
 __global__ void __launch_bounds__(NT) k_wy_gram(const WyTask* tasks, const int4* tiles) {
     constexpr int GT = 32;  // tile edge (the host plans 32 x 32 tiles)
-    __shared__ T As[GT][GT + 1], Cs[GT][GT + 1];
+    __shared__ double As[GT][GT + 1], Cs[GT][GT + 1];
     const int4 tl = tiles[blockIdx.x];  // (task, a0, c0, unused)
     const WyTask t = tasks[tl.x];
     const int a0 = tl.y, c0 = tl.z, m = t.m, k = t.k;
-    const T* Ve = reinterpret_cast<const T*>(t.Ve);
+    const double* Ve = t.Ve;
     const int tid = threadIdx.x;
     // thread -> 4 outputs: a = a0 + tid % 32, c = c0 + (tid / 32) * 4 + q
     const int ta = tid % GT, tc0 = (tid / GT) * 4;
@@ -336,22 +335,22 @@ __global__ void __launch_bounds__(NT) k_wy_gram(const WyTask* tasks, const int4*
         const int ni = min(GT, m - i0);
         for (int idx = tid; idx < GT * GT; idx += NT) {
             const int ii = idx % GT, cc = idx / GT;
-            As[ii][cc] = (ii < ni && a0 + cc < k) ? Ve[(i0 + ii) + (size_t)(a0 + cc) * m] : T(0);
-            Cs[ii][cc] = (ii < ni && c0 + cc < k) ? Ve[(i0 + ii) + (size_t)(c0 + cc) * m] : T(0);
+            As[ii][cc] = (ii < ni && a0 + cc < k) ? Ve[(i0 + ii) + (size_t)(a0 + cc) * m] : 0.0;
+            Cs[ii][cc] = (ii < ni && c0 + cc < k) ? Ve[(i0 + ii) + (size_t)(c0 + cc) * m] : 0.0;
         }
         __syncthreads();
         for (int ii = 0; ii < ni; ii++) {
             const double a = As[ii][ta];
 #pragma unroll
-            for (int q = 0; q < 4; q++) acc[q] += a * (double)Cs[ii][tc0 + q];
+            for (int q = 0; q < 4; q++) acc[q] += a * Cs[ii][tc0 + q];
         }
         __syncthreads();
     }
-    T* S = reinterpret_cast<T*>(t.S);
+    double* S = t.S;
 #pragma unroll
     for (int q = 0; q < 4; q++) {
         const int a = a0 + ta, c = c0 + tc0 + q;
-        if (a < k && c < k && a < c) S[c + (size_t)a * k] = (T)-acc[q];
+        if (a < k && c < k && a < c) S[c + (size_t)a * k] = -acc[q];
     }
 }
 
@@ -603,7 +602,7 @@ hipError_t launch_wy(const WyTask* d_tasks, int ntasks, const int4* d_tiles, int
     k_wy_explicit<T><<<dim3(ntasks, 16), NT, 0, st>>>(d_tasks);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || ntiles == 0) return e;
-    k_wy_gram<T><<<ntiles, NT, 0, st>>>(d_tasks, d_tiles);
+    k_wy_gram<<<ntiles, NT, 0, st>>>(d_tasks, d_tiles);
     return hipGetLastError();
 }
 template <typename T>

@@ -121,13 +121,14 @@ struct RrqrSlab {
     int slab;  // columns [64 * slab, 64 * slab + 64)
 };
 
-// Merge copy of one child block into a parent block (update_edges, src/tree.cpp:1133-1184).
+// Merge copy of one child block into a parent block (update_edges, src/tree.cpp:1133-1184), or
+// an identity block.
 struct CopyTask {
     const void* src;  // nullptr => identity block
     void* dst;
     int rows, cols;
     int ldd;
-    int pad;
+    int c0;           // identity block: the row of its first column's one
 };
 
 // ---------------------------------------------------------------------------------------
@@ -175,8 +176,8 @@ struct MvDevPhase {
 struct WyTask {
     const void* V;    // m x k reflectors as stored by the QR (R on and above the diagonal)
     const void* tau;
-    void* Ve;         // m x k explicit V
-    void* S;          // k x k lower: -diag(1 / tau) - stril(V^T V)
+    double* Ve;       // m x k explicit V
+    double* S;        // k x k lower: -diag(1 / tau) - stril(V^T V)
     int m, k;
 };
 struct MergeTask {  // Merge (src/operations.cpp:166-192) of children without a W phase

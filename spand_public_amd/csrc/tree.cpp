@@ -519,6 +519,7 @@ struct ScaleTask {  // ScalingLLT / ScalingPLUQ and Orthogonal of one remaining 
     int cluster, n, r;      // size and kept rank
     int xoff, dst, sib;     // own segment, place in the parent's, the sibling's segment
     bool q;                 // an Orthogonal op with a nonzero rank: W and Wb are full
+    const void* F[2];       // the triangles that W and Wb invert: L and U^T
 };
 struct GemvGroup { int xdst, n, k0, k1; };
 struct GemvTerm {
@@ -1426,12 +1427,14 @@ void Tree::plan_scaling(LevelPlan<T>& L) {
             if (n > 0) {
                 void* Li = arena_.alloc((size_t)n * n * sizeof(T));
                 void* Wi = arena_.alloc((size_t)n * n * sizeof(T));
-                inv_init.push_back({nullptr, Li, n, n, n, 0});
-                inv_init.push_back({nullptr, Wi, n, n, n, 0});
-                push_trsm(trsmA, piv.A, Li, n, n, 0, sizeof(T));
-                push_trsm(trsmA, Ut, Wi, n, n, 0, sizeof(T));
+                if constexpr (sizeof(T) == 8) {  // FP32: fold_orthogonal
+                    inv_init.push_back({nullptr, Li, n, n, n, 0});
+                    inv_init.push_back({nullptr, Wi, n, n, n, 0});
+                    push_trsm(trsmA, piv.A, Li, n, n, 0, sizeof(T));
+                    push_trsm(trsmA, Ut, Wi, n, n, 0, sizeof(T));
+                }
                 lst.flops_trsm += 2.0 * n * n * n;
-                sv_scale.push_back({Li, Wi, pp, c, n, n, (int)s.xoff, -1, -1, false});
+                sv_scale.push_back({Li, Wi, pp, c, n, n, (int)s.xoff, -1, -1, false, {piv.A, Ut}});
             }
         }
         for (int c : live) {
@@ -1468,10 +1471,12 @@ void Tree::plan_scaling(LevelPlan<T>& L) {
             factor_bytes_ += (size_t)s.size * (s.size + 1) / 2 * sizeof(T);
             if (s.size > 0) {
                 void* Li = arena_.alloc((size_t)s.size * s.size * sizeof(T));
-                inv_init.push_back({nullptr, Li, s.size, s.size, s.size, 0});
-                push_trsm(trsmA, piv.A, Li, s.size, s.size, 0, sizeof(T));
+                if constexpr (sizeof(T) == 8) {  // FP32: fold_orthogonal
+                    inv_init.push_back({nullptr, Li, s.size, s.size, s.size, 0});
+                    push_trsm(trsmA, piv.A, Li, s.size, s.size, 0, sizeof(T));
+                }
                 lst.flops_trsm += (double)s.size * s.size * s.size;
-                sv_scale.push_back({Li, Li, nullptr, c, s.size, s.size, (int)s.xoff, -1, -1, false});
+                sv_scale.push_back({Li, Li, nullptr, c, s.size, s.size, (int)s.xoff, -1, -1, false, {piv.A, nullptr}});
             }
         }
         for (int c : live) {
@@ -2100,37 +2105,73 @@ void Tree::apply_ranks(LevelPlan<T>& L) {
 // Q^T U^{-T} for PLU) over the explicit inverse, W = Linv - Ve Z with (-S) Z = -Ve^T Linv: the
 // explicit V and -S, then Y = -Ve^T Linv by the Schur kernel into a cleared block, one batched
 // triangular solve, and the update of Linv by the Schur kernel again. Zeros above the diagonal
-// of Ve and Linv clip the inner ranges of both products. Ve, S and Z are given back to the arena:
-// the later users of the memory are launched behind these on the same stream. Batches of clusters
-// bound what they take.
+// of Ve and Linv clip the inner ranges of both products.
+// All of it in FP64 whatever the factor's type. An FP32 factor's L is widened, inverted and
+// folded in FP64, and W is rounded to FP32 once: its relative error against Q^T L^{-1} of the
+// stored L, V and tau is 2.5e-8 whatever the size and the condition. An FP32 L^{-1} multiplied in
+// FP64 by V and an FP32 S^{-1}, one after the other, has 5e-8 to 5e-7; the fold in FP32
+// arithmetic 1e-7 to 8e-7 (20 to 300 rows, conditions 10 and 1000).
+// The temporaries are given back to the arena: the later users of the memory are launched behind
+// these on the same stream. Batches of clusters bound what they take.
 template <typename T>
 void Tree::fold_orthogonal(LevelPlan<T>& L) {
     constexpr size_t BATCH_BYTES = (size_t)512 << 20;
+    constexpr bool WIDEN = sizeof(T) < sizeof(double);
     std::vector<int> at(cls_.size(), -1);  // cluster -> its scaling task
     for (size_t k = 0; k < L.sv_scale.size(); k++) at[L.sv_scale[k].cluster] = (int)k;
     for (size_t q0 = 0; q0 < L.qops.size();) {
         size_t q1 = q0, bytes = 0;
         for (; q1 < L.qops.size() && (q1 == q0 || bytes < BATCH_BYTES); q1++) {
-            const size_t m = L.qops[q1].m, k = L.qops[q1].k;
-            bytes += (3 * m * k + k * k) * sizeof(T);
+            const QOp& q = L.qops[q1];
+            const size_t m = q.m, k = q.k, sides = L.run->gen ? 2 : 1;
+            bytes += ((1 + sides) * m * k + k * k + (WIDEN ? 2 * sides * m * m : 0)) * sizeof(double);
         }
         const auto mark = arena_.mark();
         fold_batch(L, q0, q1, at);
         arena_.release(mark);
         q0 = q1;
     }
+    if constexpr (WIDEN) {  // the scaled clusters without an Orthogonal op: L^{-1} as it is
+        const hipStream_t st = L.run->st;
+        std::vector<CopyTask> ident;
+        std::vector<TrsmTask> inv;
+        for (const ScaleTask& t : L.sv_scale)
+            for (int side = 0; side < (t.Wb == t.W ? 1 : 2) && !t.q; side++) {
+                void* Li = const_cast<void*>(side == 0 ? t.W : t.Wb);
+                ident.push_back({nullptr, Li, t.n, t.n, t.n, 0});
+                push_trsm(inv, t.F[side], Li, t.n, t.n, 0, sizeof(T), nullptr, nullptr, L.cwp);
+            }
+        if (ident.empty()) return;
+        Packer pl;
+        const size_t o_i = pl.add(ident), o_v = pl.add(inv);
+        void* dl = upload_tasks(pl);
+        hip_check(timed(prof_, KF_COPY, st, work_copy(ident, sizeof(T)).bytes, 0,
+                        [&] { return launch_copy<T>(Packer::at<CopyTask>(dl, o_i), (int)ident.size(), st); }),
+                  "identity blocks");
+        run_trsm<T>(st, dl, inv, o_v, "trsm scale inverse");
+    }
 }
 
 template <typename T>
 void Tree::fold_batch(LevelPlan<T>& L, size_t q0, size_t q1, const std::vector<int>& at) {
+    constexpr bool WIDEN = sizeof(T) < sizeof(double);
+    constexpr size_t esz = sizeof(double);
+    constexpr int CC = 32;  // columns per conversion task
     FactorRun& R = *L.run;
     const hipStream_t st = R.st;
-    const size_t esz = sizeof(T);
     std::vector<WyTask> wy;
     std::vector<int4> wy_tiles;
     std::vector<SchurTile> ty, tw;
     std::vector<SchurContrib> cy, cw;
-    std::vector<TrsmTask> tz;
+    std::vector<TrsmTask> ti, tz;
+    std::vector<CopyTask> widen, narrow;
+    auto columns = [=](std::vector<CopyTask>& v, const void* src, size_t ssz, void* dst, size_t dsz, int m) {
+        for (int c0 = 0; c0 < m; c0 += CC) {
+            const size_t off = (size_t)c0 * m;
+            v.push_back({src ? reinterpret_cast<const char*>(src) + off * ssz : nullptr,
+                         reinterpret_cast<char*>(dst) + off * dsz, m, std::min(CC, m - c0), m, c0});
+        }
+    };
     for (size_t x = q0; x < q1; x++) {
         const QOp& q = L.qops[x];
         ScaleTask& t = L.sv_scale[at[q.cluster]];
@@ -2140,10 +2181,19 @@ void Tree::fold_batch(LevelPlan<T>& L, size_t q0, size_t q1, const std::vector<i
         char* S = reinterpret_cast<char*>(arena_.alloc((size_t)k * k * esz));
         for (int c0 = 0; c0 < k; c0 += 32)
             for (int a0 = 0; a0 <= c0; a0 += 32) wy_tiles.push_back(make_int4((int)wy.size(), a0, c0, 0));
-        wy.push_back({q.V, q.tau, Ve, S, m, k});
+        wy.push_back({q.V, q.tau, reinterpret_cast<double*>(Ve), reinterpret_cast<double*>(S), m, k});
         t.q = true;
         for (int side = 0; side < (t.Wb == t.W ? 1 : 2); side++) {
-            char* Li = reinterpret_cast<char*>(const_cast<void*>(side == 0 ? t.W : t.Wb));
+            char* W = reinterpret_cast<char*>(const_cast<void*>(side == 0 ? t.W : t.Wb));
+            char* Li = W;
+            if constexpr (WIDEN) {
+                void* F = arena_.alloc((size_t)m * m * esz);
+                Li = reinterpret_cast<char*>(arena_.alloc((size_t)m * m * esz));
+                columns(widen, t.F[side], sizeof(T), F, esz, m);
+                columns(widen, nullptr, 0, Li, esz, m);
+                push_trsm(ti, F, Li, m, m, 0, esz, nullptr, nullptr, L.cwp);
+                columns(narrow, Li, esz, W, sizeof(T), m);
+            }
             char* Z = reinterpret_cast<char*>(arena_.alloc((size_t)k * m * esz));
             for (int c0 = 0; c0 < m; c0 += 32) {
                 const int tn = std::min(32, m - c0);
@@ -2163,11 +2213,19 @@ void Tree::fold_batch(LevelPlan<T>& L, size_t q0, size_t q1, const std::vector<i
     }
     Packer pl;
     const size_t o_w = pl.add(wy), o_t = pl.add(wy_tiles), o_z = pl.add(tz), o_ty = pl.add(ty), o_cy = pl.add(cy),
-                 o_tw = pl.add(tw), o_cw = pl.add(cw);
+                 o_tw = pl.add(tw), o_cw = pl.add(cw), o_wi = pl.add(widen), o_ti = pl.add(ti), o_na = pl.add(narrow);
     void* dl = upload_tasks(pl);
+    if constexpr (WIDEN) {
+        hip_check(timed(prof_, KF_COPY, st, work_copy(widen, sizeof(T) + esz).bytes / 2, 0,
+                        [&] {
+                            return launch_convert<T, double>(Packer::at<CopyTask>(dl, o_wi), (int)widen.size(), st);
+                        }),
+                  "widen");
+        run_trsm<double>(st, dl, ti, o_ti, "trsm scale inverse");
+    }
     double lb = 0, lf = 0;
     for (auto& w : wy) {
-        lb += (3.0 * w.m * w.k + 2.0 * w.k * w.k) * sizeof(T);
+        lb += (double)w.m * w.k * (sizeof(T) + 2 * esz) + 2.0 * w.k * w.k * esz;
         lf += (double)w.m * w.k * w.k;
     }
     hip_check(timed(prof_, KF_LARFT, st, lb, lf,
@@ -2180,14 +2238,20 @@ void Tree::fold_batch(LevelPlan<T>& L, size_t q0, size_t q1, const std::vector<i
         const Work w = work_schur(t, c, esz);
         hip_check(timed(prof_, KF_LARFT, st, w.bytes, w.flops,
                         [&] {
-                            return launch_schur<T>(Packer::at<SchurTile>(dl, o1), (int)t.size(),
-                                                   Packer::at<SchurContrib>(dl, o2), st);
+                            return launch_schur<double>(Packer::at<SchurTile>(dl, o1), (int)t.size(),
+                                                        Packer::at<SchurContrib>(dl, o2), st);
                         }),
                   "Orthogonal into scaling");
     };
     schur(ty, cy, o_ty, o_cy);
-    run_trsm<T>(st, dl, tz, o_z, "compact WY solve");
+    run_trsm<double>(st, dl, tz, o_z, "compact WY solve");
     schur(tw, cw, o_tw, o_cw);
+    if constexpr (WIDEN)
+        hip_check(timed(prof_, KF_COPY, st, work_copy(narrow, sizeof(T) + esz).bytes / 2, 0,
+                        [&] {
+                            return launch_convert<double, T>(Packer::at<CopyTask>(dl, o_na), (int)narrow.size(), st);
+                        }),
+                  "narrow");
 }
 
 // Merge (src/tree.cpp:1435-1445, 1106-1184): parents, their merged edges, and the

@@ -41,3 +41,126 @@ def test_the_folds_temporaries_are_given_back(symm, prec, monkeypatch):
     assert u.factor_info()["arena_bytes"] - kept >= esz * int(((1 + sides) * m * k + k * k).sum())
     b = np.random.default_rng(1).standard_normal(16 ** 3)
     assert np.array_equal(t.solve(b), u.solve(b))
+
+
+# -- the same operator from the stored ops, in NumPy ------------------------------------
+
+
+def inverse32(L):
+    """L^{-1} by FP32 substitution, column by column of L, each multiply-add rounded once (the
+    product of two FP32 numbers is exact in FP64; the second rounding of the sum matters for one
+    entry in 2^29 or so)."""
+    n = len(L)
+    X = np.eye(n, dtype=np.float32)
+    for k in range(n):
+        X[k] = X[k] / np.float32(L[k, k])
+        X[k + 1:] = (X[k + 1:].astype(np.float64) - np.outer(L[k + 1:, k], X[k].astype(np.float64))).astype(np.float32)
+    return X.astype(np.float64)
+
+
+def reflected(V, tau, M):
+    """Q^T M for Q = H_0 H_1 .. by reflectors, FP64."""
+    M = M.copy()
+    for a in range(len(tau)):
+        v = np.r_[np.zeros(a), 1.0, V[a + 1:, a]]
+        M -= np.outer(tau[a] * v, v @ M)
+    return M
+
+
+def replay(t, b, fp32):
+    """M^{-1} b from the recorded ops. fp32: explicit inverses as an FP32 factor holds them,
+    L^{-1} by FP32 substitution and W = Q^T L^{-1} rounded once; else exact solves."""
+    ops, cl, perm = t.ops(), t.get_clusters(), t.get_assembly_perm()
+    b = np.asarray(b)[perm]
+    x, kids = {}, {}
+    first = {}
+    for order, _, _, parent, osize, size, start in cl:
+        kids.setdefault(parent, []).append(order)
+        first[order] = (start, osize)
+    for order, (start, osize) in first.items():
+        if order not in kids:
+            x[order] = b[start:start + osize].copy()
+    data = [t.op_data(i, r) if r[5] * r[6] and r[0] <= ORTHOGONAL else {} for i, r in enumerate(ops)]
+    orth = {(r[1], r[7]): i for i, r in enumerate(ops) if r[0] == ORTHOGONAL}
+    mats = []  # per scaling op (forward matrix, backward matrix)
+    for i, r in enumerate(ops):
+        mats.append(None)
+        if r[0] > 1 or not data[i]:
+            continue
+        L = np.tril(data[i]["M"])
+        U = data[i].get("U")
+        tri = [L] if U is None else [L, np.triu(U).T]
+        q = orth.get((r[1], r[7]))
+        if not fp32:
+            inv = [np.linalg.inv(F) for F in tri]
+        elif q is None or ops[q][6] == 0:
+            inv = [inverse32(F) for F in tri]
+        else:
+            inv = [np.linalg.inv(F) for F in tri]
+        if q is not None and ops[q][6] > 0:
+            inv = [reflected(data[q]["M"], data[q]["tau"], F) for F in inv]
+            if fp32:
+                inv = [F.astype(np.float32).astype(np.float64) for F in inv]
+        mats[i] = (inv[0], inv[-1])
+    for i, (typ, c, nb, sa, sb, _, _, _) in enumerate(ops):
+        A = data[i].get("M")
+        if typ <= 1 and mats[i] is not None:
+            p = data[i].get("p")
+            x[c] = mats[i][0] @ (x[c] if p is None else x[c][p])
+        elif typ in (2, 4) and A is not None:
+            x[nb] = x[nb] - A @ x[c]
+        elif typ == 3 and A is not None:
+            x[nb] = x[nb] - A.T @ x[c]
+        elif typ == 7:
+            x[c] = np.concatenate([x[k] for k in kids[c]])
+        elif typ == 8:
+            x[c], x[nb] = x[c][:sa], x[c][sa:]
+    for i in range(len(ops) - 1, -1, -1):
+        typ, c, nb, sa, sb = ops[i][:5]
+        A = data[i].get("M")
+        if typ <= 1 and mats[i] is not None:
+            x[c] = mats[i][1].T @ x[c]
+        elif typ == 2 and A is not None:
+            x[c] = x[c] - A.T @ x[nb]
+        elif typ in (3, 5) and A is not None:
+            x[c] = x[c] - A @ x[nb]
+        elif typ == 7:
+            at = 0
+            for k in kids[c]:
+                n = len(x[k])
+                x[k] = x[c][at:at + n]
+                at += n
+        elif typ == 8:
+            x[c] = np.concatenate([x[c], x[nb]])
+    y = np.empty(len(b))
+    for order, (start, osize) in first.items():
+        if order not in kids:
+            y[perm[start:start + osize]] = x[order]
+    return y
+
+
+CASES = [(12, 3, 5, 1e-2, "SPD"), (40, 2, 5, 1e-2, "SPD"), (16, 3, 5, 1e-1, "SPD"), (10, 3, 4, 1e-2, "GEN"),
+         (36, 2, 5, 1e-3, "GEN")]
+
+
+@pytest.mark.parametrize("n,d,nl,tol,symm", CASES)
+def test_fp32_apply_rounds_the_folded_matrix_once(n, d, nl, tol, symm):
+    """An FP32 factor's apply against the stored ops: FP64 arithmetic on matrices that are rounded
+    once. Where the two round an entry of W apart (FP64 errors of about 1e-14 relative next to a
+    tie, one entry in 10^6 or so) they differ by 6e-8 there, so 1e-8 of the whole leaves an
+    order of magnitude; a fold in FP32 arithmetic is 1e-7 and more off."""
+    print(f"case fold fp32 {symm} {d}D n={n} tol={tol}", flush=True)
+    A, t = factor(n, d, nl, tol, S.FP32, symm)
+    assert (t.ops()[:, 0] == ORTHOGONAL).sum() > 5
+    b = np.random.default_rng(2).standard_normal(A.n)
+    x, y = t.solve(b), replay(t, b, True)
+    assert np.linalg.norm(x - y) <= 1e-8 * np.linalg.norm(y)
+
+
+@pytest.mark.parametrize("n,d,nl,tol,symm", CASES)
+def test_fp64_apply_is_the_stored_ops(n, d, nl, tol, symm):
+    print(f"case fold fp64 {symm} {d}D n={n} tol={tol}", flush=True)
+    A, t = factor(n, d, nl, tol, S.FP64, symm)
+    b = np.random.default_rng(3).standard_normal(A.n)
+    x, y = t.solve(b), replay(t, b, False)
+    assert np.linalg.norm(x - y) <= 1e-12 * np.linalg.norm(y)
