@@ -963,6 +963,7 @@ struct LevelPlan {
     std::vector<MergeTask> mt;
     std::vector<int2> mchildren;
     int left = 0;  // dofs left after the level
+    DeviceArena::Mark temps{};  // where the working storage of launch_level begins
 };
 
 // Cholesky batch order: <= 64, <= POTRF_SMALL_MAX, larger
@@ -1714,11 +1715,6 @@ void Tree::plan_sparsification(LevelPlan<T>& L) {
                 // stepped multi-workgroup path
                 RrqrBig b{};
                 b.nslab = std::max(1, (cols + 63) / 64);
-                t.scratch = arena_.alloc((size_t)s.size * b.nslab * 64 * sizeof(T));
-                t.norms = reinterpret_cast<double*>(arena_.alloc((size_t)2 * std::max(cols, 1) * sizeof(double)));
-                b.map = reinterpret_cast<int*>(arena_.alloc((size_t)4 * std::max(cols, 1) * sizeof(int)));
-                b.cand_v = reinterpret_cast<double*>(arena_.alloc((size_t)(2 * b.nslab + 1) * sizeof(double)));
-                b.cand_p = reinterpret_cast<int*>(arena_.alloc((size_t)2 * b.nslab * sizeof(int)));
                 b.t = t;
                 where[p] = {1, (int)wbig[w].size()};
                 for (int k = 0; k < b.nslab; k++) wslab[w].push_back({(int)wbig[w].size(), k});
@@ -1726,16 +1722,6 @@ void Tree::plan_sparsification(LevelPlan<T>& L) {
                 wsteps[w] = std::max(wsteps[w], mn);
                 wmaxrows[w] = std::max(wmaxrows[w], s.size);
             } else {
-                // LDS-resident with an odd column stride (rows | 1), else a global scratch
-                if ((long long)(s.size | 1) * cols > lds_elems)
-                    t.scratch = arena_.alloc((size_t)s.size * cols * sizeof(T));
-                else
-                    wlds_small[w] =
-                        std::max(wlds_small[w], (long long)(s.size | 1) * cols * (long long)sizeof(T));
-                if (cols > 1024) {
-                    t.norms = reinterpret_cast<double*>(arena_.alloc((size_t)2 * cols * sizeof(double)));
-                    t.jpvt = reinterpret_cast<int*>(arena_.alloc((size_t)cols * sizeof(int)));
-                }
                 where[p] = {0, (int)wtasks[w].size()};
                 wtasks[w].push_back(t);
             }
@@ -1747,6 +1733,51 @@ void Tree::plan_sparsification(LevelPlan<T>& L) {
                 where[vp.second] = {2, (int)wreg[w].size()};
                 wreg[w].push_back(ptask[vp.second]);
                 wregvar[w].push_back(vp.first);
+            }
+        }
+    }
+    // dims (one block per level) and done flags of the stepped clusters; the flags are
+    // reset before any of this level's launches
+    wflag0.assign(nwaves, 0);
+    {
+        size_t nbig = 0;
+        for (int w = 0; w < nwaves; w++) nbig += wbig[w].size();
+        int* dblock = nullptr;
+        if (nbig > 0) {
+            signal_reserve(1 + nbig);
+            dblock = reinterpret_cast<int*>(arena_.alloc(nbig * 5 * sizeof(int)));
+            size_t f = 1;
+            for (int w = 0; w < nwaves; w++) {
+                wflag0[w] = f;
+                for (auto& b : wbig[w]) {
+                    h_sig_[f] = 0;
+                    b.done = d_sig_ + f;
+                    b.dims = dblock + 5 * (f - 1);
+                    f++;
+                }
+            }
+        }
+        level_dims_.push_back({dblock, nbig});
+    }
+    // Working storage of the level's launches from here on: launch_level gives it back.
+    L.temps = arena_.mark();
+    for (int w = 0; w < nwaves; w++) {
+        for (auto& b : wbig[w]) {
+            const size_t rows = b.t.max_rows, cols = std::max(b.t.max_cols, 1);
+            b.t.scratch = arena_.alloc(rows * b.nslab * 64 * sizeof(T));
+            b.t.norms = reinterpret_cast<double*>(arena_.alloc(2 * cols * sizeof(double)));
+            b.map = reinterpret_cast<int*>(arena_.alloc(4 * cols * sizeof(int)));
+            b.cand_v = reinterpret_cast<double*>(arena_.alloc((size_t)(2 * b.nslab + 1) * sizeof(double)));
+            b.cand_p = reinterpret_cast<int*>(arena_.alloc((size_t)2 * b.nslab * sizeof(int)));
+        }
+        for (auto& t : wtasks[w]) {
+            // LDS-resident with an odd column stride (rows | 1), else a global scratch
+            const long long elems = (long long)(t.max_rows | 1) * t.max_cols;
+            if (elems > lds_elems) t.scratch = arena_.alloc((size_t)t.max_rows * t.max_cols * sizeof(T));
+            else wlds_small[w] = std::max(wlds_small[w], elems * (long long)sizeof(T));
+            if (t.max_cols > 1024) {
+                t.norms = reinterpret_cast<double*>(arena_.alloc((size_t)2 * t.max_cols * sizeof(double)));
+                t.jpvt = reinterpret_cast<int*>(arena_.alloc((size_t)t.max_cols * sizeof(int)));
             }
         }
     }
@@ -1804,29 +1835,6 @@ void Tree::plan_sparsification(LevelPlan<T>& L) {
             for (auto& b : wbig[w])
                 b.vbuf = arena_.alloc((size_t)b.nslab * 2 * std::max(b.t.max_rows, 1) * sizeof(T));
         }
-    }
-    // dims (one block per level) and done flags of the stepped clusters; the flags are
-    // reset before any of this level's launches
-    wflag0.assign(nwaves, 0);
-    {
-        size_t nbig = 0;
-        for (int w = 0; w < nwaves; w++) nbig += wbig[w].size();
-        int* dblock = nullptr;
-        if (nbig > 0) {
-            signal_reserve(1 + nbig);
-            dblock = reinterpret_cast<int*>(arena_.alloc(nbig * 5 * sizeof(int)));
-            size_t f = 1;
-            for (int w = 0; w < nwaves; w++) {
-                wflag0[w] = f;
-                for (auto& b : wbig[w]) {
-                    h_sig_[f] = 0;
-                    b.done = d_sig_ + f;
-                    b.dims = dblock + 5 * (f - 1);
-                    f++;
-                }
-            }
-        }
-        level_dims_.push_back({dblock, nbig});
     }
     lst.nwaves = nwaves;
 }
@@ -2032,6 +2040,7 @@ void Tree::launch_level(LevelPlan<T>& L) {
             if (!wbig[w].empty())
                 wave_work_.push_back({slot_init[w], slot_finish[w], slot_step[w], wsteps[w], wflag0[w] - 1,
                                       wbig[w].size(), ilvl_});
+    arena_.release(L.temps);  // the copies above waited for the level's launches
     L.t_lvl1 = wall();
     lst.t_plan = t_plan1 - t_lvl0;
     lst.t_elim_scale = t_lvl1 - t_plan1;

@@ -43,6 +43,24 @@ def test_the_folds_temporaries_are_given_back(symm, prec, monkeypatch):
     assert np.array_equal(t.solve(b), u.solve(b))
 
 
+@pytest.mark.parametrize("prec", [S.FP64, S.FP32])
+def test_the_rank_decisions_working_storage_is_given_back(prec, monkeypatch):
+    """The same with every RRQR on the slab path: at least 64 columns of m rows per op besides."""
+    print(f"case rrqr memory prec={prec}", flush=True)
+    for k in ("REG", "STEPPED_MIN_ROWS", "STEPPED_MIN_ELEMS"):
+        monkeypatch.setenv(f"SPAND_RRQR_{k}", "0")
+    _, t = factor(16, 3, 6, 1e-2, prec, "SPD")
+    ops = t.ops()
+    m, k = (ops[ops[:, 0] == ORTHOGONAL][:, c].astype(np.int64) for c in (5, 6))
+    kept = t.factor_info()["arena_bytes"]
+    monkeypatch.setenv("SPAND_ARENA_CHUNK_BYTES", "0")
+    _, u = factor(16, 3, 6, 1e-2, prec, "SPD")
+    esz = 8 if prec == S.FP64 else 4
+    assert u.factor_info()["arena_bytes"] - kept >= esz * int((2 * m * k + k * k + 64 * m).sum())
+    b = np.random.default_rng(1).standard_normal(16 ** 3)
+    assert np.array_equal(t.solve(b), u.solve(b))
+
+
 # -- the same operator from the stored ops, in NumPy ------------------------------------
 
 
