@@ -65,15 +65,16 @@ constexpr int STEP_LDS_MAX = 40960;
 template <typename T>
 hipError_t launch_rrqr_init(const RrqrBig* d_bigs, const RrqrSlab* d_slabs, int nslabs, const RrqrSeg* d_segs,
                             const int* d_size, double tol, hipStream_t st);
-// All steps of a set of whole clusters in one cooperative launch (RrqrBig::vbuf holding
-// rrqr_relay_bytes of relay words, relay = 1), one wavefront per slab of rrqr_wave_cols
+// All steps of a set of whole clusters in one launch (RrqrBig::vbuf holding rrqr_relay_bytes of
+// relay words, relay = 1), one wavefront per slab of rrqr_wave_cols
 // columns (0: clusters of max_rows rows do not fit its registers; dense: the form with more
 // rows per lane and fewer slabs); positions and columns of a
 // cluster stay below WAVE_COLS_MAX. d_slabs: the slabs by workgroup, big = -1 for a place
 // without one. The slabs of each cluster exchange their candidates through the relay words
 // (waits of at most spin_max polls, RRQR_SPIN_MAX by default: *fail is set to 1 if one gives
-// up). Returns hipErrorCooperativeLaunchTooLarge, launching nothing, when the slabs do not fit
-// the device at once; rrqr_wave_capacity gives how many do.
+// up); waits: some cluster has several slabs, and the launch is cooperative. Returns
+// hipErrorCooperativeLaunchTooLarge, launching nothing, when the slabs do not fit the device at
+// once; rrqr_wave_capacity gives how many do.
 constexpr int WAVE_COLS_MAX = 1 << 15;
 constexpr long long RRQR_SPIN_MAX = 1ll << 21;
 // with room for the rows that a wavefront reads past a cluster's last one
@@ -82,8 +83,8 @@ inline size_t rrqr_relay_bytes(size_t esz, int nsub, int max_rows) {
 }
 template <typename T> int rrqr_wave_cols(int max_rows, bool dense);
 template <typename T>
-hipError_t launch_rrqr_wave(const RrqrBig* d_bigs, const RrqrSlab* d_slabs, int nslabs, int nsteps, int max_rows,
-                            bool dense, double tol, int* fail, long long spin_max, hipStream_t st);
+hipError_t launch_rrqr_wave(const RrqrBig* d_bigs, const RrqrSlab* d_slabs, int nslabs, bool waits, int nsteps,
+                            int max_rows, bool dense, double tol, int* fail, long long spin_max, hipStream_t st);
 template <typename T>
 hipError_t rrqr_wave_capacity(int max_rows, bool dense, int* cap);
 // One pivot step per launch. waves: wavefronts per slab workgroup (4, 8 or 16; 0 picks by

@@ -1698,9 +1698,9 @@ __device__ inline void relay_put_val(GRelayWord* p, unsigned tag, T x, bool loca
     }
 }
 // One failed poll of a bounded wait: true if the wait gives up, after spin_max polls
-// (RRQR_SPIN_MAX unless the caller lowers it) or once *fail is set: the launch is cooperative,
-// so every slab is resident and a correct schedule never comes near the bound; the host turns
-// the flag into an error.
+// (RRQR_SPIN_MAX unless the caller lowers it) or once *fail is set: slabs that wait for each
+// other are launched cooperatively, so every one is resident and a correct schedule never comes
+// near the bound; the host turns the flag into an error.
 __device__ inline bool relay_give_up(long long spins, int* fail, long long spin_max) {
     if (spins >= spin_max ||
         ((spins & 63) == 63 && __hip_atomic_load(fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
@@ -2134,7 +2134,7 @@ __global__ void __launch_bounds__(SLAB * NW) k_rrqr_step(const RrqrBig* bigs, co
     }
 }
 
-// Persistent form of the stepped RRQR: one cooperative launch runs every pivot step of the
+// Persistent form of the stepped RRQR: one launch runs every pivot step of the
 // clusters of a dependency wave (or of the part of it that the device holds at once), and
 // each cluster's slabs pace each other only. A slab is one wavefront, alone in its
 // workgroup: L lanes hold a column (64 / L columns a slab), lane h of a column the rows
@@ -3339,16 +3339,16 @@ static hipError_t wave_capacity_rw(int* cap) {
 }
 
 template <typename T, int L, int RW>
-static hipError_t launch_wave_rw(const RrqrBig* d_bigs, const RrqrSlab* d_slabs, int nslabs, int nsteps, double tol,
-                                 int* fail, long long spin_max, hipStream_t st) {
+static hipError_t launch_wave_rw(const RrqrBig* d_bigs, const RrqrSlab* d_slabs, int nslabs, bool waits, int nsteps,
+                                 double tol, int* fail, long long spin_max, hipStream_t st) {
     int cap = 0;
     hipError_t e = wave_capacity_rw<T, L, RW>(&cap);
     if (e != hipSuccess) return e;
     if (cap < nslabs) return hipErrorCooperativeLaunchTooLarge;
-    // A cooperative launch goes through a queue of its own (about 12 us before and after it).
-    // Up to a quarter of what the device holds is launched plainly: launches of one process are
-    // ordered on the null stream, and even those of several processes fit together.
-    if (nslabs <= cap / 4) {
+    // Slabs that wait for each other have to be resident together whatever else the device runs,
+    // other processes' launches included, so their launch is cooperative. It goes through a queue
+    // of its own, about 12 us before and after it; a launch in which nobody waits is a plain one.
+    if (!waits) {
         k_rrqr_wave<T, L, RW><<<nslabs, 64, 0, st>>>(d_bigs, d_slabs, nsteps, tol, fail, spin_max);
         return hipGetLastError();
     }
@@ -3423,14 +3423,14 @@ hipError_t rrqr_wave_capacity(int max_rows, bool dense, int* cap) {
 // Persistent launch over nslabs slabs (whole clusters): returns hipErrorCooperativeLaunchTooLarge
 // (and launches nothing) when they cannot all be resident at once.
 template <typename T>
-hipError_t launch_rrqr_wave(const RrqrBig* d_bigs, const RrqrSlab* d_slabs, int nslabs, int nsteps, int max_rows,
-                            bool dense, double tol, int* fail, long long spin_max, hipStream_t st) {
+hipError_t launch_rrqr_wave(const RrqrBig* d_bigs, const RrqrSlab* d_slabs, int nslabs, bool waits, int nsteps,
+                            int max_rows, bool dense, double tol, int* fail, long long spin_max, hipStream_t st) {
     if (nslabs == 0 || nsteps == 0) return hipSuccess;
     if (spin_max < 1) return hipErrorInvalidValue;
     hipError_t e = hipErrorCooperativeLaunchTooLarge;
     wave_variant<T>(max_rows, dense, [&](auto l, auto rw) {
-        e = launch_wave_rw<T, decltype(l)::value, decltype(rw)::value>(d_bigs, d_slabs, nslabs, nsteps, tol, fail,
-                                                                       spin_max, st);
+        e = launch_wave_rw<T, decltype(l)::value, decltype(rw)::value>(d_bigs, d_slabs, nslabs, waits, nsteps, tol,
+                                                                       fail, spin_max, st);
     });
     return e;
 }
@@ -3474,7 +3474,7 @@ template hipError_t launch_convert<double, float>(const CopyTask*, int, hipStrea
     template hipError_t launch_copy<T>(const CopyTask*, int, hipStream_t);                        \
     template hipError_t launch_rrqr_init<T>(const RrqrBig*, const RrqrSlab*, int, const RrqrSeg*, const int*,      \
                                             double, hipStream_t);                                                  \
-    template hipError_t launch_rrqr_wave<T>(const RrqrBig*, const RrqrSlab*, int, int, int, bool, double, int*,   \
+    template hipError_t launch_rrqr_wave<T>(const RrqrBig*, const RrqrSlab*, int, bool, int, int, bool, double, int*, \
                                             long long, hipStream_t);                                               \
     template hipError_t rrqr_wave_capacity<T>(int, bool, int*);                                                    \
     template int rrqr_wave_cols<T>(int, bool);                                                                     \

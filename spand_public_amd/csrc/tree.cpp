@@ -954,7 +954,7 @@ struct LevelPlan {
     std::vector<RrqrSeg> segs;
     std::vector<size_t> wlds_step;
     std::vector<std::vector<RrqrSlab>> wplace;   // persistent launches: slabs by workgroup
-    std::vector<std::vector<std::array<int, 3>>> wchunk;  // their (first workgroup, workgroups, steps)
+    std::vector<std::vector<SlabChunk>> wchunk;  // their launches
     std::vector<char> wdense;                    // and form
     int step_waves = 0;
     std::vector<size_t> wflag0;
@@ -1501,66 +1501,6 @@ void Tree::plan_scaling(LevelPlan<T>& L) {
     }
 }
 
-// Workgroups of the persistent launches of one wave: whole clusters in chunks that the device
-// holds at once (at most cap slabs), one launch each. Block b of a launch runs on XCD b % 8, so
-// a cluster's slabs go to places of one residue, largest clusters first onto the emptiest XCD:
-// its slabs then exchange their candidates through that XCD's L2 (the kernel checks where they
-// run). A cluster that no XCD holds alone spreads over the device, in a chunk of its kind. No
-// chunk at all if some cluster exceeds cap.
-struct SlabPlan {
-    std::vector<RrqrSlab> place;
-    std::vector<std::array<int, 3>> chunk;  // first workgroup, workgroups, steps
-    int spread = 0;                         // chunks whose clusters spread over the XCDs
-};
-static SlabPlan place_slabs(const std::vector<RrqrBig>& big, int cap) {
-    constexpr int XCDS = 8;
-    const int each = cap / XCDS;
-    SlabPlan P;
-    std::vector<int> order(big.size());
-    std::iota(order.begin(), order.end(), 0);
-    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return big[a].nsub > big[b].nsub; });
-    if (order.empty() || big[order[0]].nsub > cap) return P;
-    auto steps_of = [&](int x) { return std::min(big[x].t.max_rows, big[x].t.max_cols); };
-    size_t x0 = 0;
-    while (x0 < order.size() && big[order[x0]].nsub > each) {  // too long for one XCD
-        const int first = (int)P.place.size();
-        int steps = 0;
-        while (x0 < order.size() && big[order[x0]].nsub > each &&
-               (int)P.place.size() - first + big[order[x0]].nsub <= cap) {
-            for (int k = 0; k < big[order[x0]].nsub; k++) P.place.push_back({order[x0], k});
-            steps = std::max(steps, steps_of(order[x0++]));
-        }
-        P.chunk.push_back({first, (int)P.place.size() - first, steps});
-        P.spread++;
-    }
-    std::vector<int> rest(order.begin() + x0, order.end()), later;
-    while (!rest.empty()) {
-        std::vector<RrqrSlab> on[XCDS];
-        int steps = 0;
-        size_t most = 0;
-        later.clear();
-        for (int x : rest) {
-            auto* q = &on[0];
-            for (auto& o : on)
-                if (o.size() < q->size()) q = &o;
-            if ((int)q->size() + big[x].nsub > each) {
-                later.push_back(x);
-                continue;
-            }
-            for (int k = 0; k < big[x].nsub; k++) q->push_back({x, k});
-            most = std::max(most, q->size());
-            steps = std::max(steps, steps_of(x));
-        }
-        const int first = (int)P.place.size();
-        P.place.resize(first + most * XCDS, {-1, 0});
-        for (int o = 0; o < XCDS; o++)
-            for (size_t k = 0; k < on[o].size(); k++) P.place[first + k * XCDS + o] = on[o][k];
-        P.chunk.push_back({first, (int)(most * XCDS), steps});
-        rest.swap(later);
-    }
-    return P;
-}
-
 // Sparsification plan (src/tree.cpp:1521-1533, 1292-1347): dependency waves, the RRQR
 // path of each cluster (register, one-workgroup LDS or stepped slabs) and its buffers.
 template <typename T>
@@ -1653,11 +1593,14 @@ void Tree::plan_sparsification(LevelPlan<T>& L) {
         const bool reg_path = tune.rrqr_reg != 0;
         const long long big_min_elems = tune.small_elems;
         widx.assign(plist.size(), 0);
-        // Dependency waves that one persistent launch can hold run all their clusters there (64^3
-        // Laplacian, FP32: 29.6 ms a factorization for every RRQR launch, against 37.9 ms with the
-        // shorter clusters in one workgroup each), unless they are all tiny (10 x 40 on a 512^2
-        // grid: 2.3 ms in one workgroup each, 3.1 ms there). The others, and every wave when a
-        // path is asked for through the environment, split by cluster size.
+        // Dependency waves that one persistent launch can hold run all their clusters there, unless
+        // the largest has at most TINY_ELEMS Asn elements: its few steps do not pay for the
+        // cooperative launch and the init and finish launches around it. The others, and every wave
+        // when a path is asked for through the environment, split by cluster size. ms a
+        // factorization with the limit at 0 / 2000 / 4000 / 10000 / 30000 elements: 15^3 FP64 3.19 /
+        // 3.14 / 3.14 / 3.65 / 3.65, 24^3 FP32 8.13 / 8.12 / 8.10 / 8.58 / 9.76, 24^3 PLU 11.63 /
+        // 11.63 / 11.62 / 11.79 / 14.03, 512^2 FP64 13.14 / 12.24 / 12.13 / 12.14 / 12.16; 64^3
+        // within 1%.
         constexpr long long TINY_ELEMS = 2000;
         std::vector<char> all_wave(nwaves, 0);
         if (tune.source == 0 && env_or("SPAND_RRQR_PERSISTENT", 1) != 0) {
@@ -1799,15 +1742,19 @@ void Tree::plan_sparsification(LevelPlan<T>& L) {
     // the fine form unless the dense one takes fewer launches, spread ones counted twice (their
     // exchanges pass the L2s: 3-4 us a step more with the device full)
     auto plan_wave = [&](std::vector<RrqrBig>& big, int max_rows, std::vector<RrqrSlab>& place,
-                         std::vector<std::array<int, 3>>& chunk, char& form) {
+                         std::vector<SlabChunk>& chunk, char& form) {
         size_t cost = 0;
         for (bool dense : {false, true}) {
             const int sc = rrqr_wave_cols<T>(max_rows, dense);
             int cap = 0;
             hip_check(rrqr_wave_capacity<T>(max_rows, dense, &cap), "rrqr wave capacity");
             std::vector<RrqrBig> b = big;
-            for (auto& x : b) x.nsub = std::max(1, (x.t.max_cols + sc - 1) / sc);
-            SlabPlan P = place_slabs(b, cap);
+            std::vector<int> nsub, steps;
+            for (auto& x : b) {
+                nsub.push_back(x.nsub = std::max(1, (x.t.max_cols + sc - 1) / sc));
+                steps.push_back(std::min(x.t.max_rows, x.t.max_cols));
+            }
+            SlabPlan P = place_slabs(nsub, steps, cap);
             const size_t c = P.chunk.size() + P.spread;
             if (c == 0 || (cost > 0 && c >= cost)) continue;
             cost = c;
@@ -1982,9 +1929,9 @@ void Tree::launch_level(LevelPlan<T>& L) {
         if (!L.wchunk[w].empty()) {
             const int sl = prof_.start(KF_RRQR_WAVE, st);
             for (auto& c : L.wchunk[w])
-                hip_check(launch_rrqr_wave<T>(db, Packer::at<RrqrSlab>(dt, o_p[w]) + c[0], c[1], c[2], wmaxrows[w],
-                                              L.wdense[w] != 0, tol_,
-                                              d_info_ + 1, R.spin_max, st),
+                hip_check(launch_rrqr_wave<T>(db, Packer::at<RrqrSlab>(dt, o_p[w]) + c.first, c.count, c.waits,
+                                              c.steps, wmaxrows[w], L.wdense[w] != 0, tol_, d_info_ + 1, R.spin_max,
+                                              st),
                           "rrqr wave");
             prof_.stop(sl, st, 0, 0, (int)L.wchunk[w].size());
             done = true;

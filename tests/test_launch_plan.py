@@ -61,3 +61,50 @@ def test_lu_launches_fit_the_device_and_cover_every_pivot(kind):
     for row in plan[plan[:, 0] == PANEL]:
         panels[row[3]:row[3] + row[4]] += 1
     assert (trailed == panels).all()
+
+
+def plan_slabs(nsub, steps, cap):
+    L = _lib.lib()
+    nsub, steps = (np.ascontiguousarray(v, dtype=np.int32) for v in (nsub, steps))
+    chunks, place = np.zeros((4096, 4), np.int32), np.zeros((1 << 18, 2), np.int32)
+    np_ = C.c_int()
+    p = lambda a: a.ctypes.data_as(C.c_void_p)
+    k = L.spand_plan_slabs(p(nsub), p(steps), C.c_int(len(nsub)), C.c_int(cap), p(chunks), C.c_int(len(chunks)),
+                           p(place), C.c_int(len(place)), C.byref(np_))
+    assert k <= len(chunks) and np_.value <= len(place)
+    return chunks[:k].tolist(), place[:np_.value]
+
+
+@pytest.mark.parametrize("cap", [8, 20, 64, 1000, 2048])
+@pytest.mark.parametrize("kind", ["single", "mixed", "ordinary", "long"])
+def test_persistent_rrqr_slabs_are_placed_once_and_waiting_ones_launched_together(kind, cap):
+    """Each cluster whole in one launch of at most cap workgroups, on one XCD (workgroup modulo 8)
+    unless none holds it. A launch in which a cluster has several slabs is one whose workgroups
+    wait for each other: it has to be marked, because only a cooperative launch has them all
+    resident."""
+    rng = np.random.default_rng(cap)
+    nsub = {"single": np.ones(300, int), "mixed": rng.choice([1, 1, 1, 2], 200), "ordinary": rng.integers(1, 9, 500),
+            "long": rng.integers(1, max(2, cap + 1), 40)}[kind]
+    steps = rng.integers(0, 300, len(nsub))
+    chunks, place = plan_slabs(nsub, steps, cap)
+    if nsub.max() > cap:
+        assert not chunks
+        return
+    seen, at = [], 0
+    for first, count, nsteps, waits in chunks:
+        assert first == at and 0 < count <= cap
+        at += count
+        rows = place[first:first + count]
+        used = np.flatnonzero(rows[:, 0] >= 0)
+        here = np.unique(rows[used, 0])
+        for c in here:
+            mine = used[rows[used, 0] == c]
+            assert sorted(rows[mine, 1]) == list(range(nsub[c]))  # the whole cluster, each slab once
+            assert nsub[c] > cap // 8 or len(set(mine % 8)) == 1
+        assert nsteps == steps[here].max() and bool(waits) == bool((nsub[here] > 1).any())
+        seen += list(here)
+    assert at == len(place) and sorted(seen) == list(range(len(nsub)))
+
+
+def test_a_cluster_longer_than_the_device_is_not_planned():
+    assert plan_slabs([3, 65, 2], [1, 1, 1], 64)[0] == []
