@@ -1841,8 +1841,10 @@ __global__ void __launch_bounds__(STEP_NT) k_rrqr_init(const RrqrBig* bigs, cons
             B.t.norms[mc + j] = nrm;
             B.map[j] = j;
             B.map[2 * mc + j] = j;
-            best = nrm;
-            bpos = j;
+            if (nrm >= 0.0) {  // a NaN norm is no candidate, here and in the steps
+                best = nrm;
+                bpos = j;
+            }
         }
         wave_best(best, bpos);
         if (lane == 0) {
@@ -1936,7 +1938,13 @@ __global__ void __launch_bounds__(SLAB * NW) k_rrqr_step(const RrqrBig* bigs, co
     }
     __syncthreads();
     const int p = s_p, ca = s_ca, cb = s_cb;
-    if (p < i || p >= cols) return;  // cannot happen for i < mn: some column is still free
+    if (p < i || p >= cols) {  // only NaN columns are left: the QR ends here
+        if (sl.slab == 0 && tid == 0) {
+            dims[3] = i;
+            signal_store(B.done, 1);
+        }
+        return;
+    }
     if (sl.slab == 0) {
         for (int jj = tid; jj < cols; jj += NTH) {
             p2c_nxt[jj] = p2c_cur[jj];
@@ -2123,8 +2131,10 @@ __global__ void __launch_bounds__(SLAB * NW) k_rrqr_step(const RrqrBig* bigs, co
                     vn1[j] = vn1[j] * sqrt(temp);
                 }
             }
-            best = vn1[j];
-            bpos = pos;
+            if (vn1[j] >= 0.0) {
+                best = vn1[j];
+                bpos = pos;
+            }
         }
         wave_best(best, bpos);
         if (lane == 0) {
@@ -2382,7 +2392,7 @@ __global__ void __launch_bounds__(64, (wave_occupancy<T, L, RW>()))
     auto pick = [&](int i) {  // the slab's first maximum among the columns at positions >= i
         best = -1.0;
         key = INT32_MAX;
-        if (jin && pos >= i) {
+        if (jin && pos >= i && vn1 >= 0.0) {  // a NaN norm is no candidate
             best = vn1;
             key = pos << 16 | j;
         }
@@ -2500,7 +2510,7 @@ __global__ void __launch_bounds__(64, (wave_occupancy<T, L, RW>()))
             }
         }
         const int p = key >> 16, ca = key & 0xffff;
-        if (key == INT32_MAX || p < i || p >= cols) {  // cannot happen for i < mn: some column is still free
+        if (key == INT32_MAX || p < i || p >= cols) {  // only NaN columns are left
             stop = i;
             break;
         }
