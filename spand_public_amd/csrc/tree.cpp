@@ -1530,6 +1530,13 @@ void Tree::plan_sparsification(LevelPlan<T>& L) {
     auto& wlds_step = L.wlds_step;
     auto& step_waves = L.step_waves;
     auto& wflag0 = L.wflag0;
+    // SPAND_RRQR_SLABS: at most so many slabs a persistent launch; SPAND_RRQR_DENSE: 0 or 1 fixes its form
+    const long long cap_env = env_or("SPAND_RRQR_SLABS", INT32_MAX), form_env = env_or("SPAND_RRQR_DENSE", -1);
+    auto wave_cap = [&](int max_rows, bool dense) {
+        int cap = 0;
+        hip_check(rrqr_wave_capacity<T>(max_rows, dense, &cap), "rrqr wave capacity");
+        return (int)std::min<long long>(cap, cap_env);
+    };
     if (do_sparsify_level) {
         std::vector<int> inP(cls_.size(), -1);
         for (int c : live) {
@@ -1616,12 +1623,9 @@ void Tree::plan_sparsification(LevelPlan<T>& L) {
                 const int w = wave[p], sc = rrqr_wave_cols<T>(mr[w], true);
                 if (sc > 0) slabs[w] += std::max(1, (pcols[p] + sc - 1) / sc);
             }
-            for (int w = 0; w < nwaves; w++) {
-                int cap = 0;
-                if (rrqr_wave_cols<T>(mr[w], true) == 0 || mc[w] >= WAVE_COLS_MAX) continue;
-                hip_check(rrqr_wave_capacity<T>(mr[w], true, &cap), "rrqr wave capacity");
-                all_wave[w] = slabs[w] <= cap && elems[w] > TINY_ELEMS;
-            }
+            for (int w = 0; w < nwaves; w++)
+                if (rrqr_wave_cols<T>(mr[w], true) > 0 && mc[w] < WAVE_COLS_MAX)
+                    all_wave[w] = slabs[w] <= wave_cap(mr[w], true) && elems[w] > TINY_ELEMS;
         }
         for (size_t p = 0; p < plist.size(); p++) {
             const int c = plist[p];
@@ -1745,16 +1749,15 @@ void Tree::plan_sparsification(LevelPlan<T>& L) {
                          std::vector<SlabChunk>& chunk, char& form) {
         size_t cost = 0;
         for (bool dense : {false, true}) {
+            if (form_env >= 0 && dense != (form_env != 0)) continue;
             const int sc = rrqr_wave_cols<T>(max_rows, dense);
-            int cap = 0;
-            hip_check(rrqr_wave_capacity<T>(max_rows, dense, &cap), "rrqr wave capacity");
             std::vector<RrqrBig> b = big;
             std::vector<int> nsub, steps;
             for (auto& x : b) {
                 nsub.push_back(x.nsub = std::max(1, (x.t.max_cols + sc - 1) / sc));
                 steps.push_back(std::min(x.t.max_rows, x.t.max_cols));
             }
-            SlabPlan P = place_slabs(nsub, steps, cap);
+            SlabPlan P = place_slabs(nsub, steps, wave_cap(max_rows, dense));
             const size_t c = P.chunk.size() + P.spread;
             if (c == 0 || (cost > 0 && c >= cost)) continue;
             cost = c;
