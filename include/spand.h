@@ -90,10 +90,11 @@ spand_status spand_solve_device(spand_tree* t, double* d_x, int nrhs, int ld, vo
 /* No counterpart in the reference: spand_solve_device for callers that cannot allocate
  * device memory (code under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc). The apply's workspace (8 bytes per right-hand side for every unknown twice and
- * for every unknown that each level passes on) lives in a static device array of 64 MiB that every GPU the library runs on holds
- * until the process ends; a call needing more returns SPAND_ERR_ARG and does nothing. No
- * device allocation and no event creation happen in the call. Calls that overlap on one
- * GPU share the array and race: serialize them (one stream, or host synchronization). */
+ * for every unknown that each level passes on) lives in a static device array of 64 MiB that
+ * every GPU the library runs on holds until the process ends; a call needing more returns
+ * SPAND_ERR_ARG and does nothing. No device allocation and no event creation happen in the
+ * call. Calls that overlap on one GPU share the array and race: serialize them (one stream, or
+ * host synchronization). */
 spand_status spand_solve_device_noalloc(spand_tree* t, double* d_x, int nrhs, int ld, void* stream);
 /* x <- M^{-T} x, the adjoint apply of a differentiable solve. No counterpart in the
  * reference (its Tree has no transposed solve); for callers that differentiate through a
