@@ -122,7 +122,12 @@ constexpr int MV_ROWS = 16;
 constexpr int MV_STEP = 16;
 constexpr int MV_NW_MAX = 16;
 constexpr int MV_TAIL_MAX = 16;
-constexpr long long MV_TAIL_STEPS = 96;  // a phase of at most this many steps is small
+// A phase of at most this many steps is small. Above it one workgroup takes longer than a launch:
+// us an apply with the line at 0 / 24 / 48 / 96 / 192 steps: 15^3 one column 122 / 127 / 130 / 142 /
+// 205, 40^2 one column 89 / 80 / 80 / 88 / 88, 37^3 PLU 3 columns 332 / 333 / 333 / 357 / 396,
+// 512^2 32 columns 887 / 877 / 898 / 948 / 1110, 201^2 exact 216 / 216 / 216 / 240 / 289; 64^3 the
+// same up to 96.
+constexpr long long MV_TAIL_STEPS = 24;
 struct MvTail {
     MvDevPhase ph[MV_TAIL_MAX];
     int n;

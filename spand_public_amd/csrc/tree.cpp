@@ -561,9 +561,11 @@ struct MvPlan {
     }
     // Wavefronts per chunk: enough to have MV_WAVES in flight over the device (16 on each of
     // 256 CUs), while the longest chunk has a step for each; the wavefronts of one workgroup
-    // for a phase of few steps, which runs in one. 2048 / 4096 / 8192 / 16384 wavefronts: 854
-    // / 805 / 828 / 844 us for the FP64 apply of the 64^3 Laplacian on 4 columns; two steps
-    // each instead of one: 836 us at 4096.
+    // for a phase of few steps, which runs in one. us an apply at 2048 / 4096 / 8192 / 16384
+    // wavefronts: 64^3 FP64 4 columns 824 / 774 / 798 / 816, FP32 745 / 689 / 711 / 735, FP64 32
+    // columns 1602 / 1632 / 1691 / 1820, PLU FP32 8 columns 1080 / 989 / 1010 / 1059, 37^3 PLU 3
+    // columns 362 / 356 / 357 / 357, 512^2 32 columns 946 / 951 / 962 / 1000; two steps each instead
+    // of one: 4% slower on the first.
     void finish() {
         constexpr long long MV_WAVES = 4096;
         if (steps <= MV_TAIL_STEPS) {
