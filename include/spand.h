@@ -158,7 +158,10 @@ spand_status spand_get_factor_info(const spand_tree* t, double* seconds, long lo
  * largest pivot, clusters sparsified, median and largest Asn rows, median and largest Asn
  * columns), then the configuration (register-path RRQR on, Asn elements up to which the
  * one-workgroup RRQR runs, wavefronts per stepped slab (0: by slab count), trsm chunk policy,
- * source: 0 table, 1 environment). No choice changes the arithmetic. */
+ * source: 0 table, 1 environment). This is the choice, not a record of the launches: with
+ * source 0, dependency waves that the persistent RRQR holds whole run there instead (the
+ * families rrqr_wave, rrqr_reg, rrqr and rrqr_step of spand_kernel_profile say what ran). No
+ * choice changes the arithmetic. */
 spand_status spand_get_level_tune(const spand_tree* t, int* out);
 /* The table's configuration (5 ints as above) for a level shape (8 ints as above) and a
  * factor element size of elem_bytes (4 or 8). Host only. */

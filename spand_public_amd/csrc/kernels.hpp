@@ -58,9 +58,9 @@ template <typename T>
 hipError_t launch_rrqr_reg(const RrqrTask* d_tasks, int ntasks, const RrqrSeg* d_segs, int* d_size, double tol,
                            int variant, hipStream_t st);
 // Stepped RRQR of the large clusters of one wave: init, then steps 0..nsteps-1, then finish.
-// lds_bytes is the dynamic LDS of the pivot-column / reflector buffers (2 x max_rows
-// elements for a step, max_rows for finish), or 0 when the tasks carry global buffers
-// (RrqrBig::vbuf) because they exceed STEP_LDS_MAX.
+// A step's lds_bytes is the dynamic LDS of its pivot-column / reflector buffers (2 x max_rows
+// elements), or 0 when the tasks carry global buffers (RrqrBig::vbuf) because they exceed
+// STEP_LDS_MAX.
 constexpr int STEP_LDS_MAX = 40960;
 template <typename T>
 hipError_t launch_rrqr_init(const RrqrBig* d_bigs, const RrqrSlab* d_slabs, int nslabs, const RrqrSeg* d_segs,
@@ -99,7 +99,7 @@ hipError_t launch_rrqr_step(const RrqrBig* d_bigs, const RrqrSlab* d_slabs, int 
                             double tol, size_t lds_bytes, int waves, long long* prog, long long seq, hipStream_t st);
 template <typename T>
 hipError_t launch_rrqr_finish(const RrqrBig* d_bigs, const RrqrSlab* d_slabs, int nslabs, const RrqrSeg* d_segs,
-                              int* d_size, double tol, size_t lds_bytes, hipStream_t st);
+                              int* d_size, double tol, hipStream_t st);
 template <typename T> hipError_t launch_copy(const CopyTask* d_tasks, int ntasks, hipStream_t st);
 // The same from blocks of type TS to blocks of type T.
 template <typename TS, typename T> hipError_t launch_convert(const CopyTask* d_tasks, int ntasks, hipStream_t st);

@@ -1675,7 +1675,11 @@ __device__ inline size_t slab_idx(int rows, int r, int j) {
 // scope too (through the L2, which is not coherent with the other XCDs' L2s) unless every
 // slab of the cluster runs on one XCD (`local`): then the store may stay in their common L2,
 // and a word takes 225 ns from store to reader instead of 470-640 ns (measured one way,
-// two workgroups in turn).
+// two workgroups in turn). A local store has workgroup scope, which by the language's memory
+// model promises other workgroups nothing: what is relied on is the hardware's, that a CU's
+// vector stores of any scope write through its L1 to its XCD's L2, and that a device-scope load
+// of a CU on the same XCD reads that L2. Were it otherwise, the reader would poll to its bound
+// and factorize report it.
 using RelayWord = unsigned long long;
 typedef __attribute__((address_space(1))) RelayWord GRelayWord;
 
@@ -3368,7 +3372,15 @@ static hipError_t launch_wave_rw(const RrqrBig* d_bigs, const RrqrSlab* d_slabs,
 }
 
 // One dispatch table for the slab width, the capacity query and the launch: f(lanes per
-// column, rows / 16 per lane) of the variant for max_rows; false beyond WAVE_ROWS_MAX.
+// column, rows / 16 per lane) of the variant for max_rows; false beyond the last one.
+// Each form against the next longer one at the rows it just holds, ms for the three separators of
+// a band matrix (two waves of about `rows` steps). Fine FP32: 32 rows 0.135 / 0.179, 64 0.401 /
+// 0.448, 96 0.657 / 0.629, 128 0.819 / 0.896, 192 1.33 / 1.39, 256 1.87 / 2.11, 384 3.29 / 3.67,
+// 512 4.95 / 6.88, 768 11.4 / 13.1; FP64: 32 0.147 / 0.195, 64 0.442 / 0.451, 96 0.665 / 0.683, 128
+// 0.897 / 0.921, 192 1.40 / 1.50, 256 2.03 / 2.38, 384 4.00 / 4.52. The dense forms take
+// from 9% less to 25% more than the fine ones here (they are for waves that would not fit the
+// device in one launch); each against the next: FP32 64 0.365 / 0.448, 96 0.803 / 0.783, 192 1.54 / 1.69, 384 3.48 / 4.64,
+// 768 10.7 / 13.1; FP64 48 0.317 / 0.393, 96 0.762 / 0.777, 192 1.54 / 1.77, 384 3.74 / 4.50.
 template <typename T, typename F>
 static bool wave_variant(int max_rows, bool dense, F&& f) {
 #define SPAND_WAVE(L, RW)                                                                 \
@@ -3447,9 +3459,9 @@ hipError_t launch_rrqr_wave(const RrqrBig* d_bigs, const RrqrSlab* d_slabs, int 
 
 template <typename T>
 hipError_t launch_rrqr_finish(const RrqrBig* d_bigs, const RrqrSlab* d_slabs, int nslabs, const RrqrSeg* d_segs,
-                              int* d_size, double tol, size_t lds_bytes, hipStream_t st) {
+                              int* d_size, double tol, hipStream_t st) {
     if (nslabs == 0) return hipSuccess;
-    k_rrqr_finish<T><<<nslabs, NT, lds_bytes, st>>>(d_bigs, d_slabs, d_segs, d_size, tol);
+    k_rrqr_finish<T><<<nslabs, NT, 0, st>>>(d_bigs, d_slabs, d_segs, d_size, tol);
     return hipGetLastError();
 }
 
@@ -3491,7 +3503,7 @@ template hipError_t launch_convert<double, float>(const CopyTask*, int, hipStrea
     template hipError_t launch_rrqr_step<T>(const RrqrBig*, const RrqrSlab*, int, int, int, double, size_t, int,  \
                                             long long*, long long, hipStream_t);                                                       \
     template hipError_t launch_rrqr_finish<T>(const RrqrBig*, const RrqrSlab*, int, const RrqrSeg*, int*, double,  \
-                                              size_t, hipStream_t);
+                                              hipStream_t);
 SPAND_INST(float)
 SPAND_INST(double)
 

@@ -1972,7 +1972,7 @@ void Tree::launch_level(LevelPlan<T>& L) {
         hip_check(timed(prof_, KF_RRQR_FINISH, st, 0, 0,
                         [&] {
                             return launch_rrqr_finish<T>(db, ds, nsl, Packer::at<RrqrSeg>(dt, o_sg), d_size_, tol_,
-                                                         0, st);
+                                                         st);
                         },
                         &slot_finish[w]),
                   "rrqr finish");
@@ -2728,8 +2728,9 @@ void Tree::solve_interleaved(double* d_x, int nrhs, hipStream_t st, bool transpo
 }
 
 // Tree::solve (src/tree.cpp:1610-1635): permute in, forward sweep over the levels, backward
-// sweep in reverse, permute out. Split ops need no work: a sibling's segment aliases the
-// tail of its original cluster's segment.
+// sweep in reverse, permute out. Split ops need no work: the W phase writes the kept part to
+// its place in the parent's segment and the eliminated part to the sibling's.
+//
 // Instantiated graphs of the apply, by launch configuration; dropped at every factorization
 // (the plans they launch are rebuilt there).
 void Tree::drop_apply_graphs() {
