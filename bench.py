@@ -11,10 +11,11 @@ residual ||b - A x|| / ||b|| of the last step is checked in FP64 on the host.
 
 Kernel timing: during the warmup steps every library launch is bracketed by HIP events on
 its stream (spand_set_profiling); the family with the largest summed time is the dominant
-kernel. During the timed steps only that family carries events (the stepped RRQR's steps
-per dependency wave: two events around all steps of a wave), so the instrumentation stays
-out of the measured time; the roofline's achieved rate is the algorithmic bytes (or flops)
-of those launches divided by their summed event time.
+kernel. The timed steps carry no events: a launch that is timed is not part of a replayed
+graph, so the apply would be another one than a program gets. As many steps again, after the
+timed ones, have events around the dominant family (the stepped RRQR's steps per dependency
+wave: two events around all steps of a wave); the roofline's achieved rate is the algorithmic
+bytes (or flops) of those launches divided by their summed event time.
 
 Warmup: the first factorization of a pattern grows the device arenas and the pinned
 staging buffer, and the second still spends about 15 ms more host time between launches
@@ -90,8 +91,8 @@ def make_tree(S, A, X, nlevels, prec):
 
 
 def run_steps(S, torch, t, Am, d_b, d_x, N, steps, warmup, profile):
-    """warmup + timed steps of factorize + PCG; returns (s/step, iters, all-family warmup
-    profile, timed profile of the dominant family)."""
+    """warmup + timed steps of factorize + PCG, and as many profiled ones; returns (s/step,
+    iters, all-family warmup profile, profile of the dominant family)."""
     its = None
 
     def one_step():
@@ -110,18 +111,22 @@ def run_steps(S, torch, t, Am, d_b, d_x, N, steps, warmup, profile):
     torch.cuda.synchronize()
     wprof = t.kernel_profile() if profile else {}
     dominant = max(wprof.items(), key=lambda kv: kv[1]["ms"])[0] if wprof else "rrqr_step"
-    # timed steps: only the dominant family carries events (the stepped RRQR is timed per
-    # dependency wave, two events around all of its steps)
-    t.set_profiling(dominant if profile else False)
-    t.profile_reset()
+    t.set_profiling(False)
     torch.cuda.synchronize()
     t0 = time.perf_counter()
     for _ in range(steps):
         one_step()
     torch.cuda.synchronize()
     dt = (time.perf_counter() - t0) / max(steps, 1)
-    tprof = t.kernel_profile() if profile else {}
-    t.set_profiling(False)
+    tprof = {}
+    if profile:  # the dominant family's launches, outside the timed region
+        t.set_profiling(dominant)
+        t.profile_reset()
+        for _ in range(steps):
+            one_step()
+        torch.cuda.synchronize()
+        tprof = t.kernel_profile()
+        t.set_profiling(False)
     return dt, its.tolist(), wprof, tprof
 
 
@@ -272,7 +277,7 @@ def main():
     ap.add_argument("--no-fp64", action="store_true", help="skip the FP64-factor comparison")
     ap.add_argument("--fp64-only", action="store_true",
                     help="only the FP64-factor steps (for profiling its kernels); the JSON line carries them")
-    ap.add_argument("--no-profile", action="store_true", help="no per-launch HIP events in the timed steps")
+    ap.add_argument("--no-profile", action="store_true", help="no per-launch HIP events, and no profiled steps after the timed ones")
     ap.add_argument("--differentiable", action="store_true",
                     help="only the differentiable-solve workload (2D 512^2 variable kappa, 32 RHS)")
     ap.add_argument("--copy-probe", type=int, default=0, metavar="MIB",
