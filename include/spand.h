@@ -146,7 +146,11 @@ spand_status spand_get_flops_log(const spand_tree* t, long long* count, int* out
 /* No counterpart in the reference: fallbacks the library took at run time, as bits of *flags.
  * Bit 0: the stepped RRQR's launch throttle (the host keeps at most 12 step launches ahead of
  * the device by polling a progress counter) gave up after a wait longer than two seconds;
- * later steps were launched without it (same results, possibly more empty step launches). */
+ * later steps were launched without it (same results, possibly more empty step launches).
+ * Bit 1: a wait of the persistent RRQR gave up (after about two seconds: something else held
+ * the places of the workgroups waited for, such as other processes' persistent launches); the
+ * factorization was done again with one launch per pivot step, and so are the tree's later ones
+ * (same results, slower). */
 spand_status spand_get_status_flags(const spand_tree* t, unsigned* flags);
 /* Wall seconds of the last spand_factorize, device bytes of the stored factor, of the arena. */
 spand_status spand_get_factor_info(const spand_tree* t, double* seconds, long long* factor_bytes,

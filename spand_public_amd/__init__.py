@@ -217,10 +217,14 @@ class Tree:
         return [dict(zip(self.TUNE_FIELDS, (int(v) for v in row))) for row in out.reshape(self.nlevels, nf)]
 
     def status_flags(self) -> dict:
-        """Run-time fallbacks taken so far (spand_get_status_flags)."""
+        """Run-time fallbacks taken so far (spand_get_status_flags); "persistent_rrqr_gave_up" is
+        there once it has happened."""
         f = C.c_uint()
         _check(self._h, self._L.spand_get_status_flags(self._h, C.byref(f)))
-        return {"step_throttle_gave_up": bool(f.value & 1)}
+        flags = {"step_throttle_gave_up": bool(f.value & 1)}
+        if f.value & 2:
+            flags["persistent_rrqr_gave_up"] = True
+        return flags
 
     def factor_info(self):
         s, fb, ab = C.c_double(), C.c_longlong(), C.c_longlong()

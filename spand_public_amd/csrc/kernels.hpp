@@ -72,7 +72,7 @@ hipError_t launch_rrqr_init(const RrqrBig* d_bigs, const RrqrSlab* d_slabs, int 
 // cluster stay below WAVE_COLS_MAX. d_slabs: the slabs by workgroup, big = -1 for a place
 // without one. The slabs of each cluster exchange their candidates through the relay words
 // (waits of at most spin_max polls, RRQR_SPIN_MAX by default: *fail is set to 1 if one gives
-// up); waits: some cluster has several slabs, and the launch is cooperative. Returns
+// up); waits: some cluster has several slabs, and a large launch is cooperative. Returns
 // hipErrorCooperativeLaunchTooLarge, launching nothing, when the slabs do not fit the device at
 // once; rrqr_wave_capacity gives how many do.
 constexpr int WAVE_COLS_MAX = 1 << 15;

@@ -1679,7 +1679,7 @@ __device__ inline size_t slab_idx(int rows, int r, int j) {
 // model promises other workgroups nothing: what is relied on is the hardware's, that a CU's
 // vector stores of any scope write through its L1 to its XCD's L2, and that a device-scope load
 // of a CU on the same XCD reads that L2. Were it otherwise, the reader would poll to its bound
-// and factorize report it.
+// and the host factorize again without these launches.
 using RelayWord = unsigned long long;
 typedef __attribute__((address_space(1))) RelayWord GRelayWord;
 
@@ -1702,9 +1702,9 @@ __device__ inline void relay_put_val(GRelayWord* p, unsigned tag, T x, bool loca
     }
 }
 // One failed poll of a bounded wait: true if the wait gives up, after spin_max polls
-// (RRQR_SPIN_MAX unless the caller lowers it) or once *fail is set: slabs that wait for each
-// other are launched cooperatively, so every one is resident and a correct schedule never comes
-// near the bound; the host turns the flag into an error.
+// (RRQR_SPIN_MAX unless the caller lowers it) or once *fail is set. With the cluster's slabs all
+// resident a wait never comes near the bound; where they are not (launch_wave_rw), the host does
+// the factorization again with per-step launches.
 __device__ inline bool relay_give_up(long long spins, int* fail, long long spin_max) {
     if (spins >= spin_max ||
         ((spins & 63) == 63 && __hip_atomic_load(fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
@@ -2738,7 +2738,7 @@ __global__ void __launch_bounds__(64, (wave_occupancy<T, L, RW>()))
         }
     }
     if (abandoned) {
-        // the host reports the failed wait. The cluster's maps and slab storage are not the
+        // the host factorizes again without these launches. The cluster's maps and slab storage are not the
         // QR's (this slab's registers are dropped; its cluster's other slabs abandon too, or
         // finish without it): rows = 0 makes k_rrqr_finish leave the cluster alone
         if (lane == 0) gp(B.dims)[0] = 0;
@@ -3359,10 +3359,16 @@ static hipError_t launch_wave_rw(const RrqrBig* d_bigs, const RrqrSlab* d_slabs,
     hipError_t e = wave_capacity_rw<T, L, RW>(&cap);
     if (e != hipSuccess) return e;
     if (cap < nslabs) return hipErrorCooperativeLaunchTooLarge;
-    // Slabs that wait for each other have to be resident together whatever else the device runs,
-    // other processes' launches included, so their launch is cooperative. It goes through a queue
-    // of its own, about 12 us before and after it; a launch in which nobody waits is a plain one.
-    if (!waits) {
+    // Slabs that wait for each other have to be resident together. A cooperative launch sees to
+    // that; it goes through a queue of its own, 12 us before and after it, and far more beside
+    // other streams' work: factor + PCG of 15^3 (FP64, 14 waves) takes 6.76 ms with every launch
+    // cooperative, 4.27 with plain ones. A launch in which nobody waits needs neither. One of up to
+    // a quarter of what the device holds is a plain one too: this process's launches are ordered on
+    // the null stream and other work leaves its places in time. Other processes' slabs can keep
+    // them, when they wait for places in turn (plain launches of five or more processes, or one
+    // cooperative launch): then the waits give up at their bound, all workgroups return, and the
+    // host factorizes again without these launches.
+    if (!waits || nslabs <= cap / 4) {
         k_rrqr_wave<T, L, RW><<<nslabs, 64, 0, st>>>(d_bigs, d_slabs, nsteps, tol, fail, spin_max);
         return hipGetLastError();
     }

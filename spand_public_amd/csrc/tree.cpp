@@ -490,6 +490,12 @@ hipStream_t Tree::aux_stream() {
     return aux_st_;
 }
 
+// A wait of the persistent RRQR gave up: its slabs were not all resident, because something
+// else held the device (another process's launches, say, whose slabs in turn wait for places
+// that these hold). The factorization is done again with one launch per pivot step, which needs
+// no two workgroups resident together, and so are the tree's later ones; status_flags() reports it.
+struct WaveGaveUp {};
+
 void Tree::factorize() {
     if (state_ != State::Assembled && state_ != State::Factorized)
         throw Error(ERR_STATE, "factorize() must follow assemble()");
@@ -498,10 +504,16 @@ void Tree::factorize() {
     // next factorize() succeeds
     state_ = State::Assembled;
     fprec_ = prec_;
-    if (prec_ == 0)
-        factorize_impl<double>();
-    else
-        factorize_impl<float>();
+    auto run = [&] {
+        if (prec_ == 0) factorize_impl<double>();
+        else factorize_impl<float>();
+    };
+    try {
+        run();
+    } catch (const WaveGaveUp&) {
+        wave_gave_up_ = true;
+        run();
+    }
     state_ = State::Factorized;
 }
 
@@ -1532,6 +1544,9 @@ void Tree::plan_sparsification(LevelPlan<T>& L) {
     auto& wlds_step = L.wlds_step;
     auto& step_waves = L.step_waves;
     auto& wflag0 = L.wflag0;
+    // The persistent launch is the default (SPAND_RRQR_PERSISTENT=0 returns to one launch
+    // per step, about 10.5 us a step on the 64^3 Laplacian against 2-4 us).
+    const bool persistent = !wave_gave_up_ && env_or("SPAND_RRQR_PERSISTENT", 1) != 0;
     // SPAND_RRQR_SLABS: at most so many slabs a persistent launch; SPAND_RRQR_DENSE: 0 or 1 fixes its form
     const long long cap_env = env_or("SPAND_RRQR_SLABS", INT32_MAX), form_env = env_or("SPAND_RRQR_DENSE", -1);
     auto wave_cap = [&](int max_rows, bool dense) {
@@ -1612,7 +1627,7 @@ void Tree::plan_sparsification(LevelPlan<T>& L) {
         // within 1%.
         constexpr long long TINY_ELEMS = 2000;
         std::vector<char> all_wave(nwaves, 0);
-        if (tune.source == 0 && env_or("SPAND_RRQR_PERSISTENT", 1) != 0) {
+        if (tune.source == 0 && persistent) {
             std::vector<int> mr(nwaves, 0), mc(nwaves, 0);
             std::vector<long long> slabs(nwaves, 0), elems(nwaves, 0);
             for (size_t p = 0; p < plist.size(); p++) {
@@ -1739,9 +1754,6 @@ void Tree::plan_sparsification(LevelPlan<T>& L) {
     L.wplace.assign(nwaves, {});
     L.wchunk.assign(nwaves, {});
     L.wdense.assign(nwaves, 0);
-    // The persistent launch is the default (SPAND_RRQR_PERSISTENT=0 returns to one launch
-    // per step, about 10.5 us a step on the 64^3 Laplacian against 2-4 us).
-    const bool persistent = env_or("SPAND_RRQR_PERSISTENT", 1) != 0;
     step_waves = tune.step_waves;  // 4, 8, 16; 0: by slab count
     tunes_[ilvl_] = tune;
     shapes_[ilvl_] = shape;
@@ -1980,7 +1992,7 @@ void Tree::launch_level(LevelPlan<T>& L) {
     int info2[2] = {0, 0};
     hip_check(hipMemcpy(info2, d_info_, 2 * sizeof(int), hipMemcpyDeviceToHost), "read info");
     const int info = info2[0];
-    if (info2[1] != 0) throw Error(ERR_HIP, "persistent RRQR: a wait for another slab's candidate gave up");
+    if (info2[1] != 0) throw WaveGaveUp();
     if (info != 0) {
         if (gen) throw Error(ERR_SINGULAR, "Error: Singular Pivot (cluster order " + std::to_string(info - 1) + ")");
         throw Error(ERR_NOT_SPD, "Error: Non-SPD Pivot (cluster order " + std::to_string(info - 1) + ")");

@@ -212,7 +212,7 @@ class Tree {
     void set_monitor_flops(bool on) { monitor_flops_ = on; }
     // Run-time fallbacks taken so far (bit 0: the stepped-RRQR launch throttle stopped after
     // a wait for the device longer than two seconds; later steps launched without it).
-    unsigned status_flags() const { return throttle_gave_up_ ? 1u : 0u; }
+    unsigned status_flags() const { return (throttle_gave_up_ ? 1u : 0u) | (wave_gave_up_ ? 2u : 0u); }
     const std::vector<ShapeRec>& flops_log() const { return flops_log_; }
     double factor_seconds() const { return t_factor_; }
     size_t factor_bytes() const { return factor_bytes_; }
@@ -296,6 +296,7 @@ class Tree {
     long long sig_seq_ = 0;
     bool sig_throttle_ = true;  // off after a wait that timed out
     bool throttle_gave_up_ = false;  // a wait timed out (reported by status_flags)
+    bool wave_gave_up_ = false;      // so did one of the persistent RRQR: per-step launches from then on
 
     // options
     int nlevels_;

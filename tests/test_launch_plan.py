@@ -77,11 +77,10 @@ def plan_slabs(nsub, steps, cap):
 
 @pytest.mark.parametrize("cap", [8, 20, 64, 1000, 2048])
 @pytest.mark.parametrize("kind", ["single", "mixed", "ordinary", "long"])
-def test_persistent_rrqr_slabs_are_placed_once_and_waiting_ones_launched_together(kind, cap):
+def test_persistent_rrqr_slabs_are_placed_once_and_waiting_ones_marked(kind, cap):
     """Each cluster whole in one launch of at most cap workgroups, on one XCD (workgroup modulo 8)
     unless none holds it. A launch in which a cluster has several slabs is one whose workgroups
-    wait for each other: it has to be marked, because only a cooperative launch has them all
-    resident."""
+    wait for each other: it has to be marked, because they have to be resident together."""
     rng = np.random.default_rng(cap)
     nsub = {"single": np.ones(300, int), "mixed": rng.choice([1, 1, 1, 2], 200), "ordinary": rng.integers(1, 9, 500),
             "long": rng.integers(1, max(2, cap + 1), 40)}[kind]
