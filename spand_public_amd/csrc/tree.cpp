@@ -1618,13 +1618,13 @@ void Tree::plan_sparsification(LevelPlan<T>& L) {
         const long long big_min_elems = tune.small_elems;
         widx.assign(plist.size(), 0);
         // Dependency waves that one persistent launch can hold run all their clusters there, unless
-        // the largest has at most TINY_ELEMS Asn elements: its few steps do not pay for the
-        // cooperative launch and the init and finish launches around it. The others, and every wave
-        // when a path is asked for through the environment, split by cluster size. ms a
-        // factorization with the limit at 0 / 2000 / 4000 / 10000 / 30000 elements: 15^3 FP64 3.19 /
-        // 3.14 / 3.14 / 3.65 / 3.65, 24^3 FP32 8.13 / 8.12 / 8.10 / 8.58 / 9.76, 24^3 PLU 11.63 /
-        // 11.63 / 11.62 / 11.79 / 14.03, 512^2 FP64 13.14 / 12.24 / 12.13 / 12.14 / 12.16; 64^3
-        // within 1%.
+        // the largest has at most TINY_ELEMS Asn elements: its few steps do not pay for the init and
+        // finish launches around it. The others, and every wave when a path is asked for through the
+        // environment, split by cluster size. ms a factorization with three Krylov iterations, the
+        // limit at 0 / 2000 / 4000 / 10000 / 30000 elements: 15^3 FP64 3.97 / 3.96 / 4.02 / 4.73 /
+        // 4.70, 24^3 FP32 9.19 / 9.20 / 9.16 / 9.83 / 11.2, 24^3 PLU 13.3 / 13.3 / 13.3 / 13.5 / 15.9,
+        // 512^2 FP64 15.1 / 14.7 / 14.7 / 14.7 / 14.7, 512^2 FP32 14.9 / 14.6 / 14.7 / 14.7 / 14.6;
+        // 64^3 within 1%.
         constexpr long long TINY_ELEMS = 2000;
         std::vector<char> all_wave(nwaves, 0);
         if (tune.source == 0 && persistent) {
