@@ -2161,7 +2161,8 @@ __global__ void __launch_bounds__(SLAB * NW) k_rrqr_step(const RrqrBig* bigs, co
 // column (registers of L lanes, or relay words) into a vector that all lanes read. Measured
 // against slabs of 64 columns held by 4 or 8 wavefronts with about ten barriers a step, on the
 // same clusters: 64^3 Laplacian 34.9 -> 21.7 ms a factorization (FP32), 48.0 -> 33.3 (FP64),
-// 96^3 variable kappa (FP32, with the per-step launches of clusters over 512 rows) 204 -> 129.
+// 96^3 variable kappa (FP32, with the per-step launches of clusters over 512 rows) 204 -> 129. With
+// the shorter clusters that the waves now hold as well: 23.2 (FP32) and 32.5 ms (FP64) at 64^3.
 // A step takes 3.5 (90 rows) to 6 us (300 rows): candidates 1.1, the pivot column 0.5, dlarfg
 // 0.4, v 0.15, w_j 0.3, the downdate 0.3, the slab's best 0.3, update 0.15, publication 0.5.
 // Step i: wait for every slab's candidate (norm, position, column), take the first maximum,
